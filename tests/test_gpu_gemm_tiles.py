@@ -1,0 +1,67 @@
+"""The matrix-core GEMM at the edges of its tiles and of its K loop, bit-exact on integer-valued
+operands (every partial sum is an exact f32 integer times a power of two): rows around 16- and
+32-row tiles and a workgroup's 64 and 128, tokens around 32, 64 and 128, and block counts around
+its four-block groups, its unrolled round and the cut of a split K loop (16 blocks, between
+super-blocks of 8)."""
+import numpy as np
+import pytest
+
+from test_oracle_gemv_cpu import int_matrix
+from ziglm_amd import bridge as B
+from ziglm_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+# columns: 1-5 blocks (odd counts load single blocks), 16-18 and 31 (split), 24 (uneven halves)
+COLS = {B.Q4_0: (32, 96, 128, 160, 512, 544, 992), B.Q8_0: (32, 64, 160, 512, 544, 992), B.BF16: (32, 96, 512, 992),
+        B.Q4_K: (256, 512, 768), B.Q6_K: (256, 512, 768)}
+CASES = [(q, c) for q in COLS for c in COLS[q]]
+
+
+def operands(qtype, rows, cols, batch, seed):
+    raw, wd = int_matrix(qtype, rows, cols, seed=seed, scale_pow=-1)
+    x = np.random.default_rng(seed).integers(-3, 4, (batch, cols)).astype(np.float32)
+    return raw, x, x.astype(np.float64) @ wd.T
+
+
+@pytest.mark.parametrize("qtype,cols", CASES)
+@pytest.mark.parametrize("rows,batch", [(1, 129), (31, 128), (33, 160), (127, 161), (129, 257)])
+def test_f32_edges(dev, qtype, cols, rows, batch):
+    raw, x, exact = operands(qtype, rows, cols, batch, rows + cols + batch)
+    assert np.all(np.abs(exact) < 2 ** 24)
+    y = dev.alloc(batch * rows * 4)
+    y.fill(0xAB)
+    dev.gemmEx(qtype, dev.from_numpy(raw), None, B.F32, dev.from_numpy(x), B.F32, y, batch, rows, cols)
+    np.testing.assert_array_equal(y.to_numpy((batch, rows), np.float32), exact.astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype,cols", CASES)
+@pytest.mark.parametrize("rows,batch", [(1, 1), (15, 31), (17, 33), (65, 130)])
+def test_bf16_and_pair_edges(dev, qtype, cols, rows, batch):
+    """bf16 activations into f32 outputs (exact), and the gate.up pair (both matrices the same one)
+    against the product's own GeGLU: the same sums, so at most bf16's rounding apart."""
+    raw, x, exact = operands(qtype, rows, cols, batch, rows + cols + batch)
+    w = dev.from_numpy(raw)
+    xb = dev.from_numpy(synth.f32_to_bf16(x))
+    y = dev.alloc(batch * rows * 4)
+    y.fill(0xAB)
+    dev.gemmEx(qtype, w, None, B.BF16, xb, B.F32, y, batch, rows, cols)
+    got = y.to_numpy((batch, rows), np.float32)
+    np.testing.assert_array_equal(got, exact.astype(np.float32))
+    g = dev.alloc(batch * rows * 4)
+    dev.geglu(y, y, g, batch * rows)
+    want = g.to_numpy((batch, rows), np.float32)
+    p = dev.alloc(batch * rows * 2)
+    dev.gemmEx(qtype, w, w, B.BF16, xb, B.BF16, p, batch, rows, cols)
+    pair = synth.bf16_to_f32(p.to_numpy((batch, rows), np.uint16))
+    # gelu and its product are the same f32 expression in both, up to a fused rounding (2^-23)
+    np.testing.assert_allclose(pair, want, rtol=2.0 ** -8, atol=1e-30)
+
+
+def test_large_tiles(dev):
+    """The 64 x 256 tile (three workgroups per CU) with ragged last tiles in both dimensions."""
+    rows, cols, batch = 8200, 160, 1990
+    raw, x, exact = operands(B.Q4_0, rows, cols, batch, 5)
+    y = dev.alloc(batch * rows * 4)
+    dev.gemmEx(B.Q4_0, dev.from_numpy(raw), None, B.F32, dev.from_numpy(x), B.F32, y, batch, rows, cols)
+    np.testing.assert_array_equal(y.to_numpy((batch, rows), np.float32), exact.astype(np.float32))

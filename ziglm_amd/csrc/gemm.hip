@@ -33,21 +33,23 @@
 // 2^-24 of a product, so a dot product lies within the f32 rounding of the sum, like the
 // decode GEMV's.
 //
-// Tiling. A 256-thread workgroup owns 32*WT*2 tokens x 32*WR*2 rows; its 4 waves form a 2 x 2
-// grid, each computing WT x WR tiles of 32 tokens x 32 rows with v_mfma_f32_32x32x16_bf16
-// (tokens on the A side, so a lane's accumulators are one weight row: the block scale is one
-// value per lane and tile, and stores of 32 lanes are 128 contiguous bytes of a token's output
-// row). The K loop takes one 32-column block per step, software-pipelined: the LDS holds block
-// k as bf16 terms (rows padded to 80 bytes against bank conflicts; a block scale sits in its
-// row's padding) while registers hold block k + 1's raw X and W, and block k's MFMAs run while
-// the same waves convert block k + 1 into the LDS and issue block k + 2's global loads, so the
-// matrix cores work during the conversion rather than after it. Where two operand buffers fit
-// two workgroups per CU (f32 or bf16 activations with one weight term: 80 KB) block k + 1 goes
-// to the other buffer and a step takes one barrier; otherwise every wave first reads all of
-// block k's operands into registers and a barrier frees the buffer. Activations load through a
-// range-checked resource (tokens past the batch read zeros) and weights from clamped rows with
-// zeros selected afterwards, so the loop body has no branches and the compiler interleaves the
-// MFMAs with the conversion.
+// Tiling. A workgroup of 4 waves owns 32 WT tokens x 128 WR rows; wave w computes all of the
+// tokens for its own 32 WR rows, as WT x WR tiles of v_mfma_f32_32x32x16_bf16 (tokens on the A
+// side, so a lane's accumulators are one weight row: the block scale is one value per lane and
+// tile, and stores of 32 lanes are 128 contiguous bytes of a token's output row). No two waves
+// share a weight row, so a lane loads the codes of its row straight into registers in the
+// B-operand layout and converts them there, once per workgroup, and only the activations go
+// through the LDS: a step's LDS reads are the activation terms alone (staged through the LDS
+// the weights were half of them, and their loop ran at 2-3 times the LDS traffic of this one).
+// With GE the wave's first tile column is 32 gate rows and its second the same 32 up rows, so
+// gelu(gate) * up needs no exchange.
+// The K loop takes one 32-column block per step. The LDS holds block k as bf16 terms (rows
+// padded to 80 bytes against bank conflicts) in one of two buffers while the registers hold the
+// raw bytes of the next blocks (UX activation and UW weight blocks ahead, more for the smaller
+// tiles, whose steps are shorter than a memory round trip); block k + 1 is converted into the
+// other buffer during block k's MFMAs, so a step takes one barrier. Activations load through a
+// range-checked resource (tokens past the batch read zeros); weight rows past the end are the
+// last row again, and nothing of them is stored.
 #include "zl_common.h"
 #include "zl_host.h"
 
@@ -56,9 +58,13 @@ namespace zl {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kGemmThreads = 256;
 constexpr int kKB = 32;       // columns per K step (one Q4_0 / Q8_0 block)
-constexpr int kLdsRow = 40;   // bf16 per LDS row: 32 + 8 padding (80 bytes)
+// A token's LDS row is the block's 32 columns of one term: 64 bytes, its four 16-byte chunks
+// permuted by the row so that neither the reads (8 rows' same chunk a cycle) nor the writes (two
+// whole rows a cycle) meet on a bank. (Rows padded to 80 bytes: the writes' conflicts were 12% of
+// the kernel's cycles.)
+constexpr int kLdsRow = 32;
+__device__ __forceinline__ int lds_chunk(int row, int c) { return row * kLdsRow + ((c ^ (row >> 2)) & 3) * 8; }
 
 // Weight terms (bf16 planes) per type: Q4_0 / Q8_0 quants are exact in bf16 and their block
 // scale multiplies each 32-column partial sum; BF16 weights are exact; F16 weights are two
@@ -68,9 +74,11 @@ constexpr int kLdsRow = 40;   // bf16 per LDS row: 32 + 8 padding (80 bytes)
 // Q6_K: its scale per 16-column half multiplies each K = 16 MFMA half's partial sum, the
 // quants u - 32 one exact term. (sc * (u - 32) as two exact terms with one scale d per step
 // instead: 5 term products, 10240 x 2560 x 2048 with f32 activations 555 against 453 us.)
+// Q4_0 rows whose block count is no multiple of four (see WGrp).
+constexpr int kQ4_0Odd = 0x100 + HIP_BRIDGE_Q4_0;
 template <int QT>
-constexpr bool w_halves() {
-    return QT == HIP_BRIDGE_Q6_K;
+constexpr bool is_q4_0() {
+    return QT == HIP_BRIDGE_Q4_0 || QT == kQ4_0Odd;
 }
 template <int QT>
 constexpr int w_terms() {
@@ -78,14 +86,8 @@ constexpr int w_terms() {
 }
 template <int QT>
 constexpr bool w_scaled() {
-    return QT == HIP_BRIDGE_Q4_0 || QT == HIP_BRIDGE_Q8_0 || QT == HIP_BRIDGE_Q4_K || QT == HIP_BRIDGE_Q6_K;
+    return is_q4_0<QT>() || QT == HIP_BRIDGE_Q8_0 || QT == HIP_BRIDGE_Q4_K || QT == HIP_BRIDGE_Q6_K;
 }
-// K-quant super-blocks: 8 K steps of 32 columns each
-template <int QT>
-constexpr bool k_quant() {
-    return QT == HIP_BRIDGE_Q4_K || QT == HIP_BRIDGE_Q6_K;
-}
-
 // bf16 (RNE) of two floats and the f32 values of the result.
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b, float& ra, float& rb) {
     const uint32_t p = pack_bf16x2(a, b);
@@ -110,6 +112,7 @@ __device__ __forceinline__ void split2(float x0, float x1, uint32_t* t) {
     t[1] = pack_bf16x2(x0 - a, x1 - b);
 }
 
+
 struct GemmArgs {
     const unsigned char* w;
     const unsigned char* wu;  // GeGLU: the up matrix (same type and shape as w)
@@ -117,232 +120,242 @@ struct GemmArgs {
     void* y;                  // f32 or bf16 [batch][rows]
     int64_t row_bytes;
     int rows, cols, batch;
+    int y_bf16;
 };
-
-// Raw weight bytes of one 32-column block for half a row (the thread's half: h = 0 or 1).
-template <int QT>
-struct WRaw;
-template <>
-struct WRaw<HIP_BRIDGE_Q4_0> {  // d + bytes [8h, 8h + 8): elements 8h.. and 16 + 8h..
-    uint32_t d, q0, q1;
-};
-template <>
-struct WRaw<HIP_BRIDGE_Q8_0> {  // d + int8 [16h, 16h + 16)
-    uint32_t d, q[4];
-};
-template <>
-struct WRaw<HIP_BRIDGE_BF16> {
-    u32x4 v[2];  // elements [16h, 16h + 16)
-};
-template <>
-struct WRaw<HIP_BRIDGE_F16> {
-    u32x4 v[2];
-};
-template <>
-struct WRaw<HIP_BRIDGE_F32> {
-    u32x4 v[4];
-};
-template <>
-struct WRaw<HIP_BRIDGE_Q4_K> {  // {d, dmin}, scales[12], qs bytes [16h, 16h + 16) of sub-block j's span
-    uint32_t dm, s[3], q[4], j;
-};
-template <>
-struct WRaw<HIP_BRIDGE_Q6_K> {  // ql / qh bytes of the half's 16 columns, its int8 scale, d
-    uint32_t ql[4], qh[4], sc, d, t;
-};
-
-// 32-bit load from a 2-byte aligned address (block quants sit at offset 2 of 18 / 34-byte
-// blocks): one global_load_dword, which gfx950 serves unaligned.
-typedef uint32_t u32_a2 __attribute__((aligned(2)));
-__device__ __forceinline__ uint32_t ld_u32_unaligned(const unsigned char* p) {
-    return *reinterpret_cast<const u32_a2*>(p);
-}
-
-// `blk` is always a valid block address (the caller clamps it); `ok` false gives zeros, selected
-// after the loads so that no load sits under a branch. K-quants: `blk` is the super-block and
-// `sub` the K step within it (0..7).
-__device__ __forceinline__ u32x4 sel4(bool ok, u32x4 v) { return ok ? v : u32x4{0, 0, 0, 0}; }
-template <int QT>
-__device__ __forceinline__ void load_w(const unsigned char* blk, int sub, int h, bool ok, WRaw<QT>& r) {
-    if constexpr (QT == HIP_BRIDGE_Q4_K) {
-        // 144-byte super-block {f16 d, f16 dmin, scales[12], qs[128]} (types.zig:170-175);
-        // sub-block j's 32 values are the low (j even) or high (j odd) nibbles of
-        // qs[32 (j / 2) .. + 32)
-        uint32_t v[8];
-        v[0] = ld_u32_unaligned(blk);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) v[1 + i] = ld_u32_unaligned(blk + 4 + 4 * i);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[4 + i] = ld_u32_unaligned(blk + 16 + 32 * (sub >> 1) + 16 * h + 4 * i);
-        r.dm = ok ? v[0] : 0u;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) r.s[i] = ok ? v[1 + i] : 0u;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r.q[i] = ok ? v[4 + i] : 0u;
-        r.j = (uint32_t)sub;
-    } else if constexpr (QT == HIP_BRIDGE_Q6_K) {
-        // 210-byte super-block {ql[128], qh[64], int8 scales[16], f16 d} (types.zig:187-192).
-        // K step sub = 4 n + t covers values [128 n + 32 t, + 32): value l of it takes the
-        // low (t < 2) or high nibble of ql[64 n + 32 (t & 1) + l], bits 2t, 2t + 1 of
-        // qh[32 n + l] and scale sc[8 n + l / 16 + 2 t] (quant.zig:357-385); the half h is
-        // l in [16 h, 16 h + 16), one scale
-        const int n = sub >> 2, t = sub & 3;
-        uint32_t ql[4], qh[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            ql[i] = ld_u32_unaligned(blk + 64 * n + 32 * (t & 1) + 16 * h + 4 * i);
-            qh[i] = ld_u32_unaligned(blk + 128 + 32 * n + 16 * h + 4 * i);
-        }
-        const uint32_t scw = *(const uint16_t*)(blk + 192 + 8 * n + 2 * t);  // scales 8n+2t, +1
-        const uint32_t d = *(const uint16_t*)(blk + 208);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            r.ql[i] = ok ? ql[i] : 0u;
-            r.qh[i] = ok ? qh[i] : 0u;
-        }
-        r.sc = ok ? (scw >> (8 * h)) & 0xffu : 0u;
-        r.d = ok ? d : 0u;
-        r.t = (uint32_t)t;
-    } else if constexpr (QT == HIP_BRIDGE_Q4_0) {
-        const uint32_t d = *(const uint16_t*)blk, q0 = ld_u32_unaligned(blk + 2 + 8 * h),
-                       q1 = ld_u32_unaligned(blk + 6 + 8 * h);
-        r.d = ok ? d : 0u;
-        r.q0 = ok ? q0 : 0u;
-        r.q1 = ok ? q1 : 0u;
-    } else if constexpr (QT == HIP_BRIDGE_Q8_0) {
-        const uint32_t d = *(const uint16_t*)blk;
-        r.d = ok ? d : 0u;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t q = ld_u32_unaligned(blk + 2 + 16 * h + 4 * i);
-            r.q[i] = ok ? q : 0u;
-        }
-    } else if constexpr (QT == HIP_BRIDGE_F32) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r.v[i] = sel4(ok, ld16(blk + 64 * h + 16 * i));
-    } else {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) r.v[i] = sel4(ok, ld16(blk + 32 * h + 16 * i));
-    }
-}
 
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
+// Two f32 values that bf16 holds exactly -> a packed pair (the high halves).
+__device__ __forceinline__ uint32_t pack_exact(float a, float b) {
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+// The signed (unsigned) bytes of two words as 8 bf16 values, exact.
+__device__ __forceinline__ bf16x8 bytes_s(uint32_t v, uint32_t w) {
+    return __builtin_bit_cast(bf16x8, u32x4{pack_exact((float)(int8_t)v, (float)(int8_t)(v >> 8)),
+                                            pack_exact((float)(int8_t)(v >> 16), (float)(int8_t)(v >> 24)),
+                                            pack_exact((float)(int8_t)w, (float)(int8_t)(w >> 8)),
+                                            pack_exact((float)(int8_t)(w >> 16), (float)(int8_t)(w >> 24))});
+}
+__device__ __forceinline__ bf16x8 bytes_u(uint32_t v, uint32_t w) {
+    return __builtin_bit_cast(bf16x8, u32x4{pack_exact((float)(v & 0xffu), (float)((v >> 8) & 0xffu)),
+                                            pack_exact((float)((v >> 16) & 0xffu), (float)(v >> 24)),
+                                            pack_exact((float)(w & 0xffu), (float)((w >> 8) & 0xffu)),
+                                            pack_exact((float)((w >> 16) & 0xffu), (float)(w >> 24))});
+}
+// a = {a of lanes 0-31, b of lanes 0-31}, b = {a of lanes 32-63, b of lanes 32-63}
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
 
-// Convert the thread's half row into bf16 terms: sw[t][row][...]; a block scale goes into the
-// padding of the row's first plane (bf16 slots 32, 33: kScaleSlot).
-constexpr int kScaleSlot = 32;
-constexpr int kMinSlot = 34;  // Q4_K: the block's min factor B_j = dmin * m_j (bf16 slots 34, 35)
+// A lane's share of a weight row: the 16 columns of each 32-column block that its half h =
+// lane / 32 multiplies in the block's two MFMAs. wk(s, h) is the first of the 8 columns that
+// half h takes in MFMA s; the activations are read from the LDS in the same order. Q4_0 holds
+// columns c and c + 16 in one byte and Q6_K has a scale per 16 columns, so there MFMA s covers
+// columns 16 s .. + 16; elsewhere a half takes 16 consecutive columns.
 template <int QT>
-__device__ __forceinline__ void store_w(const WRaw<QT>& r, int h, uint16_t* sw, int plane, int row) {
-    uint16_t* dst = sw + row * kLdsRow;
-    if constexpr (QT == HIP_BRIDGE_Q4_K) {
+__device__ __forceinline__ constexpr int wk(int s, int h) {
+    return (is_q4_0<QT>() || QT == HIP_BRIDGE_Q6_K) ? 16 * s + 8 * h : 16 * h + 8 * s;
+}
+
+// 32-, 64- and 128-bit loads from 2-byte aligned addresses (block codes sit at offset 2 of 18-
+// and 34-byte blocks; a 210-byte super-block may start anywhere), which gfx950 serves unaligned.
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+struct WSrc {  // the lane's weight row; offsets: the lane's, and a wave-uniform one
+    const unsigned char* row;
+    __device__ __forceinline__ u32x4 b128(uint32_t o, uint32_t so) const { return *(const u32x4_a2*)(row + so + o); }
+    __device__ __forceinline__ u32x2 b64(uint32_t o, uint32_t so) const { return *(const u32x2_a2*)(row + so + o); }
+    __device__ __forceinline__ uint32_t b32(uint32_t o, uint32_t so) const { return *(const u32_a2*)(row + so + o); }
+    __device__ __forceinline__ uint32_t b16(uint32_t o, uint32_t so) const { return *(const uint16_t*)(row + so + o); }
+};
+
+// Raw bytes of G consecutive 32-column blocks (blocks kb .. kb + G, kb a multiple of G from the
+// first block of the row): load() issues the loads, open() rearranges them once they are here,
+// ops<S>(u) gives the B operands of block kb + u's MFMA S, and scale() the block's scale(s)
+// (one per MFMA for Q6_K) and min factor (Q4_K). A lane's loads are few and wide: its row lies
+// alone in its cache line, so an instruction costs as many cache accesses as it has rows
+// whatever its width, and with two narrow loads per block these were the kernel's next limit
+// (the texture path busy for half of the time).
+// Signed 4- and 6-bit codes are taken as 16 (u - 8) and 4 (u - 32), the signed bytes that a
+// shift and a sign flip leave, so each costs one conversion; the power of two goes into the
+// scale.
+template <int QT>
+struct WGrp;
+template <>
+struct WGrp<HIP_BRIDGE_Q4_0> {
+    // Half h loads blocks 2 h and 2 h + 1 (36 bytes: f16 d, 16 code bytes, twice); open()
+    // swaps code bytes between the halves so that each has bytes [8 h, + 8) of all four.
+    static constexpr int G = 4;
+    u32x4 a, b;
+    uint32_t c;
+    __device__ __forceinline__ void load(const WSrc& s, int kb, int h) {
+        const uint32_t o = 36u * h, so = 18u * (uint32_t)kb;
+        a = s.b128(o, so);
+        b = s.b128(o + 16, so);
+        c = s.b32(o + 32, so);
+    }
+    __device__ __forceinline__ void open() {
+        // codes of the first block: the halfwords from byte 2 on; the second starts at byte 18
+        uint32_t q0 = __builtin_amdgcn_alignbit(a.y, a.x, 16), q1 = __builtin_amdgcn_alignbit(a.z, a.y, 16);
+        uint32_t q2 = __builtin_amdgcn_alignbit(a.w, a.z, 16), q3 = __builtin_amdgcn_alignbit(b.x, a.w, 16);
+        uint32_t d0 = __builtin_amdgcn_perm(b.x, a.x, 0x07060100u), d1 = d0;  // both blocks' d
+        swap_halves(q0, q2);
+        swap_halves(q1, q3);
+        uint32_t p0 = b.y, p1 = b.z, p2 = b.w, p3 = c;
+        swap_halves(p0, p2);
+        swap_halves(p1, p3);
+        swap_halves(d0, d1);
+        q[0][0] = q0 ^ 0x88888888u, q[0][1] = q1 ^ 0x88888888u;
+        q[1][0] = p0 ^ 0x88888888u, q[1][1] = p1 ^ 0x88888888u;
+        q[2][0] = q2 ^ 0x88888888u, q[2][1] = q3 ^ 0x88888888u;
+        q[3][0] = p2 ^ 0x88888888u, q[3][1] = p3 ^ 0x88888888u;
+        d[0] = d0, d[1] = d1;
+    }
+    uint32_t q[4][2], d[2];
+    template <int S>
+    __device__ __forceinline__ void ops(int u, bf16x8 (&o)[1]) const {
+        // byte j: low nibble = element j, high nibble = element j + 16
+        if constexpr (S == 0) o[0] = bytes_s((q[u][0] << 4) & 0xf0f0f0f0u, (q[u][1] << 4) & 0xf0f0f0f0u);
+        else o[0] = bytes_s(q[u][0] & 0xf0f0f0f0u, q[u][1] & 0xf0f0f0f0u);
+    }
+    __device__ __forceinline__ void scale(int u, int, float (&dv)[2], float&) const {
+        dv[0] = f16_bits_to_f32(u & 1 ? d[u >> 1] >> 16 : d[u >> 1] & 0xffffu) * 0.0625f;
+    }
+};
+template <>
+struct WGrp<kQ4_0Odd> {
+    // Any block count: one block at a time (a group's loads would reach past the row).
+    static constexpr int G = 1;
+    u32x2 q;
+    uint32_t d;
+    __device__ __forceinline__ void load(const WSrc& s, int kb, int h) {
+        const uint32_t so = 18u * (uint32_t)kb;
+        d = s.b16(0, so);
+        q = s.b64(2 + 8u * h, so);
+    }
+    __device__ __forceinline__ void open() {}
+    template <int S>
+    __device__ __forceinline__ void ops(int, bf16x8 (&o)[1]) const {
+        const uint32_t x = q.x ^ 0x88888888u, y = q.y ^ 0x88888888u;
+        if constexpr (S == 0) o[0] = bytes_s((x << 4) & 0xf0f0f0f0u, (y << 4) & 0xf0f0f0f0u);
+        else o[0] = bytes_s(x & 0xf0f0f0f0u, y & 0xf0f0f0f0u);
+    }
+    __device__ __forceinline__ void scale(int, int, float (&dv)[2], float&) const {
+        dv[0] = f16_bits_to_f32(d) * 0.0625f;
+    }
+};
+template <>
+struct WGrp<HIP_BRIDGE_Q8_0> {
+    static constexpr int G = 1;
+    u32x4 q;
+    uint32_t d;
+    __device__ __forceinline__ void load(const WSrc& s, int kb, int h) {
+        const uint32_t so = 34u * (uint32_t)kb;
+        d = s.b16(0, so);
+        q = s.b128(2 + 16u * h, so);
+    }
+    __device__ __forceinline__ void open() {}
+    template <int S>
+    __device__ __forceinline__ void ops(int, bf16x8 (&o)[1]) const {
+        o[0] = bytes_s(q[2 * S], q[2 * S + 1]);
+    }
+    __device__ __forceinline__ void scale(int, int, float (&dv)[2], float&) const { dv[0] = f16_bits_to_f32(d); }
+};
+template <>
+struct WGrp<HIP_BRIDGE_Q4_K> {
+    // Half of a 144-byte super-block {f16 d, f16 dmin, scales[12], qs[128]} (types.zig:170-175):
+    // sub-block j's 32 values are the low (j even) or high (j odd) nibbles of
+    // qs[32 (j / 2) .. + 32)
+    static constexpr int G = 4;
+    u32x4 hd, q[2];
+    __device__ __forceinline__ void load(const WSrc& s, int kb, int h) {
+        const uint32_t so = 144u * (uint32_t)(kb >> 3), qo = 16u + 16u * h, sq = so + 16u * (uint32_t)(kb & 4);
+        hd = s.b128(0, so);
+        q[0] = s.b128(qo, sq);
+        q[1] = s.b128(qo + 32, sq);
+    }
+    __device__ __forceinline__ void open() {}
+    template <int S>
+    __device__ __forceinline__ void ops(int u, bf16x8 (&o)[1]) const {
+        const int sh = (u & 1) * 4;
+        o[0] = bytes_u((q[u >> 1][2 * S] >> sh) & 0x0f0f0f0fu, (q[u >> 1][2 * S + 1] >> sh) & 0x0f0f0f0fu);
+    }
+    __device__ __forceinline__ void scale(int u, int kb, float (&dv)[2], float& mn) const {
         // 6-bit scale and min of sub-block j (quant.zig:285-290): j < 4: scales[j] & 63 and
         // scales[j + 4] & 63; else the low / high nibble of scales[j + 4] with the top two
         // bits of scales[j - 4] / scales[j] above them
-        const uint32_t j = r.j, b = 8u * (j & 3u);
-        const uint32_t s0 = (r.s[0] >> b) & 0xffu, s1 = (r.s[1] >> b) & 0xffu, s2 = (r.s[2] >> b) & 0xffu;
-        const uint32_t sc = j < 4 ? (s0 & 63u) : ((s2 & 15u) | ((s0 >> 6) << 4));
-        const uint32_t m = j < 4 ? (s1 & 63u) : ((s2 >> 4) | ((s1 >> 6) << 4));
-        *reinterpret_cast<float*>(dst + kScaleSlot) = f16_bits_to_f32(r.dm & 0xffffu) * (float)sc;
-        *reinterpret_cast<float*>(dst + kMinSlot) = f16_bits_to_f32(r.dm >> 16) * (float)m;
-        const int sh = (int)(j & 1u) * 4;
-        uint32_t p[8];
+        const uint32_t b = 8u * (uint32_t)u;
+        const uint32_t s0 = (hd.y >> b) & 0xffu, s1 = (hd.z >> b) & 0xffu, s2 = (hd.w >> b) & 0xffu;
+        const uint32_t hi = 0u - (((uint32_t)kb >> 2) & 1u);  // j >= 4: all ones (masks: no branch)
+        const uint32_t sc = (s0 & 63u & ~hi) | (((s2 & 15u) | ((s0 >> 6) << 4)) & hi);
+        const uint32_t m = (s1 & 63u & ~hi) | (((s2 >> 4) | ((s1 >> 6) << 4)) & hi);
+        dv[0] = f16_bits_to_f32(hd.x & 0xffffu) * (float)sc;
+        mn = f16_bits_to_f32(hd.x >> 16) * (float)m;
+    }
+};
+template <>
+struct WGrp<HIP_BRIDGE_Q6_K> {
+    // Half n of a 210-byte super-block {ql[128], qh[64], int8 scales[16], f16 d}
+    // (types.zig:187-192): block t covers values [128 n + 32 t, + 32), value l of it takes the
+    // low (t < 2) or high nibble of ql[64 n + 32 (t & 1) + l], bits 2t, 2t + 1 of qh[32 n + l]
+    // and scale sc[8 n + l / 16 + 2 t] (quant.zig:357-385). Half h loads l in [16 h, + 16);
+    // open() swaps 8 bytes so that MFMA s's words hold l in [16 s + 8 h, + 8).
+    static constexpr int G = 4;
+    u32x4 ql[2], qh;
+    u32x2 sc;
+    uint32_t d;
+    __device__ __forceinline__ void load(const WSrc& s, int kb, int h) {
+        const uint32_t so = 210u * (uint32_t)(kb >> 3), n = (uint32_t)(kb >> 2) & 1u, ho = 16u * h;
+        ql[0] = s.b128(ho, so + 64 * n);
+        ql[1] = s.b128(ho + 32, so + 64 * n);
+        qh = s.b128(ho + 128, so + 32 * n);
+        sc = s.b64(192, so + 8 * n);
+        d = s.b16(208, so);
+    }
+    __device__ __forceinline__ void open() {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t v = (r.q[i] >> sh) & 0x0f0f0f0fu;
-            p[2 * i] = pack_bf16x2((float)(v & 0xffu), (float)((v >> 8) & 0xffu));
-            p[2 * i + 1] = pack_bf16x2((float)((v >> 16) & 0xffu), (float)(v >> 24));
-        }
-        *reinterpret_cast<u32x4*>(dst + 16 * h) = u32x4{p[0], p[1], p[2], p[3]};
-        *reinterpret_cast<u32x4*>(dst + 16 * h + 8) = u32x4{p[4], p[5], p[6], p[7]};
-    } else if constexpr (QT == HIP_BRIDGE_Q6_K) {
-        // the half's scale d * sc (exact) in slot 32 + 2h; quants u - 32, exact in bf16
-        *reinterpret_cast<float*>(dst + kScaleSlot + 2 * h) = f16_bits_to_f32(r.d) * (float)(int8_t)(uint8_t)r.sc;
-        const int nsh = r.t < 2 ? 0 : 4, hsh = 2 * (int)r.t;
-        uint32_t p[8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t u = ((r.ql[i] >> (8 * e + nsh)) & 15u) | (((r.qh[i] >> (8 * e + hsh)) & 3u) << 4);
-                v[e] = (float)((int)u - 32);
-            }
-            p[2 * i] = pack_bf16x2(v[0], v[1]);
-            p[2 * i + 1] = pack_bf16x2(v[2], v[3]);
-        }
-        *reinterpret_cast<u32x4*>(dst + 16 * h) = u32x4{p[0], p[1], p[2], p[3]};
-        *reinterpret_cast<u32x4*>(dst + 16 * h + 8) = u32x4{p[4], p[5], p[6], p[7]};
-    } else if constexpr (QT == HIP_BRIDGE_Q4_0) {
-        *reinterpret_cast<float*>(dst + kScaleSlot) = f16_bits_to_f32(r.d);  // both halves store it
-        // byte j: low nibble = element j, high nibble = element j + 16 (value u - 8, exact)
-        uint32_t lo[4], hi[4];
-        const uint32_t q[2] = {r.q0, r.q1};
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const uint32_t lo4 = q[w] & 0x0f0f0f0fu, hi4 = (q[w] >> 4) & 0x0f0f0f0fu;
-#pragma unroll
-            for (int b = 0; b < 4; b += 2) {
-                lo[w * 2 + b / 2] = pack_bf16x2((float)((lo4 >> (8 * b)) & 0xffu) - 8.0f, (float)((lo4 >> (8 * b + 8)) & 0xffu) - 8.0f);
-                hi[w * 2 + b / 2] = pack_bf16x2((float)((hi4 >> (8 * b)) & 0xffu) - 8.0f, (float)((hi4 >> (8 * b + 8)) & 0xffu) - 8.0f);
-            }
-        }
-        *reinterpret_cast<u32x4*>(dst + 8 * h) = u32x4{lo[0], lo[1], lo[2], lo[3]};
-        *reinterpret_cast<u32x4*>(dst + 16 + 8 * h) = u32x4{hi[0], hi[1], hi[2], hi[3]};
-    } else if constexpr (QT == HIP_BRIDGE_Q8_0) {
-        *reinterpret_cast<float*>(dst + kScaleSlot) = f16_bits_to_f32(r.d);  // both halves store it
-        uint32_t p[8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int32_t v = (int32_t)r.q[i];
-            p[2 * i] = pack_bf16x2((float)(int8_t)(v & 0xff), (float)(int8_t)((v >> 8) & 0xff));
-            p[2 * i + 1] = pack_bf16x2((float)(int8_t)((v >> 16) & 0xff), (float)(int8_t)((v >> 24) & 0xff));
-        }
-        *reinterpret_cast<u32x4*>(dst + 16 * h) = u32x4{p[0], p[1], p[2], p[3]};
-        *reinterpret_cast<u32x4*>(dst + 16 * h + 8) = u32x4{p[4], p[5], p[6], p[7]};
-    } else if constexpr (QT == HIP_BRIDGE_BF16) {
-        *reinterpret_cast<u32x4*>(dst + 16 * h) = r.v[0];
-        *reinterpret_cast<u32x4*>(dst + 16 * h + 8) = r.v[1];
-    } else if constexpr (QT == HIP_BRIDGE_F16) {
-        uint32_t t[2][8];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const uint32_t w4[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                uint32_t s[2];
-                split2(f16_bits_to_f32(w4[j] & 0xffffu), f16_bits_to_f32(w4[j] >> 16), s);
-                t[0][4 * i + j] = s[0];
-                t[1][4 * i + j] = s[1];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            uint16_t* d = sw + u * plane + row * kLdsRow + 16 * h;
-            *reinterpret_cast<u32x4*>(d) = u32x4{t[u][0], t[u][1], t[u][2], t[u][3]};
-            *reinterpret_cast<u32x4*>(d + 8) = u32x4{t[u][4], t[u][5], t[u][6], t[u][7]};
-        }
-    } else {  // F32: elements [16h, 16h + 16)
-        uint32_t t[3][8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t s[3];
-            split3(__uint_as_float(r.v[i].x), __uint_as_float(r.v[i].y), s);
-            t[0][2 * i] = s[0], t[1][2 * i] = s[1], t[2][2 * i] = s[2];
-            split3(__uint_as_float(r.v[i].z), __uint_as_float(r.v[i].w), s);
-            t[0][2 * i + 1] = s[0], t[1][2 * i + 1] = s[1], t[2][2 * i + 1] = s[2];
-        }
-#pragma unroll
-        for (int u = 0; u < 3; ++u) {
-            uint16_t* d = sw + u * plane + row * kLdsRow + 16 * h;
-            *reinterpret_cast<u32x4*>(d) = u32x4{t[u][0], t[u][1], t[u][2], t[u][3]};
-            *reinterpret_cast<u32x4*>(d + 8) = u32x4{t[u][4], t[u][5], t[u][6], t[u][7]};
+        for (int i = 0; i < 3; ++i) {
+            u32x4& v = i < 2 ? ql[i & 1] : qh;
+            uint32_t x = v.x, y = v.y, z = v.z, w = v.w;
+            swap_halves(x, z);
+            swap_halves(y, w);
+            v = u32x4{x, y, z, w};
         }
     }
-}
-
+    template <int S>
+    __device__ __forceinline__ void ops(int u, bf16x8 (&o)[1]) const {
+        const int nsh = u < 2 ? 0 : 4, hsh = 2 * u;
+        auto code = [&](uint32_t l, uint32_t hb) {  // 4 (u - 32) as signed bytes
+            return ((((l >> nsh) & 0x0f0f0f0fu) << 2) | (((hb >> hsh) & 0x03030303u) << 6)) ^ 0x80808080u;
+        };
+        o[0] = bytes_s(code(ql[u & 1][2 * S], qh[2 * S]), code(ql[u & 1][2 * S + 1], qh[2 * S + 1]));
+    }
+    __device__ __forceinline__ void scale(int u, int, float (&dv)[2], float&) const {
+        const float d4 = f16_bits_to_f32(d) * 0.25f;
+        const uint32_t p = u < 2 ? sc.x >> (16 * u) : sc.y >> (16 * (u - 2));
+        dv[0] = d4 * (float)(int8_t)p;
+        dv[1] = d4 * (float)(int8_t)(p >> 8);
+    }
+};
+template <>
+struct WGrp<HIP_BRIDGE_BF16> {
+    static constexpr int G = 1;
+    u32x4 v[2];
+    __device__ __forceinline__ void load(const WSrc& s, int kb, int h) {
+        v[0] = s.b128(32u * h, 64u * (uint32_t)kb);
+        v[1] = s.b128(32u * h + 16, 64u * (uint32_t)kb);
+    }
+    __device__ __forceinline__ void open() {}
+    template <int S>
+    __device__ __forceinline__ void ops(int, bf16x8 (&o)[1]) const {
+        o[0] = __builtin_bit_cast(bf16x8, v[S]);
+    }
+    __device__ __forceinline__ void scale(int, int, float (&)[2], float&) const {}
+};
 // The (x term, w term) products accumulated, largest first: down to relative size 2^-16
 // (x in XT terms: 3 for f32 activations, 1 for bf16 ones, which are exact).
 template <int XT, int NW>
@@ -368,83 +381,480 @@ struct TermPairs<1, NW> {
     static constexpr int xt[3] = {0, 0, 0}, wt[3] = {0, 1, 2};
 };
 
-// Workgroup order. Workgroups are dispatched to the 8 XCDs in turn (linear id i on XCD i % 8),
-// and each XCD has its own L2. With ZL_GEMM_XCD the linear id is renumbered so that XCD k
-// takes the k-th eighth of the tiles in row-fastest order (the workgroups of one XCD then
-// share their token tile's activations in its L2). Measured neutral (within 2% either way
-// over the prefill products: the kernel is bound by its instruction issue, not by operand
-// fetches), so off by default.
-#ifndef ZL_GEMM_XCD
-#define ZL_GEMM_XCD 0
-#endif
-// Two operand buffers with f32 activations too (there the block-partial and total accumulators
-// leave too few registers and the loop spills a few).
-#ifndef ZL_GEMM_DB_F32X
-#define ZL_GEMM_DB_F32X 0
-#endif
-// Wave priority raised while a wave issues its MFMAs (s_setprio 1 over the block's MFMAs, 0
-// for the conversion and the scale products): taken for three-plane activations at 64-token
-// tiles, where three workgroups share a CU (10240 x 2560 weights, 2048 tokens: 498 -> 407 us);
-// at 128-token tiles it slows the products (292 -> 363 us), and elsewhere it is neutral.
-// ZL_GEMM_PRIO=1 forces it everywhere, -1 turns it off.
-#ifndef ZL_GEMM_PRIO
-#define ZL_GEMM_PRIO 0
-#endif
+
 
 // XK: activation form (X_F32: f32, split into three terms while staging; X_BF16: bf16, one
 // term; X_TERMS: three bf16 planes split beforehand, staged as they are). GE: gate.up GeGLU
-// pairs (the W tile's first
-// half holds gate rows, its second half the same rows of the up matrix; out = gelu(g) * u).
-// YB: bf16 output (else f32).
+// pairs (out = gelu(g) * u).
 enum XKind { X_F32 = 0, X_BF16 = 1, X_TERMS = 2 };
+
+// Activation blocks a thread holds ahead: more for the smaller tiles, whose steps are shorter.
+template <int WT>
+constexpr int x_ahead() {
+    return WT >= 4 ? 1 : WT >= 2 ? 2 : 4;
+}
+
+template <int QT, int XK, int WT, int RT, int WAVES, bool GE>
+__global__ __launch_bounds__(64 * WAVES, 2) void k_gemm_mfma(GemmArgs a) {
+    constexpr int NT = 64 * WAVES;             // threads
+    constexpr int XT = XK == X_BF16 ? 1 : 3;  // activation terms
+    constexpr int NW = w_terms<QT>();
+    constexpr bool SCALED = w_scaled<QT>();
+    constexpr bool HALVES = QT == HIP_BRIDGE_Q6_K;  // a scale per MFMA rather than per block
+    constexpr int BT = 32 * WT;                // tokens per workgroup
+    constexpr int TR = GE ? 16 : 32;           // output rows per tile
+    constexpr int OR = TR * WAVES * RT;        // and per workgroup
+    constexpr int XPLANE = BT * kLdsRow;
+    // Q4_K: per-token sums of each K step's activations (f32 or bf16 x: one sum; pre-split
+    // planes: one per plane, added in plane order), four steps' worth.
+    constexpr bool MIN = QT == HIP_BRIDGE_Q4_K;
+    constexpr int XSP = XK == X_TERMS ? 3 : 1;  // sum planes
+    __shared__ __attribute__((aligned(16))) uint16_t s_x[2 * XT * XPLANE];
+    __shared__ __attribute__((aligned(16))) float s_xs[MIN ? 4 : 1][MIN ? XSP * BT : 1];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int gx = (a.rows + OR - 1) / OR;
+    const int r_base = ((int)blockIdx.x % gx) * OR, b_base = ((int)blockIdx.x / gx) * BT;
+    // K steps [kbb, kbe): all of them, or with a split launch (gridDim.y = 2, f32 output,
+    // added into zeroed y) one half per workgroup row, cut between super-blocks
+    const int nkb_all = a.cols / kKB;
+    const int mid = gridDim.y > 1 ? (nkb_all / 2 + 7) & ~7 : nkb_all;
+    const int kbb = blockIdx.y ? mid : 0;
+    const int kbe = blockIdx.y ? nkb_all : mid;
+
+    // X staging. f32 x: chunk c = tid + NT i is token c / 8, columns 4 (c % 8) .. (four
+    // floats); bf16 x: token c / 4, columns 8 (c % 4) .. (eight bf16); term planes: the same
+    // within each plane. Loads through range-checked resources over the workgroup's tokens.
+    constexpr int XE = XK == X_F32 ? 4 : 8;          // elements per 16-byte chunk
+    constexpr int XCPT = kKB / XE;                  // chunks per token per block (per plane)
+    constexpr int XPL = XK == X_TERMS ? 3 : 1;      // planes loaded
+    constexpr int XPP = (BT * XCPT + NT - 1) / NT;  // passes per plane
+    constexpr int XCC = BT * XCPT;                  // chunks per plane; with more threads than
+                                                    // chunks several hold (and write) the same one
+    constexpr int NXI = XPL * XPP;                  // chunks per thread
+    const int xes = XK == X_F32 ? 4 : 2;
+    const int64_t tok_left = (int64_t)a.batch - b_base;
+    const int64_t xbytes = (tok_left < BT ? tok_left : BT) * (int64_t)a.cols * xes;
+    const uint32_t xrange = (uint32_t)(xbytes < 0xffffffffLL ? xbytes : 0xffffffffLL);
+    const int64_t plane_bytes = (int64_t)a.batch * a.cols * xes;
+    __amdgpu_buffer_rsrc_t rsx[XPL];
+#pragma unroll
+    for (int u = 0; u < XPL; ++u)
+        rsx[u] = buf_rsrc((const unsigned char*)a.x + u * plane_bytes + (int64_t)b_base * a.cols * xes, xrange);
+    constexpr int UX = x_ahead<WT>();
+    constexpr int U = 4;  // K steps per unrolled round
+    u32x4 xr[UX][NXI];
+    uint32_t xoff[XPP];
+#pragma unroll
+    for (int i = 0; i < XPP; ++i) {
+        const int cc = (tid + NT * i) % XCC;
+        xoff[i] = (uint32_t)(((int64_t)(cc / XCPT) * a.cols + XE * (cc % XCPT)) * xes);
+    }
+    const int last = kbe - 1;
+    const int lastg = last & ~3;  // the last group's first block (rows are whole groups where G > 1)
+    auto load_x = [&](int kb, int q, u32x4 (&r)[NXI]) {
+        r[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             rsx[q / XPP], xoff[q % XPP], (uint32_t)(min(kb, last) * kKB * xes), 0));
+    };
+    auto store_x = [&](int kb, int buf, int q, const u32x4& v) {
+        uint16_t* const sx = s_x + buf * (XT * XPLANE) + (q / XPP) * XPLANE;
+        const int cc = (tid + NT * (q % XPP)) % XCC, tok = cc / XCPT, k = XE * (cc % XCPT);
+        uint16_t* const dst = sx + lds_chunk(tok, k / 8) + k % 8;
+        // (MIN) the token's sum over the step's 32 columns of one term: pairs, then the
+        // XCPT consecutive lanes holding its chunks (8 of 4 f32 or 4 of 8 bf16: the same
+        // tree over the 32 values); each of them writes it (a branch would cut the step in two)
+        auto put_sum = [&](float cs) { s_xs[MIN ? kb & 3 : 0][(q / XPP) * BT + tok] = group_sum<XCPT>(cs); };
+        if constexpr (XK == X_F32) {
+            uint32_t t0[3], t1[3];
+            split3(__uint_as_float(v.x), __uint_as_float(v.y), t0);
+            split3(__uint_as_float(v.z), __uint_as_float(v.w), t1);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                *reinterpret_cast<u32x2*>(dst + p * XPLANE) = u32x2{t0[p], t1[p]};
+            if constexpr (MIN)
+                put_sum((__uint_as_float(v.x) + __uint_as_float(v.y)) + (__uint_as_float(v.z) + __uint_as_float(v.w)));
+        } else {
+            *reinterpret_cast<u32x4*>(dst) = v;
+            if constexpr (MIN)
+                put_sum(((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
+                        ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w))));
+        }
+    };
+
+    // W: RT tiles of 32 rows, a row per lane and half (the last row again past the end); GE: a
+    // tile is 16 gate rows and the same 16 rows of the up matrix, so that an output's two sums
+    // lie 16 lanes apart.
+    const int trow = GE ? lane & 15 : lane & 31;
+    const int wrow = r_base + TR * RT * wave;
+    WSrc ws[RT];
+#pragma unroll
+    for (int j = 0; j < RT; ++j)
+        ws[j].row = (GE && (lane & 16) ? a.wu : a.w) + (int64_t)min(wrow + TR * j + trow, a.rows - 1) * a.row_bytes;
+    using WQ = WGrp<QT>;
+    constexpr int G = WQ::G;
+    constexpr int RING = G == 1 ? 2 : 1;  // G = 1: blocks in flight; else the next group
+    WQ cur[RT], nxt[RING][RT];
+
+    f32x16 acc[WT][RT];
+#pragma unroll
+    for (int i = 0; i < WT; ++i)
+#pragma unroll
+        for (int j = 0; j < RT; ++j) acc[i][j] = f32x16{};
+    using TP = TermPairs<XT, NW>;
+    constexpr int NP = TP::n;
+
+    // Operands of the current step and, while it runs, of the next: [step parity].
+    bf16x8 wb[2][RT][2][NW];
+    float dv[2][RT][2], mn[2][RT];
+#pragma unroll
+    for (int j = 0; j < RT; ++j) dv[1][j][0] = dv[1][j][1] = mn[1][j] = 0.0f;
+    // A unit is one chain of MFMAs into a partial sum that a scale then adds into the
+    // accumulators: a block of one tile, or with HALVES each of its MFMAs.
+    constexpr int UPT = HALVES ? 2 : 1, UNITS = WT * RT * UPT, NMU = 2 * NP / UPT;
+    f32x16 part[2] = {f32x16{}, f32x16{}};
+    f32x4 xsv[MIN ? 4 : 1];  // the unit's per-token sums (Q4_K)
+    // FMAs [r0, r1) of a finished unit: acc += d * part [- mn * (token sums)]
+    auto scale_unit = [&](int unit, const f32x16& pt, int par, int kb, int r0, int r1) {
+        const int tile = unit / UPT / RT, j = unit / UPT % RT;
+        const float d = dv[par][j][HALVES ? unit & 1 : 0], m = mn[par][j];
+        if constexpr (MIN) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (r < r0 || r >= r1) continue;
+                if (r % 4 == 0) {
+                    // lane (l, r) of a tile holds token 8 (r / 4) + 4 (l / 32) + r % 4
+                    const int t0 = 32 * tile + 8 * (r >> 2) + 4 * h;
+                    f32x4 v = *reinterpret_cast<const f32x4*>(&s_xs[kb & 3][t0]);
+#pragma unroll
+                    for (int u = 1; u < XSP; ++u) {
+                        const f32x4 w = *reinterpret_cast<const f32x4*>(&s_xs[kb & 3][u * BT + t0]);
+                        v.x += w.x, v.y += w.y, v.z += w.z, v.w += w.w;
+                    }
+                    xsv[r >> 2] = v;
+                }
+                acc[tile][j][r] = fmaf(d, pt[r], fmaf(-m, xsv[r >> 2][r & 3], acc[tile][j][r]));
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (r >= r0 && r < r1) acc[tile][j][r] = fmaf(d, pt[r], acc[tile][j][r]);
+        }
+    };
+
+    // One K step: block kb from LDS buffer `u & 1` with wb[u & 1]. Between its MFMAs, a slice
+    // each, run the scale products of the unit before, the conversion of block kb + 1's
+    // activations (into the other buffer) and weights, and the loads of the blocks after: the
+    // matrix cores take 32 cycles per MFMA, in which the wave can issue about seven vector
+    // instructions; left to themselves the conversion and the scale products form runs of their
+    // own beside which the matrix cores idle (10240 x 2560 x 2048 Q4_0, f32: 356 us).
+    int xlane[2];  // the lane's place in a tile's LDS rows, per MFMA
+#pragma unroll
+    for (int s = 0; s < 2; ++s) xlane[s] = lds_chunk(lane & 31, wk<QT>(s, h) / 8);
+    auto step = [&](int u, int kb) {
+        const int pc = u & 1, pn = pc ^ 1;
+        const uint16_t* const sx = s_x + pc * (XT * XPLANE);
+        bf16x8 xa[2][2][XT];
+        auto read_tile = [&](int i) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int t = 0; t < XT; ++t)
+                    xa[i & 1][s][t] = *reinterpret_cast<const bf16x8*>(sx + t * XPLANE + 32 * i * kLdsRow + xlane[s]);
+        };
+        constexpr int NS = WT * RT * 2 * NP;  // MFMAs (slices)
+        auto w_item = [&](int j, int s) {     // block kb + 1's weights of tile j, MFMA s
+            const int un = G == 1 ? 0 : (u + 1) & 3;
+            WQ& q = G == 1 ? nxt[pn][j] : cur[j];
+            if (s == 0) {
+                if (G > 1 && un == 0) {
+                    cur[j] = nxt[0][j];
+                    cur[j].open();
+                    nxt[0][j].load(ws[j], min(kb + 1 + G, lastg), h);
+                }
+                q.scale(un, kb + 1, dv[pn][j], mn[pn][j]);
+                q.template ops<0>(un, wb[pn][j][0]);
+            } else {
+                q.template ops<1>(un, wb[pn][j][1]);
+                if (G == 1) q.load(ws[j], min(kb + 3, last), h);
+            }
+        };
+        read_tile(0);
+        if constexpr (SCALED) scale_unit(UNITS - 1, part[(UNITS - 1) & 1], pn, kb - 1, 0, 16);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < WT; ++i) {
+            if (i + 1 < WT) read_tile(i + 1);
+#pragma unroll
+            for (int j = 0; j < RT; ++j)
+#pragma unroll
+                for (int s = 0; s < 2; ++s)
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) {
+                        const int t = ((i * RT + j) * 2 + s) * NP + p;           // slice
+                        const int unit = (i * RT + j) * UPT + (HALVES ? s : 0);  // and its place in its unit
+                        const int m = HALVES ? p : s * NP + p;
+                        const bf16x8 A = xa[i & 1][s][TP::xt[p]], Bv = wb[pc][j][s][TP::wt[p]];
+                        if constexpr (SCALED)
+                            part[unit & 1] =
+                                __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, m == 0 ? f32x16{} : part[unit & 1], 0, 0, 0);
+                        else
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, acc[i][j], 0, 0, 0);
+                        if (SCALED && unit > 0) {
+                            constexpr int M1 = NMU > 1 ? NMU - 1 : 1;
+                            const int mm = NMU > 1 ? m - 1 : 0;
+                            if (mm >= 0)
+                                scale_unit(unit - 1, part[(unit - 1) & 1], pc, kb, 16 * mm / M1, 16 * (mm + 1) / M1);
+                        }
+#pragma unroll
+                        for (int q = 0; q < NXI; ++q)
+                            if (q * NS / NXI == t) {
+                                store_x(kb + 1, pn, q, xr[(u + 1) % UX][q]);
+                                load_x(kb + 1 + UX, q, xr[(u + 1) % UX]);
+                            }
+#pragma unroll
+                        for (int w = 0; w < 2 * RT; ++w)  // after the last step's scale products
+                            if ((2 * w + 1) * NS / (4 * RT) == t) w_item(w >> 1, w & 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+        }
+        __syncthreads();  // block kb + 1 is in its buffer, and block kb's is free
+    };
+
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+        cur[j].load(ws[j], kbb, h);
+        if constexpr (G > 1) {
+            nxt[0][j].load(ws[j], min(kbb + G, lastg), h);
+        } else {
+            nxt[1 % RING][j].load(ws[j], min(kbb + 1, last), h);
+            nxt[0][j].load(ws[j], min(kbb + 2, last), h);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NXI; ++q) load_x(kbb, q, xr[0]);
+#pragma unroll
+    for (int q = 0; q < NXI; ++q) store_x(kbb, 0, q, xr[0][q]);
+#pragma unroll
+    for (int b = 0; b < UX; ++b)
+#pragma unroll
+        for (int q = 0; q < NXI; ++q) load_x(kbb + 1 + b, q, xr[(b + 1) % UX]);
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+        cur[j].open();
+        cur[j].scale(0, kbb, dv[0][j], mn[0][j]);
+        cur[j].template ops<0>(0, wb[0][j][0]);
+        cur[j].template ops<1>(0, wb[0][j][1]);
+    }
+    if constexpr (MIN) {  // the first step's scaling of "the unit before" adds 0 * 0
+        if (tid < BT)
+#pragma unroll
+            for (int u = 0; u < XSP; ++u) s_xs[3][u * BT + tid] = 0.0f;
+    }
+    __syncthreads();
+    // A branch per step keeps each in a basic block of its own: unrolled into one, instruction
+    // selection moves the scale products of several steps together, and their partial sums spill.
+    for (int k0 = kbb; k0 < kbe; k0 += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k0 + u < kbe) step(u, k0 + u);  // uniform
+    }
+    if constexpr (SCALED) {  // the last unit's scale products
+        if ((kbe - kbb) & 1) scale_unit(UNITS - 1, part[(UNITS - 1) & 1], 0, kbe - 1, 0, 16);
+        else scale_unit(UNITS - 1, part[(UNITS - 1) & 1], 1, kbe - 1, 0, 16);
+    }
+
+    // Epilogue: lane (l, r) of tile (i, j) holds token 8 (r / 4) + 4 (l / 32) + r % 4 and row
+    // l % 32.
+    auto out = [&](auto put) {
+#pragma unroll
+        for (int j = 0; j < RT; ++j) {
+            const int row = wrow + TR * j + trow;
+#pragma unroll
+            for (int i = 0; i < WT; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float v = acc[i][j][r];
+                    if constexpr (GE) v = gelu_fast(v) * __shfl_xor(v, 16);
+                    const int tok = b_base + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+                    if (tok < a.batch && row < a.rows && !(GE && (lane & 16))) put((int64_t)tok * a.rows + row, v);
+                }
+        }
+    };
+    if (a.y_bf16)
+        out([&](int64_t o, float v) { ((uint16_t*)a.y)[o] = (uint16_t)(pack_bf16x2(v, 0.0f) & 0xffffu); });
+    else if (gridDim.y > 1)  // two K halves into zeroed y: 0 + a + b in either order
+        out([&](int64_t o, float v) { unsafeAtomicAdd((float*)a.y + o, v); });
+    else
+        out([&](int64_t o, float v) { ((float*)a.y)[o] = v; });
+}
+
+__global__ __launch_bounds__(256) void k_zero_f32(float* __restrict__ y, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) y[i] = 0.0f;
+}
+void launch_zero_f32(float* y, int64_t n, hipStream_t s) {
+    k_zero_f32<<<(unsigned)std::min<int64_t>(cdiv(n, 256), 8192), 256, 0, s>>>(y, n);
+}
+
+// Two K halves per output tile (gridDim.y), added into zeroed y by float atomics: with exactly
+// two addends (0 + a + b in either order) the sum does not depend on their order, so results stay
+// bit-reproducible. f32 output only; 16 blocks at least, so that a cut between super-blocks
+// leaves both halves some.
+static unsigned split_k(const GemmArgs& a, bool ge, bool want, hipStream_t s) {
+    if (!want || ge || a.y_bf16 || a.cols < 16 * kKB) return 1;
+    launch_zero_f32((float*)a.y, (int64_t)a.batch * a.rows, s);
+    return 2;
+}
+
+template <int QT, int XK, bool GE, int WT, int RT>
+static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
+    constexpr int W = 4;
+    const dim3 grid((unsigned)(cdiv(a.rows, (GE ? 16 : 32) * W * RT) * cdiv(a.batch, 32 * WT)), ky);
+    k_gemm_mfma<QT, XK, WT, RT, W, GE><<<grid, 64 * W, 0, s>>>(a);
+}
+// Workgroup tile (tokens x rows; GE: half the output rows), for 256 CUs that hold two workgroups
+// each. Large tiles convert an operand for more MFMAs, small ones fill the chip:
+//   bf16 activations: 128 x 128 from 1.5 workgroups per CU (10240 x 2560 x 2048 Q4_0: 140 us,
+//     64 x 128 151, 32 x 128 212), else 64 x 128 likewise, else 32 x 128.
+//   f32 (three-term) activations: 64 x 256 from three per CU for the types whose conversion
+//     leaves it registers (it reads the LDS half as often per MFMA; the same product: 284 us,
+//     128 x 128 336, 64 x 128 322), else 64 x 128 from 1.5 per CU, else 32 x 128 (512 tokens of
+//     2048 x 2560: 39 us, 64 x 128 49).
+// Two K halves per tile (f32 output) where the tiles do not fill the CUs twice (512 tokens of 2048
+// x 2560 39 -> 32 us, 1024 rows 38 -> 26), or four times for deep products (2560 x 10240 x 2048:
+// 365 -> 341 us; at 333 tokens Q6_K 168 -> 117); at 333 tokens of 10240 x 2560 (480 tiles) the
+// halves cost more than they fill (87 -> 97 us).
+template <int QT, int XK, bool GE>
+static void launch_qt(const GemmArgs& a, hipStream_t s) {
+    constexpr bool BIG = XK != X_BF16 && !GE && (QT == HIP_BRIDGE_Q4_0 || QT == HIP_BRIDGE_BF16);
+    auto wgs = [&](int wt, int rt) { return cdiv(a.rows, 128 * rt / (GE ? 2 : 1)) * cdiv(a.batch, 32 * wt); };
+    const bool big = BIG && wgs(2, 2) >= 768;
+    const int wt = XK == X_BF16 && wgs(4, 1) >= 384 ? 4 : big || wgs(2, 1) >= 384 ? 2 : 1;
+    const int64_t n = wgs(wt, big ? 2 : 1);
+    const unsigned ky = split_k(a, GE, n < 384 || (n < 1024 && a.cols >= kSplitMinCols), s);
+    if constexpr (BIG) {
+        if (big) {
+            launch_tile<QT, XK, GE, 2, 2>(a, ky, s);
+            return;
+        }
+    }
+    if constexpr (XK == X_BF16) {
+        if (wt == 4) {
+            launch_tile<QT, XK, GE, 4, 1>(a, ky, s);
+            return;
+        }
+    }
+    if (wt == 2) launch_tile<QT, XK, GE, 2, 1>(a, ky, s);
+    else launch_tile<QT, XK, GE, 1, 1>(a, ky, s);
+}
+
+// ---- dense weights ---------------------------------------------------------------------------
+// F16 and F32 weights (two and three terms), and BF16 weights with bf16 activations. A dense row
+// is 64-128 bytes per step, so fetching each lane's row into its registers touches a cache line
+// per lane and instruction for 16 bytes of it; here the threads load half rows that neighbour
+// each other and stage them through the LDS like the activations (BF16 x bf16, 2048 tokens:
+// 10240 x 2560 149 us, rows in registers 160; gate.up 21504 x 5376 1807 against 2080. With f32
+// activations the three terms hide the fetch and the register form is the faster one from 333
+// tokens (111 -> 71 us) and equal at 2048, so BF16 weights take it there.)
+// A 256-thread workgroup owns 64 WT tokens x 64 WR rows; its 4 waves form a 2 x 2 grid of WT x WR
+// tiles of 32 x 32. The LDS holds block k's terms (rows padded to 80 bytes) while registers hold
+// block k + 1's raw X and W; where two operand buffers fit two workgroups per CU a step takes one
+// barrier.
+constexpr int kDenseThreads = 256;
+constexpr int kDenseRow = 40;  // bf16 per LDS row: 32 + 8 padding (80 bytes)
+template <int QT>
+struct DRaw {
+    u32x4 v[QT == HIP_BRIDGE_F32 ? 4 : 2];  // elements [16h, 16h + 16) of a row's block
+};
+__device__ __forceinline__ u32x4 sel4(bool ok, u32x4 v) { return ok ? v : u32x4{0, 0, 0, 0}; }
+// `blk` is always a valid address (the caller clamps the row); `ok` false gives zeros, selected
+// after the loads so that no load sits under a branch.
+template <int QT>
+__device__ __forceinline__ void load_d(const unsigned char* blk, int h, bool ok, DRaw<QT>& r) {
+    constexpr int n = QT == HIP_BRIDGE_F32 ? 4 : 2;
+#pragma unroll
+    for (int i = 0; i < n; ++i) r.v[i] = sel4(ok, ld16(blk + 16 * n * h + 16 * i));
+}
+template <int QT>
+__device__ __forceinline__ void store_d(const DRaw<QT>& r, int h, uint16_t* sw, int plane, int row) {
+    uint16_t* dst = sw + row * kDenseRow;
+    if constexpr (QT == HIP_BRIDGE_BF16) {
+        *reinterpret_cast<u32x4*>(dst + 16 * h) = r.v[0];
+        *reinterpret_cast<u32x4*>(dst + 16 * h + 8) = r.v[1];
+    } else if constexpr (QT == HIP_BRIDGE_F16) {
+        uint32_t t[2][8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t w4[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint32_t s[2];
+                split2(f16_bits_to_f32(w4[j] & 0xffffu), f16_bits_to_f32(w4[j] >> 16), s);
+                t[0][4 * i + j] = s[0];
+                t[1][4 * i + j] = s[1];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            uint16_t* d = sw + u * plane + row * kDenseRow + 16 * h;
+            *reinterpret_cast<u32x4*>(d) = u32x4{t[u][0], t[u][1], t[u][2], t[u][3]};
+            *reinterpret_cast<u32x4*>(d + 8) = u32x4{t[u][4], t[u][5], t[u][6], t[u][7]};
+        }
+    } else {  // F32: elements [16h, 16h + 16)
+        uint32_t t[3][8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t s[3];
+            split3(__uint_as_float(r.v[i].x), __uint_as_float(r.v[i].y), s);
+            t[0][2 * i] = s[0], t[1][2 * i] = s[1], t[2][2 * i] = s[2];
+            split3(__uint_as_float(r.v[i].z), __uint_as_float(r.v[i].w), s);
+            t[0][2 * i + 1] = s[0], t[1][2 * i + 1] = s[1], t[2][2 * i + 1] = s[2];
+        }
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            uint16_t* d = sw + u * plane + row * kDenseRow + 16 * h;
+            *reinterpret_cast<u32x4*>(d) = u32x4{t[u][0], t[u][1], t[u][2], t[u][3]};
+            *reinterpret_cast<u32x4*>(d + 8) = u32x4{t[u][4], t[u][5], t[u][6], t[u][7]};
+        }
+    }
+}
+
 
 // Workgroups per CU the launch asks registers for: three (170 VGPRs a lane) for bf16
 // activations when the LDS holds three, so a third wave per SIMD has MFMAs ready while the
 // others read operands or wait at a barrier; two otherwise (the three-term activations' loop
 // needs more registers: held to 170 it spills).
 template <int QT, int XK, int WT, int WR>
-constexpr int gemm_wgs_per_cu() {
+constexpr int dense_wgs_per_cu() {
     constexpr int bt = 64 * WT, br = 64 * WR;
-    constexpr int oper = (bt + w_terms<QT>() * br) * kLdsRow * 2;  // bf16 activations: one term
-    // (Q4_K's min term needs the registers: held to 170 its loop spills)
-    return XK == X_BF16 && QT != HIP_BRIDGE_Q4_K && 2 * oper * 3 <= 160 * 1024 ? 3 : 2;
+    constexpr int oper = (bt + w_terms<QT>() * br) * kDenseRow * 2;  // bf16 activations: one term
+    return XK == X_BF16 && 2 * oper * 3 <= 160 * 1024 ? 3 : 2;
 }
 
-template <int QT, int XK, int WT, int WR, bool GE, bool YB>
-__global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) void k_gemm_mfma(GemmArgs a) {
+template <int QT, int XK, int WT, int WR, bool GE>
+__global__ __launch_bounds__(kDenseThreads, (dense_wgs_per_cu<QT, XK, WT, WR>())) void k_gemm_dense(GemmArgs a) {
     constexpr int XT = XK == X_BF16 ? 1 : 3;  // activation terms
     constexpr int NW = w_terms<QT>();
-    constexpr bool SCALED = w_scaled<QT>();
     constexpr int BT = 2 * 32 * WT;  // tokens per workgroup
     constexpr int BR = 2 * 32 * WR;  // W rows per workgroup (GE: BR / 2 gate + BR / 2 up rows)
     constexpr int OR = GE ? BR / 2 : BR;  // output rows per workgroup
-    constexpr int XPLANE = BT * kLdsRow, WPLANE = BR * kLdsRow;
+    constexpr int XPLANE = BT * kDenseRow, WPLANE = BR * kDenseRow;
     constexpr int OPER_BYTES = (XT * XPLANE + NW * WPLANE) * 2;
     // Two operand buffers (block kb read while block kb + 1 is written: one barrier per step)
-    // when they fit two workgroups per CU in the 160 KB of LDS; else one (also for Q4_K with
-    // three activation planes, whose two-buffer loop needs 284 registers: one wave per SIMD).
-    constexpr bool DB = 2 * OPER_BYTES <= 80 * 1024 && (XK != X_F32 || ZL_GEMM_DB_F32X) &&
-                        !(QT == HIP_BRIDGE_Q4_K && XK == X_TERMS);
+    // when they fit two workgroups per CU in the 160 KB of LDS; else one.
+    constexpr bool DB = 2 * OPER_BYTES <= 80 * 1024 && XK != X_F32;
     constexpr int NBUF = DB ? 2 : 1;
     constexpr int XCH_BYTES = GE ? 2 * WT * WR * 16 * kWave * 4 : 0;  // up accumulators, two waves
-    // Q4_K: per-token sums of each K step's activations (f32 or bf16 x: one sum; pre-split
-    // planes: one per plane, added in plane order), in two slots by step parity: step kb + 1's
-    // sums are written while step kb's are read. (Summing f32 x's three terms instead, so that
-    // both f32 forms agree bit for bit, cost 3 reductions a step: 10240 x 2560 x 2048, 531 us.)
-    constexpr bool MIN = QT == HIP_BRIDGE_Q4_K;
-    constexpr int XSP = XK == X_TERMS ? 3 : 1;  // sum planes
-    constexpr int XS_FLOATS = MIN ? 2 * XSP * BT : 0;
     constexpr int MAIN_BYTES = NBUF * OPER_BYTES > XCH_BYTES ? NBUF * OPER_BYTES : XCH_BYTES;
-    __shared__ __attribute__((aligned(16))) unsigned char s_raw[MAIN_BYTES + XS_FLOATS * 4];
+    __shared__ __attribute__((aligned(16))) unsigned char s_raw[MAIN_BYTES];
     auto sx_of = [&](int b) { return reinterpret_cast<uint16_t*>(s_raw + b * OPER_BYTES); };
     auto sw_of = [&](int b) { return reinterpret_cast<uint16_t*>(s_raw + b * OPER_BYTES) + XT * XPLANE; };
-    float* const s_xs = reinterpret_cast<float*>(s_raw + MAIN_BYTES);  // [slot][plane][token]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    int tile = blockIdx.x;
-    const int gx = (a.rows + OR - 1) / OR, nwg = (int)gridDim.x;
-    if (ZL_GEMM_XCD && nwg % 8 == 0) tile = (tile % 8) * (nwg / 8) + tile / 8;
+    const int tile = blockIdx.x;
+    const int gx = (a.rows + OR - 1) / OR;
     const int r_base = (tile % gx) * OR, b_base = (tile / gx) * BT;
     // K steps [kbb, kbe): all of them, or with a split launch (gridDim.y = 2, f32 output,
     // added into zeroed y) one half per workgroup row
@@ -459,7 +869,7 @@ __global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) 
     constexpr int XE = XK == X_F32 ? 4 : 8;          // elements per 16-byte chunk
     constexpr int XCPT = kKB / XE;                  // chunks per token per block (per plane)
     constexpr int XPL = XK == X_TERMS ? 3 : 1;      // planes loaded
-    constexpr int XCH = XPL * BT * XCPT / kGemmThreads;
+    constexpr int XCH = XPL * BT * XCPT / kDenseThreads;
     const int xes = XK == X_F32 ? 4 : 2;
     const int64_t tok_left = (int64_t)a.batch - b_base;
     const int64_t xbytes = (tok_left < BT ? tok_left : BT) * (int64_t)a.cols * xes;
@@ -473,83 +883,65 @@ __global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) 
     // A plane is a whole number of 256-chunk passes, so pass i's plane is a constant of the
     // unrolled loop: the resource it selects stays in scalar registers (a plane index
     // computed from tid would make each load a loop over the lanes' distinct resources).
-    static_assert((BT * XCPT) % kGemmThreads == 0, "X plane not a whole number of passes");
+    static_assert((BT * XCPT) % kDenseThreads == 0, "X plane not a whole number of passes");
     auto load_x = [&](int kb) {
 #pragma unroll
         for (int i = 0; i < XCH; ++i) {
             constexpr int PC = BT * XCPT;  // chunks per plane
-            const int pl = kGemmThreads * i / PC, cc = tid + kGemmThreads * i % PC, tok = cc / XCPT;
+            const int pl = kDenseThreads * i / PC, cc = tid + kDenseThreads * i % PC, tok = cc / XCPT;
             const uint32_t off = (uint32_t)(((int64_t)tok * a.cols + kb * kKB + XE * (cc % XCPT)) * xes);
             xr[i] = bldp<POL_DEFAULT>(rsx[pl], off);
         }
     };
-    auto store_x = [&](int buf, int slot) {
+    auto store_x = [&](int buf) {
         uint16_t* const sx = sx_of(buf);
 #pragma unroll
         for (int i = 0; i < XCH; ++i) {
             constexpr int PC = BT * XCPT;
-            const int pl = kGemmThreads * i / PC, cc = tid + kGemmThreads * i % PC;
+            const int pl = kDenseThreads * i / PC, cc = tid + kDenseThreads * i % PC;
             const int tok = cc / XCPT, k = XE * (cc % XCPT);
-            // (MIN) the token's sum over the step's 32 columns of one term: pairs, then the
-            // XCPT consecutive lanes holding its chunks (8 of 4 f32 or 4 of 8 bf16: the same
-            // tree over the 32 values)
-            auto put_sum = [&](float cs, int plane) {
-                cs = group_sum<XCPT>(cs);
-                if (cc % XCPT == 0) s_xs[(slot * XSP + plane) * BT + tok] = cs;
-            };
             if constexpr (XK == X_F32) {
                 uint32_t t0[3], t1[3];
                 split3(__uint_as_float(xr[i].x), __uint_as_float(xr[i].y), t0);
                 split3(__uint_as_float(xr[i].z), __uint_as_float(xr[i].w), t1);
 #pragma unroll
                 for (int u = 0; u < 3; ++u)
-                    *reinterpret_cast<u32x2*>(sx + u * XPLANE + tok * kLdsRow + k) = u32x2{t0[u], t1[u]};
-                if constexpr (MIN)
-                    put_sum((__uint_as_float(xr[i].x) + __uint_as_float(xr[i].y)) +
-                                (__uint_as_float(xr[i].z) + __uint_as_float(xr[i].w)),
-                            0);
+                    *reinterpret_cast<u32x2*>(sx + u * XPLANE + tok * kDenseRow + k) = u32x2{t0[u], t1[u]};
             } else {
-                *reinterpret_cast<u32x4*>(sx + pl * XPLANE + tok * kLdsRow + k) = xr[i];
-                if constexpr (MIN)
-                    put_sum(((bf16_lo(xr[i].x) + bf16_hi(xr[i].x)) + (bf16_lo(xr[i].y) + bf16_hi(xr[i].y))) +
-                                ((bf16_lo(xr[i].z) + bf16_hi(xr[i].z)) + (bf16_lo(xr[i].w) + bf16_hi(xr[i].w))),
-                            pl);
+                *reinterpret_cast<u32x4*>(sx + pl * XPLANE + tok * kDenseRow + k) = xr[i];
             }
         }
     };
     // W staging: half rows (BR rows x 2 halves over 256 threads: BR / 128 passes, or the
     // first 2 BR threads when BR < 128). GE: tile rows [0, OR) are gate rows, [OR, BR) the
     // same rows of the up matrix.
-    constexpr int WPASS = BR * 2 >= kGemmThreads ? BR * 2 / kGemmThreads : 1;
-    // bytes per K step (K-quants: per super-block of 8 steps)
-    constexpr int64_t blk_bytes = QT == HIP_BRIDGE_Q4_0 ? 18 : QT == HIP_BRIDGE_Q8_0 ? 34 : QT == HIP_BRIDGE_F32 ? 128
-                                  : QT == HIP_BRIDGE_Q4_K ? 144 : QT == HIP_BRIDGE_Q6_K ? 210 : 64;
-    WRaw<QT> wr[WPASS];
+    constexpr int WPASS = BR * 2 >= kDenseThreads ? BR * 2 / kDenseThreads : 1;
+    constexpr int64_t blk_bytes = QT == HIP_BRIDGE_F32 ? 128 : 64;  // per K step
+    DRaw<QT> wr[WPASS];
     auto load_wt = [&](int kb) {
-        const int64_t boff = k_quant<QT>() ? (int64_t)(kb >> 3) * blk_bytes : (int64_t)kb * blk_bytes;
+        const int64_t boff = (int64_t)kb * blk_bytes;
 #pragma unroll
         for (int i = 0; i < WPASS; ++i) {
-            const int hr = tid + kGemmThreads * i, row = hr >> 1, h = hr & 1;
+            const int hr = tid + kDenseThreads * i, row = hr >> 1, h = hr & 1;
             const bool up = GE && row >= OR;
             const int gr = r_base + (up ? row - OR : row);
             const bool ok = hr < 2 * BR && gr < a.rows;
             const unsigned char* wm = up ? a.wu : a.w;
-            load_w<QT>(wm + (int64_t)min(gr, a.rows - 1) * a.row_bytes + boff, kb & 7, h, ok, wr[i]);
+            load_d<QT>(wm + (int64_t)min(gr, a.rows - 1) * a.row_bytes + boff, h, ok, wr[i]);
         }
     };
     auto store_wt = [&](int buf) {
         uint16_t* const swb = sw_of(buf);
 #pragma unroll
         for (int i = 0; i < WPASS; ++i) {
-            const int hr = tid + kGemmThreads * i;
-            if (2 * BR >= kGemmThreads || hr < 2 * BR) store_w<QT>(wr[i], hr & 1, swb, WPLANE, hr >> 1);
+            const int hr = tid + kDenseThreads * i;
+            if (2 * BR >= kDenseThreads || hr < 2 * BR) store_d<QT>(wr[i], hr & 1, swb, WPLANE, hr >> 1);
         }
     };
 
     const int wt0 = (wave >> 1) * 32 * WT;  // the wave's first token (within the workgroup)
     const int wr0 = (wave & 1) * 32 * WR;   // the wave's first W row (GE: wave & 1 = up)
     f32x16 acc[WT][WR];
-    f32x16 part[WT][WR];
 #pragma unroll
     for (int i = 0; i < WT; ++i)
 #pragma unroll
@@ -557,32 +949,28 @@ __global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) 
 
     using TP = TermPairs<XT, NW>;
     constexpr int NP = TP::n;
-    constexpr bool PRIO = ZL_GEMM_PRIO > 0 || (ZL_GEMM_PRIO == 0 && XK == X_TERMS && WT == 1);
-    // One K step: block kb's operands from LDS buffer `buf` into registers, its MFMAs (into the
-    // block partial when SCALED), then `convert` (block kb + 1 into the LDS and the loads of
-    // kb + 2), then the block scale products.
-    auto step = [&](int buf, int slot, bool single, auto convert) {
+    // One K step: block kb's operands from LDS buffer `buf` into registers, its MFMAs, then
+    // `convert` (block kb + 1 into the LDS and the loads of kb + 2).
+    auto step = [&](int buf, auto convert) {
         const uint16_t* const sx = sx_of(buf);
         const uint16_t* const sw = sw_of(buf);
         // with one buffer every wave holds all of block kb's operands before the barrier;
         // with two, each K = 16 half's operands are read just before its MFMAs (half the
         // registers)
         constexpr int KH = DB ? 1 : 2;
-        constexpr bool HALVES = w_halves<QT>();
         bf16x8 xa[KH][WT][XT], wb[KH][WR][NW];
-        float dv[WR], bv[MIN ? WR : 1], dv1[HALVES ? WR : 1];
         auto read_ops = [&](int ks, int slot) {
             const int ko = 16 * ks + 8 * (lane >> 5);
 #pragma unroll
             for (int i = 0; i < WT; ++i)
 #pragma unroll
                 for (int u = 0; u < XT; ++u)
-                    xa[slot][i][u] = *reinterpret_cast<const bf16x8*>(sx + u * XPLANE + (wt0 + 32 * i + (lane & 31)) * kLdsRow + ko);
+                    xa[slot][i][u] = *reinterpret_cast<const bf16x8*>(sx + u * XPLANE + (wt0 + 32 * i + (lane & 31)) * kDenseRow + ko);
 #pragma unroll
             for (int j = 0; j < WR; ++j)
 #pragma unroll
                 for (int u = 0; u < NW; ++u)
-                    wb[slot][j][u] = *reinterpret_cast<const bf16x8*>(sw + u * WPLANE + (wr0 + 32 * j + (lane & 31)) * kLdsRow + ko);
+                    wb[slot][j][u] = *reinterpret_cast<const bf16x8*>(sw + u * WPLANE + (wr0 + 32 * j + (lane & 31)) * kDenseRow + ko);
         };
         auto mfmas = [&](int ks, int slot) {
 #pragma unroll
@@ -592,86 +980,23 @@ __global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) 
 #pragma unroll
                     for (int p = 0; p < NP; ++p) {
                         const bf16x8 A = xa[slot][i][TP::xt[p]], Bv = wb[slot][j][TP::wt[p]];
-                        if constexpr (SCALED) {
-                            part[i][j] = ((ks == 0 || HALVES) && p == 0)
-                                             ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, f32x16{}, 0, 0, 0)
-                                             : __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, part[i][j], 0, 0, 0);
-                        } else {
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, acc[i][j], 0, 0, 0);
-                        }
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, acc[i][j], 0, 0, 0);
                     }
         };
-        if constexpr (SCALED) {
-#pragma unroll
-            for (int j = 0; j < WR; ++j) {
-                dv[j] = *reinterpret_cast<const float*>(sw + (wr0 + 32 * j + (lane & 31)) * kLdsRow + kScaleSlot);
-                if constexpr (MIN)
-                    bv[j] = *reinterpret_cast<const float*>(sw + (wr0 + 32 * j + (lane & 31)) * kLdsRow + kMinSlot);
-                if constexpr (HALVES)
-                    dv1[j] = *reinterpret_cast<const float*>(sw + (wr0 + 32 * j + (lane & 31)) * kLdsRow + kScaleSlot + 2);
-            }
-        }
-        // HALVES: the first half's partial sums scaled into acc before the second half's MFMAs
-        auto scale_first_half = [&]() {
-            if constexpr (HALVES) {
-#pragma unroll
-                for (int j = 0; j < WR; ++j)
-#pragma unroll
-                    for (int i = 0; i < WT; ++i)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(dv[j], part[i][j][r], acc[i][j][r]);
-            }
-        };
-        if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
         if constexpr (DB) {
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
                 read_ops(ks, 0);
                 mfmas(ks, 0);
-                if (ks == 0) scale_first_half();
             }
         } else {
             read_ops(0, 0);
             read_ops(1, 1);
-            if (single) __syncthreads();
+            __syncthreads();
             mfmas(0, 0);
-            scale_first_half();
             mfmas(1, 1);
         }
-        if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
         convert();
-        if constexpr (MIN) {
-            // acc += A_j * part - B_j * (sum of the token's x over the step: its terms' sums
-            // added in order); lane (l, r) of tile i holds token 32 i + 8 (r / 4) + 4 (l / 32) +
-            // r % 4: four runs of four
-#pragma unroll
-            for (int i = 0; i < WT; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int t0 = wt0 + 32 * i + 8 * q + 4 * (lane >> 5);
-                    f32x4 v = *reinterpret_cast<const f32x4*>(s_xs + slot * XSP * BT + t0);
-#pragma unroll
-                    for (int u = 1; u < XSP; ++u) {
-                        const f32x4 w = *reinterpret_cast<const f32x4*>(s_xs + (slot * XSP + u) * BT + t0);
-                        v.x += w.x, v.y += w.y, v.z += w.z, v.w += w.w;
-                    }
-                    const float xs[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                    for (int j = 0; j < WR; ++j)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const int r = 4 * q + e;
-                            acc[i][j][r] = fmaf(dv[j], part[i][j][r], fmaf(-bv[j], xs[e], acc[i][j][r]));
-                        }
-                }
-        } else if constexpr (SCALED) {
-#pragma unroll
-            for (int j = 0; j < WR; ++j)
-#pragma unroll
-                for (int i = 0; i < WT; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][j][r] = fmaf(HALVES ? dv1[j] : dv[j], part[i][j][r], acc[i][j][r]);
-        }
     };
 
     // Pipeline. The raw registers hold block kb + 1 while the MFMAs of block kb run; they are
@@ -680,7 +1005,7 @@ __global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) 
     // during the conversion rather than after it. Past the end: the last block again, unused.
     load_x(kbb);
     load_wt(kbb);
-    store_x(0, kbb & 1);
+    store_x(0);
     store_wt(0);
     __syncthreads();
     load_x(min(kbb + 1, kbe - 1));
@@ -688,8 +1013,8 @@ __global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) 
     for (int it = 0; it < kbe - kbb; ++it) {
         const int kb = kbb + it;
         const int cur = DB ? (it & 1) : 0, nxt = DB ? (cur ^ 1) : 0;
-        step(cur, kb & 1, !DB, [&]() {
-            store_x(nxt, (kb + 1) & 1);
+        step(cur, [&]() {
+            store_x(nxt);
             store_wt(nxt);
             load_x(min(kb + 2, kbe - 1));
             load_wt(min(kb + 2, kbe - 1));
@@ -730,7 +1055,7 @@ __global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) 
             for (int r = 0; r < 16; ++r) {
                 const int tok = b_base + wt0 + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 if (tok < a.batch) {
-                    if constexpr (YB)
+                    if (a.y_bf16)
                         ((uint16_t*)a.y)[(int64_t)tok * a.rows + row] = (uint16_t)(pack_bf16x2(acc[i][j][r], 0.0f) & 0xffffu);
                     else if (gridDim.y > 1)  // two K halves into zeroed y: 0 + a + b in either order
                         unsafeAtomicAdd((float*)a.y + (int64_t)tok * a.rows + row, acc[i][j][r]);
@@ -741,54 +1066,44 @@ __global__ __launch_bounds__(kGemmThreads, (gemm_wgs_per_cu<QT, XK, WT, WR>())) 
         }
 }
 
+
 // Workgroup tile: the largest of 128 x 128, 64 x 128 and 64 x 64 (tokens x W rows) that still
 // gives at least two workgroups per CU (bigger tiles convert each operand for more MFMAs;
-// smaller ones fill the chip at small batches).
-// Split K (ZL_GEMM_SPLITK, zl_host.h: two halves of the K steps per output tile, summed into
-// zeroed y by float atomic adds; with exactly two addends the sum does not depend on their
-// order, so results stay bit-reproducible) for deep products with f32 output that give fewer
-// than two rounds of workgroups: 2560 x 10240 x 2048, 640 -> 1280 workgroups: Q4_0 435 -> 401
-// us, Q4_K 520 -> 479, Q6_K 634 -> 559; at 128 tokens Q4_0 250 -> 129 us.
-__global__ __launch_bounds__(256) void k_zero_f32(float* __restrict__ y, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) y[i] = 0.0f;
-}
-void launch_zero_f32(float* y, int64_t n, hipStream_t s) {
-    k_zero_f32<<<(unsigned)std::min<int64_t>(cdiv(n, 256), 8192), 256, 0, s>>>(y, n);
-}
-template <int QT, int XK, bool GE, bool YB>
-static void launch_qt(const GemmArgs& a, hipStream_t s) {
+// smaller ones fill the chip at small batches). Deep products with f32 output that give fewer
+// than two rounds of workgroups run each tile as two K halves.
+template <int QT, int XK, bool GE>
+static void launch_dense(const GemmArgs& a, hipStream_t s) {
     constexpr int64_t kFill = 512;
     auto wgs = [&](int bt, int br) { return cdiv(a.rows, GE ? br / 2 : br) * cdiv(a.batch, bt); };
     const int64_t n = wgs(128, 128) >= kFill ? wgs(128, 128) : wgs(64, 128) >= kFill ? wgs(64, 128) : wgs(64, 64);
-    // Deep products with f32 output and fewer than two rounds of workgroups: two K halves per
-    // tile, added into zeroed y
-    unsigned ky = 1;
-    if constexpr (!GE && !YB) {
-        if (ZL_GEMM_SPLITK && n < 2 * kFill && a.cols >= ZL_GEMM_SPLITK_MIN_COLS) {
-            ky = 2;
-            launch_zero_f32((float*)a.y, (int64_t)a.batch * a.rows, s);
-        }
-    }
+    const unsigned ky = split_k(a, GE, n < 2 * kFill && a.cols >= kSplitMinCols, s);
     const dim3 grid((unsigned)n, ky);
     if (wgs(128, 128) >= kFill) {
-        k_gemm_mfma<QT, XK, 2, 2, GE, YB><<<grid, kGemmThreads, 0, s>>>(a);
+        k_gemm_dense<QT, XK, 2, 2, GE><<<grid, kDenseThreads, 0, s>>>(a);
     } else if (wgs(64, 128) >= kFill) {
-        k_gemm_mfma<QT, XK, 1, 2, GE, YB><<<grid, kGemmThreads, 0, s>>>(a);
+        k_gemm_dense<QT, XK, 1, 2, GE><<<grid, kDenseThreads, 0, s>>>(a);
     } else {
-        k_gemm_mfma<QT, XK, 1, 1, GE, YB><<<grid, kGemmThreads, 0, s>>>(a);
+        k_gemm_dense<QT, XK, 1, 1, GE><<<grid, kDenseThreads, 0, s>>>(a);
     }
 }
 
-template <int QT, int XK>
-static void launch_qx(const GemmArgs& a, bool ge, bool y_bf16, hipStream_t s) {
-    if (ge) y_bf16 ? launch_qt<QT, XK, true, true>(a, s) : launch_qt<QT, XK, true, false>(a, s);
-    else y_bf16 ? launch_qt<QT, XK, false, true>(a, s) : launch_qt<QT, XK, false, false>(a, s);
-}
 template <int QT>
-static void launch_q(const GemmArgs& a, int xk, bool ge, bool y_bf16, hipStream_t s) {
-    if (xk == X_F32) launch_qx<QT, X_F32>(a, ge, y_bf16, s);
-    else if (xk == X_BF16) launch_qx<QT, X_BF16>(a, ge, y_bf16, s);
-    else launch_qx<QT, X_TERMS>(a, ge, y_bf16, s);
+static void launch_q(const GemmArgs& a, int xk, bool ge, hipStream_t s) {
+    if constexpr (QT == HIP_BRIDGE_F16 || QT == HIP_BRIDGE_F32) {
+        if (xk == X_F32) ge ? launch_dense<QT, X_F32, true>(a, s) : launch_dense<QT, X_F32, false>(a, s);
+        else if (xk == X_BF16) ge ? launch_dense<QT, X_BF16, true>(a, s) : launch_dense<QT, X_BF16, false>(a, s);
+        else ge ? launch_dense<QT, X_TERMS, true>(a, s) : launch_dense<QT, X_TERMS, false>(a, s);
+    } else {
+        if (xk == X_F32) {
+            ge ? launch_qt<QT, X_F32, true>(a, s) : launch_qt<QT, X_F32, false>(a, s);
+        } else if (xk == X_TERMS) {
+            ge ? launch_qt<QT, X_TERMS, true>(a, s) : launch_qt<QT, X_TERMS, false>(a, s);
+        } else if constexpr (QT == HIP_BRIDGE_BF16) {
+            ge ? launch_dense<QT, X_BF16, true>(a, s) : launch_dense<QT, X_BF16, false>(a, s);
+        } else {
+            ge ? launch_qt<QT, X_BF16, true>(a, s) : launch_qt<QT, X_BF16, false>(a, s);
+        }
+    }
 }
 
 // 0 = launched; otherwise why not (the caller decides between a fallback and an error).
@@ -809,17 +1124,21 @@ int launch_gemm_mfma_ex(int qtype, const void* w, const void* wu, int64_t row_by
     if (cols % (kq ? 256 : kKB) != 0 || !aligned16(x) || !w_ok(w) || (wu && !w_ok(wu))) return HIP_BRIDGE_EUNSUPPORTED;
     // 32-bit byte offsets within a token tile's activations (per plane)
     if ((int64_t)128 * cols * (x_dtype == HIP_BRIDGE_F32 ? 4 : 2) > 0xffffffffLL) return HIP_BRIDGE_EUNSUPPORTED;
-    const GemmArgs a{(const unsigned char*)w, (const unsigned char*)wu, x, y, row_bytes, rows, cols, batch};
+    const GemmArgs a{(const unsigned char*)w, (const unsigned char*)wu, x, y, row_bytes, rows, cols, batch,
+                     y_dtype == HIP_BRIDGE_BF16};
     const int xk = x_dtype == HIP_BRIDGE_BF16 ? X_BF16 : x_dtype == HIP_BRIDGE_F32_TERMS ? X_TERMS : X_F32;
-    const bool ge = wu != nullptr, yb = y_dtype == HIP_BRIDGE_BF16;
+    const bool ge = wu != nullptr;
     switch (qtype) {
-        case HIP_BRIDGE_Q4_0: launch_q<HIP_BRIDGE_Q4_0>(a, xk, ge, yb, s); break;
-        case HIP_BRIDGE_Q8_0: launch_q<HIP_BRIDGE_Q8_0>(a, xk, ge, yb, s); break;
-        case HIP_BRIDGE_F16: launch_q<HIP_BRIDGE_F16>(a, xk, ge, yb, s); break;
-        case HIP_BRIDGE_BF16: launch_q<HIP_BRIDGE_BF16>(a, xk, ge, yb, s); break;
-        case HIP_BRIDGE_Q4_K: launch_q<HIP_BRIDGE_Q4_K>(a, xk, ge, yb, s); break;
-        case HIP_BRIDGE_Q6_K: launch_q<HIP_BRIDGE_Q6_K>(a, xk, ge, yb, s); break;
-        default: launch_q<HIP_BRIDGE_F32>(a, xk, ge, yb, s); break;
+        case HIP_BRIDGE_Q4_0:
+            if (cols % (4 * kKB) == 0) launch_q<HIP_BRIDGE_Q4_0>(a, xk, ge, s);
+            else launch_q<kQ4_0Odd>(a, xk, ge, s);
+            break;
+        case HIP_BRIDGE_Q8_0: launch_q<HIP_BRIDGE_Q8_0>(a, xk, ge, s); break;
+        case HIP_BRIDGE_F16: launch_q<HIP_BRIDGE_F16>(a, xk, ge, s); break;
+        case HIP_BRIDGE_BF16: launch_q<HIP_BRIDGE_BF16>(a, xk, ge, s); break;
+        case HIP_BRIDGE_Q4_K: launch_q<HIP_BRIDGE_Q4_K>(a, xk, ge, s); break;
+        case HIP_BRIDGE_Q6_K: launch_q<HIP_BRIDGE_Q6_K>(a, xk, ge, s); break;
+        default: launch_q<HIP_BRIDGE_F32>(a, xk, ge, s); break;
     }
     check_launch();
     return 0;

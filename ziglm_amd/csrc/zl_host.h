@@ -47,14 +47,8 @@ inline int device_cus() {
 // launches and returns true when the type, shape (cols % 32 == 0, K-quants % 256) and
 // alignment suit it, else launches nothing and returns false (the caller takes the vector
 // path).
-// Split K in the matrix-core kernel (gemm.hip launch_qt): products at least this deep with
-// f32 output run each tile as two K halves when their tiles number fewer than two rounds.
-#ifndef ZL_GEMM_SPLITK
-#define ZL_GEMM_SPLITK 1
-#endif
-#ifndef ZL_GEMM_SPLITK_MIN_COLS
-#define ZL_GEMM_SPLITK_MIN_COLS 4096
-#endif
+// Products at least this deep count as deep for the split of K in two halves (gemm.hip).
+constexpr int kSplitMinCols = 4096;
 // The matrix-core kernel's smallest workgroup tile is 64 tokens x 64 rows, so below a few
 // hundred tiles it leaves most of the chip idle (2560 x 10240 at up to 128 tokens: 40-80
 // workgroups; split in two K halves ~130 us for Q4_0 whatever the batch), while the vector
@@ -73,7 +67,7 @@ void launch_zero_f32(float* y, int64_t n, hipStream_t s);
 inline int gemm_mfma_min_batch(int qtype, int rows, int cols) {
     if (ZL_GEMM_MIN_BATCH) return ZL_GEMM_MIN_BATCH;
     const bool wide = rows >= 128 * 64;  // enough row tiles to fill half the chip's workgroup slots
-    const bool deep = ZL_GEMM_SPLITK && cols >= ZL_GEMM_SPLITK_MIN_COLS;
+    const bool deep = cols >= kSplitMinCols;
     if (qtype == HIP_BRIDGE_Q4_K) return wide ? 128 : 96;
     if (qtype == HIP_BRIDGE_Q6_K) return wide ? 64 : 96;
     return wide ? 96 : deep ? 64 : 128;
