@@ -628,6 +628,282 @@ static void launch_attn(int kv_dtype, AttnArgs& a, size_t ws_bytes, hipStream_t 
     check_launch();
 }
 
+// ---- causal chunks on the matrix cores ------------------------------------------------------
+// hip_attention_batched: tokens b of one sequence at positions pos_base + b over an f32 cache.
+// Every token of a chunk reads nearly the same K/V rows, so on the decode kernel, which streams a
+// token's rows for itself, 512 tokens over 512-1024 positions of 8 / 4 heads x 256 read 2 GB
+// through the L2 and took 218 us. Here a workgroup takes 16 query rows of one kv head (16 / gq
+// tokens x gq heads), its 8 waves the 16-key blocks of the rows' range in turn, with the f32 MFMA
+// 16x16x4 (exact f32 products and f32 sums, a quarter of the vector units' instruction count per
+// product; splitting K and V into bf16 terms instead would cost more vector work per workgroup
+// than the faster MFMA saves, at 16 rows per conversion).
+// Scores are formed transposed, S^T = K Q^T, so that lane (n = lane % 16, g = lane / 16) holds query
+// row n and keys 4 g + r in register r, which is the A operand of P V as it stands: MFMA r
+// contracts keys {r, 4 + r, 8 + r, 12 + r}. K and V go from the cache straight into operand
+// registers by 128-bit loads, four MFMAs to a load (the order of the contraction and of the output
+// columns follows the loads); each quarter of a block's rows is requested one quarter (a
+// thousand cycles at head size 256) ahead. The waves' online softmax states merge through LDS.
+// Limited by the f32 matrix rate (64 multiply-adds per cycle and CU).
+typedef float acc4 __attribute__((ext_vector_type(4)));
+constexpr int kChunkWaves = 8;
+template <int D>
+__global__ __launch_bounds__(kChunkWaves * kWave, 2) void k_attn_chunk(AttnArgs a) {
+    constexpr int NI = D / 16;   // 128-bit loads of a lane per K block and head row
+    constexpr int NC = D / 64;   // and per V row
+    constexpr int NH = D / 32;   // loads of half a K (V) block
+    constexpr int SLOTS = 4;
+    __shared__ float s_o[SLOTS][D / 4 * kWave];
+    __shared__ float s_m[kChunkWaves][16], s_l[kChunkWaves][16];
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int tpw = 16 / a.gq;  // tokens per workgroup
+    const int kvh = (int)blockIdx.x % a.nkv;
+    // the last tokens, whose ranges are the longest, first
+    const int tile = ((int)gridDim.x - 1 - (int)blockIdx.x) / a.nkv;
+    const int b0 = tile * tpw, b1 = min(b0 + tpw, a.batch) - 1;
+    // the lane's query row and its range of keys [lo, hi]
+    const int b = b0 + n / a.gq, p = a.pos_base + b;
+    const bool valid = b <= b1 && p >= 0 && p < a.max_len;
+    const int hi = valid ? p : -1;
+    const int lo = a.window > 0 ? max(0, p + 1 - a.window) : 0;
+    // the workgroup's keys [ks, ke) and the part of them that every row sees
+    const int ke = min(a.pos_base + b1, a.max_len - 1) + 1;
+    const int ks = a.window > 0 ? max(0, a.pos_base + b0 + 1 - a.window) : 0;
+    const bool whole = b0 + tpw <= a.batch && a.pos_base + b0 >= 0 && a.pos_base + b1 < a.max_len;
+    const int all_lo = a.window > 0 ? max(0, a.pos_base + b1 + 1 - a.window) : 0, all_hi = a.pos_base + b0;
+    const int nblk = ke > ks ? (ke - ks + 15) / 16 : 0;
+
+    const float* const kbase = (const float*)a.kc + a.row0 * a.row_stride + kvh * D + 4 * g;
+    const float* const vbase = (const float*)a.vc + a.row0 * a.row_stride + kvh * D + 4 * n;
+    // The query rows in operand order, in the LDS that the merge takes over (in registers they
+    // leave too few for the loads in flight): all waves read the same.
+    float* const s_q = &s_o[0][0] + 4 * lane;
+    {
+        const float* qrow = a.q + ((int64_t)min(b, a.batch - 1) * a.nh + kvh * a.gq + n % a.gq) * D + 4 * g;
+        for (int i = wave; i < NI; i += kChunkWaves) *reinterpret_cast<f32x4*>(s_q + 4 * kWave * i) = ldf4(qrow + 16 * i);
+    }
+    __syncthreads();
+    acc4 o[NC * 4];
+#pragma unroll
+    for (int i = 0; i < NC * 4; ++i) o[i] = acc4{};
+    float m = -INFINITY, l = 0.0f;
+
+    f32x4 bx[NH], by[NH];
+    // keys past the range load the range's last row (in bounds, masked)
+    auto load_k = [&](f32x4 (&r)[NH], int blk, int half) {
+        const float* kp = kbase + (int64_t)min(ks + 16 * blk + n, ke - 1) * a.row_stride;
+#pragma unroll
+        for (int i = 0; i < NH; ++i) r[i] = ldf4(kp + 16 * (NH * half + i));
+    };
+    auto load_v = [&](f32x4 (&r)[NH], int blk, int half) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const float* vp = vbase + (int64_t)min(ks + 16 * blk + 4 * g + 2 * half + j, ke - 1) * a.row_stride;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) r[NC * j + c] = ldf4(vp + 64 * c);
+        }
+    };
+    if (wave < nblk) load_k(bx, wave, 0);
+    for (int blk = wave; blk < nblk; blk += kChunkWaves) {
+        const int k0 = ks + 16 * blk;
+        // Scores: 16 products at a time into a fresh accumulator, these summed in two chains (one
+        // chain over the whole row is two to three times as far from the exact dot product, which
+        // large scores show: 8 / 1 heads x 256 with scale 1, 5.5e-7 -> 1.5e-6).
+        acc4 st[2] = {acc4{}, acc4{}}, sp = acc4{};
+        f32x4 q = *reinterpret_cast<const f32x4*>(s_q);
+        auto scores = [&](const f32x4 (&kr)[NH], int half) {
+#pragma unroll
+            for (int i = 0; i < NH; ++i) {
+                const f32x4 qn = *reinterpret_cast<const f32x4*>(s_q + 4 * kWave * ((NH * half + i + 1) % NI));
+                acc4 c = acc4{};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[i][e], q[e], c, 0, 0, 0);
+                st[i & 1] += sp;  // the load before, done by now
+                sp = c;
+                q = qn;
+                __builtin_amdgcn_sched_barrier(0);  // (the next row parts not all at once)
+            }
+        };
+        load_k(by, blk, 1);
+        scores(bx, 0);
+        __builtin_amdgcn_sched_barrier(0);  // the next loads into bx stay behind its last use
+        load_v(bx, blk, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        scores(by, 1);
+        st[0] += sp;
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(by, blk, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool edge = !(whole && k0 >= all_lo && k0 + 15 <= all_hi);  // uniform
+        float s[4], mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float v = (st[0][r] + st[1][r]) * a.scale;
+            if (a.softcap > 0.0f) v = a.softcap * tanh_fast(div_by_uniform(v, a.softcap, a.inv_cap));
+            const int key = k0 + 4 * g + r;
+            s[r] = key >= lo && key <= hi ? v : -INFINITY;
+            mx = fmaxf(mx, s[r]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16));
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float mn = fmaxf(m, mx), ms = mn == -INFINITY ? 0.0f : mn;
+        const float c = exp2f((m - ms) * kLog2e);
+        float pr[4], ps = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            pr[r] = exp2f((s[r] - ms) * kLog2e);
+            ps += pr[r];
+        }
+        l = l * c + ps;
+        m = mn;
+        if (!__all(c == 1.0f)) {  // rows 4 g + r of the output accumulators
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float cr = __shfl(c, 4 * g + r);
+#pragma unroll
+                for (int i = 0; i < NC * 4; ++i) o[i][r] *= cr;
+            }
+        }
+        if (edge) {
+            float z = 0.0f;  // NaN if a V value is infinite or NaN
+#pragma unroll
+            for (int i = 0; i < NH; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) z += bx[i][e] * 0.0f + by[i][e] * 0.0f;
+            if (__any(!(z == 0.0f))) {
+                // Some of the query rows see such a row and others do not: 0 * V would reach the
+                // others, so each takes just the keys it sees, and the products below add zeros.
+#pragma unroll 1
+                for (int k = 0; k < 16; ++k) {
+                    const float* vp = vbase + (int64_t)min(k0 + k, ke - 1) * a.row_stride;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float pk = __shfl(k & 2 ? (k & 1 ? pr[3] : pr[2]) : (k & 1 ? pr[1] : pr[0]),
+                                                4 * g + r + 16 * (k >> 2));
+                        const int rlo = __shfl(lo, 4 * g + r), rhi = __shfl(hi, 4 * g + r);
+                        if (k0 + k >= rlo && k0 + k <= rhi) {
+#pragma unroll
+                            for (int cc = 0; cc < NC; ++cc) {
+                                const f32x4 v = ldf4(vp + 64 * cc);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) o[cc * 4 + e][r] = fmaf(pk, v[e], o[cc * 4 + e][r]);
+                            }
+                        }
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) pr[r] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < NH; ++i) bx[i] = by[i] = f32x4{};
+            }
+        }
+        auto pv = [&](const f32x4 (&v)[NH], int half) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int cc = 0; cc < NC; ++cc)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        o[cc * 4 + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(pr[2 * half + j], v[NC * j + cc][e],
+                                                                             o[cc * 4 + e], 0, 0, 0);
+        };
+        pv(bx, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(bx, min(blk + kChunkWaves, nblk - 1), 0);
+        pv(by, 1);
+    }
+
+    // Merge: each wave's state scaled to the common maximum, waves 0-3 and then 4-7 into the four
+    // slots, which every thread then adds in slot order.
+    __syncthreads();  // every wave is done with the query rows
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (g == 0) {
+        s_m[wave][n] = m;
+        s_l[wave][n] = l;
+    }
+    __syncthreads();
+    // exp(m_w - M) of this wave for row `row`, and L of that row
+    auto factor = [&](int row) {
+        float M = s_m[0][row];
+#pragma unroll
+        for (int w = 1; w < kChunkWaves; ++w) M = fmaxf(M, s_m[w][row]);
+        return M == -INFINITY ? 0.0f : exp2f((s_m[wave][row] - M) * kLog2e);
+    };
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float f = factor(4 * g + r);
+#pragma unroll
+        for (int i = 0; i < NC * 4; ++i) o[i][r] *= f;
+    }
+    float* const slot = s_o[wave % SLOTS] + lane;
+    if (wave < SLOTS) {
+#pragma unroll
+        for (int i = 0; i < NC * 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) slot[(i * 4 + r) * kWave] = o[i][r];
+    }
+    __syncthreads();
+    if (wave >= SLOTS) {
+#pragma unroll
+        for (int i = 0; i < NC * 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) slot[(i * 4 + r) * kWave] += o[i][r];
+    }
+    __syncthreads();
+    // row = 4 g + r, columns 64 c + 4 n + e: four of a row per thread
+    for (int t = threadIdx.x; t < 16 * D / 4; t += kChunkWaves * kWave) {
+        const int row = t / (D / 4), col = t % (D / 4), c = col / 16, nn = col % 16;
+        const int bb = b0 + row / a.gq;
+        if (bb > b1) continue;
+        float M = s_m[0][row], L = 0.0f;
+#pragma unroll
+        for (int w = 1; w < kChunkWaves; ++w) M = fmaxf(M, s_m[w][row]);
+#pragma unroll
+        for (int w = 0; w < kChunkWaves; ++w) L += M == -INFINITY ? 0.0f : s_l[w][row] * exp2f((s_m[w][row] - M) * kLog2e);
+        const int pp = a.pos_base + bb;
+        const bool ok = pp >= 0 && pp < a.max_len;
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float x = 0.0f;
+#pragma unroll
+            for (int w = 0; w < SLOTS; ++w) x += s_o[w][((c * 4 + e) * 4 + (row & 3)) * kWave + 16 * (row >> 2) + nn];
+            v[e] = ok ? x / L : 0.0f;
+        }
+        *reinterpret_cast<f32x4*>(a.out + ((int64_t)bb * a.nh + kvh * a.gq + row % a.gq) * D + 4 * col) = v;
+    }
+}
+
+// Launches k_attn_chunk where it is the faster kernel; false: the decode kernel is to take the
+// call (which also reports bad arguments). The decode kernel runs a workgroup per token and kv
+// head, so it loses with the tokens that share their rows, this one while its workgroups leave
+// most CUs idle. Measured (us, decode kernel / this; span: keys seen by the last token): 8 / 4
+// heads x 256: 128 tokens over 128 keys 13.3 / 14.3, 256 over 256 31.6 / 20.4, 100 over 200
+// 18.4 / 18.0, 64 over 364 22.6 / 24.2, 48 over 2548 129 / 112, 512 over 1024 216 / 56; 32 / 16
+// heads x 128: 16 tokens over 116 7.2 / 8.4, 24 over 1024 37 / 27, 64 over 64 11.0 / 7.2, 512
+// over 1024 360 / 84. With 8 heads per kv head two tokens fill the rows: 8 tokens over 108 keys
+// 23 / 13, over 3008 427 / 129 (fewer tokens: 4 over 3004 88 / 129).
+static bool launch_chunk(AttnArgs& a, hipStream_t s) {
+    if (!a.q || !a.kc || !a.vc || !a.out || a.nkv <= 0 || a.nh <= 0 || a.nh % a.nkv != 0 || a.max_len <= 0) return false;
+    a.gq = a.nh / a.nkv;
+    const bool shapes = (a.D == 64 || a.D == 128 || a.D == 256) && (a.gq == 1 || a.gq == 2 || a.gq == 4 || a.gq == 8) &&
+                        (int64_t)a.nkv * a.D <= a.row_stride;
+    const bool aligned = aligned16(a.q) && aligned16(a.out) && aligned16(a.kc) && aligned16(a.vc) && a.row_stride % 4 == 0;
+    if (!shapes || !aligned) return false;
+    const int64_t wgs = cdiv(a.batch, 16 / a.gq) * a.nkv, end = (int64_t)a.pos_base + a.batch;
+    const int64_t span = a.window > 0 ? std::min<int64_t>(a.window, end) : end;
+    const bool faster = a.gq == 8 ? a.batch >= 8 : wgs >= 96 || (wgs >= 48 && span >= 200) || (wgs >= 24 && span >= 2048);
+    if (!faster || wgs > INT32_MAX || end > INT32_MAX) return false;
+    a.inv_cap = a.softcap > 0.0f ? 1.0f / a.softcap : 0.0f;
+    const dim3 grid((unsigned)wgs), threads(kChunkWaves * kWave);
+    if (a.D == 64) k_attn_chunk<64><<<grid, threads, 0, s>>>(a);
+    else if (a.D == 128) k_attn_chunk<128><<<grid, threads, 0, s>>>(a);
+    else k_attn_chunk<256><<<grid, threads, 0, s>>>(a);
+    check_launch();
+    return true;
+}
+
 static AttnArgs base_attn(const float* q, const void* kc, const void* vc, float* out, int n_heads,
                           int n_kv_heads, int head_dim, float scale, float softcap, int window) {
     AttnArgs a{};
@@ -818,7 +1094,7 @@ void hip_attention_batched(const float* q, const float* k_cache, const float* v_
     a.pos_base = pos;
     a.max_len = max_seq;
     a.batch = batch_size;
-    launch_attn(HIP_BRIDGE_F32, a, 0, stream_of(stream));
+    if (!launch_chunk(a, stream_of(stream))) launch_attn(HIP_BRIDGE_F32, a, 0, stream_of(stream));
 }
 
 }  // extern "C"
