@@ -296,8 +296,8 @@ void hip_gemm(int qtype, const void* weights, const float* x, float* y, int batc
  * (one term), so a bf16 norm output feeds the product directly. Q4_0, Q8_0, F16, BF16, F32
  * weights with cols % 32 == 0, Q4_K and Q6_K with cols % 256 == 0; x 16-byte aligned;
  * 128 * cols * sizeof(x element) < 4 GiB; else EUNSUPPORTED. f32 x and y without
- * up_weights is hip_gemm, which takes the matrix cores from 96 tokens for 8192 rows or more,
- * 64 for fewer rows at least 4096 deep, else 128 (Q4_K 128 / 96 / 96, Q6_K 64 / 96 / 96), and
+ * up_weights is hip_gemm, which chooses by type, shape and batch between the matrix-core GEMM
+ * (quantised and BF16 weights of 8192 rows or more from 17-33 tokens, narrower ones from 64-129),
  * the small-batch or vector kernels below. */
 void hip_gemm_ex(int qtype, const void* weights, const void* up_weights /*NULL*/, int x_dtype,
                  const void* x, int y_dtype, void* y, int batch_size, int rows, int cols,

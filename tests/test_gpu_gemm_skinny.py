@@ -1,0 +1,70 @@
+"""Small-batch products (k_gemm_skinny, reached by hip_gemm for the batches and shapes of its launch
+rule) bit-exact on integer-valued operands, where every partial sum is an exact f32 integer times
+a power of two: batches around the 8, 16 and 32 tokens of its operand packings and one past them,
+ragged row tiles, block counts that share out unevenly over the waves and the two K halves. A
+second call gives the same bits (the halves are two addends)."""
+import numpy as np
+import pytest
+
+from test_oracle_gemv_cpu import int_matrix
+from ziglm_amd import bridge as B
+
+pytestmark = pytest.mark.gpu
+
+GROUPED = (B.Q4_0, B.Q4_K, B.Q6_K)
+
+
+def check(dev, qtype, rows, cols, batch):
+    raw, wd = int_matrix(qtype, rows, cols, seed=rows + cols + batch, scale_pow=-1)
+    x = np.random.default_rng(batch).integers(-2, 3, (batch, cols)).astype(np.float32)
+    exact = x.astype(np.float64) @ wd.T
+    assert np.all(np.abs(x).astype(np.float64) @ np.abs(wd).T < 2 ** 23)
+    w, xd = dev.from_numpy(raw), dev.from_numpy(x)
+    got = []
+    for _ in range(2):
+        y = dev.alloc(batch * rows * 4)
+        y.fill(0xAB)
+        dev.gemm(qtype, w, xd, y, batch, rows, cols)
+        got.append(y.to_numpy((batch, rows), np.float32))
+    np.testing.assert_array_equal(got[0], exact.astype(np.float32), err_msg=f"qtype={qtype} {rows}x{cols} b={batch}")
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
+# two K halves: 4096 columns (32 groups of four blocks), 4352 (34: 17 a half, uneven over the waves)
+@pytest.mark.parametrize("qtype,batches", [(q, (5, 8, 9, 16, 17, 31, 33, 128)) for q in GROUPED] +
+                         [(B.Q8_0, (9, 16, 17, 33, 128)), (B.BF16, (17, 32, 64, 128))])
+@pytest.mark.parametrize("rows,cols", [(1, 4096), (33, 4352), (95, 4096)])
+def test_deep(dev, qtype, batches, rows, cols):
+    for batch in batches:
+        check(dev, qtype, rows, cols, batch)
+
+
+# many rows: one and two row tiles per wave, a single group of blocks (128 columns; K-quants two)
+@pytest.mark.parametrize("qtype", GROUPED)
+@pytest.mark.parametrize("rows,cols,batches", [(8193, 256, (3, 7, 8, 9, 15, 17, 32)), (5121, 768, (3, 16, 33, 63)),
+                                               (1537, 256, (9, 17, 65, 127))])
+def test_wide(dev, qtype, rows, cols, batches):
+    for batch in batches:
+        check(dev, qtype, rows, cols, batch)
+
+
+@pytest.mark.parametrize("cols", [128, 384, 640])
+def test_single_groups(dev, cols):
+    for batch in (2, 12, 30):
+        check(dev, B.Q4_0, 8192, cols, batch)
+
+
+def test_infinite_activation_stays_in_its_token(dev):
+    """Packed tokens share an operand's rows with their own other columns only."""
+    rows, cols = 40, 4096
+    raw, wd = int_matrix(B.Q4_0, rows, cols, seed=1, scale_pow=-1)
+    for batch in (6, 12, 20):
+        x = np.random.default_rng(batch).integers(-2, 3, (batch, cols)).astype(np.float32)
+        exact = (x.astype(np.float64) @ wd.T).astype(np.float32)
+        x[3, 1000] = np.inf
+        y = dev.alloc(batch * rows * 4)
+        dev.gemm(B.Q4_0, dev.from_numpy(raw), dev.from_numpy(x), y, batch, rows, cols)
+        got = y.to_numpy((batch, rows), np.float32)
+        keep = np.arange(batch) != 3
+        np.testing.assert_array_equal(got[keep], exact[keep])
+        assert not np.any(np.isfinite(got[3]) & (got[3] == exact[3]))

@@ -1106,6 +1106,249 @@ static void launch_q(const GemmArgs& a, int xk, bool ge, hipStream_t s) {
     }
 }
 
+// ---- small batches -----------------------------------------------------------------------------
+// Products of a few tokens (f32 activations and output): a matrix-vector product's traffic, one
+// read of the weights, with every weight used for up to 32 tokens. A wave takes RT tiles of 32
+// rows over a share of the blocks, alone: weights and activations go from memory straight into
+// its registers in operand layout, blocks ahead of their use, are converted there, and the waves
+// of a workgroup add their sums through the LDS at the end, so there is no barrier in the loop and
+// a wave's round trips overlap. Tokens past the batch repeat the last one.
+// Up to 32 / P tokens leave the A operand's other rows free, and those hold the same tokens' other
+// columns: P = 2 (16 tokens) the block's second MFMA's, P = 4 (8 tokens) the next block's too. An
+// MFMA then gives its own sums in 32 / P of its rows (the rest is dropped), and a lane splits
+// and loads 1 / P of the activations: their split, 5.5 vector instructions a value, is what
+// bounds the kernel beside the weights' conversion.
+template <int QT, int P, int RT>
+__global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
+    constexpr bool SCALED = w_scaled<QT>(), HALVES = QT == HIP_BRIDGE_Q6_K, MIN = QT == HIP_BRIDGE_Q4_K;
+    constexpr int TOK = 32 / P, VR = 16 / P;  // tokens; accumulator registers of an MFMA's own rows
+    constexpr int MAXH = 4;                   // half of the most waves
+    __shared__ __attribute__((aligned(16))) float s_red[MAXH * RT][VR * kWave];
+    const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), ks = (int)blockDim.x / kWave;
+    const int r_base = (int)blockIdx.x * 32 * RT, t_base = (int)blockIdx.y * TOK;
+    // The wave's groups of four blocks: its share of all of them, or with gridDim.z = 2 of half
+    const int ng = a.cols / (4 * kKB);
+    const int z0 = (int)((int64_t)ng * blockIdx.z / gridDim.z), z1 = (int)((int64_t)ng * (blockIdx.z + 1) / gridDim.z);
+    const int g0 = z0 + (int)((int64_t)(z1 - z0) * wave / ks), g1 = z0 + (int)((int64_t)(z1 - z0) * (wave + 1) / ks);
+    const int lastb = 4 * g1 - 1;
+
+    // The lane's columns of a block (P = 4: of a pair of blocks): MFMA s takes xr[2 s], [2 s + 1]
+    // (P = 1) or the only two, the MFMA (and block) given by the lane's row group c / TOK
+    constexpr int XS = P == 1 ? 2 : 1, XB = P == 4 ? 2 : 1;  // MFMAs held apart; blocks per load
+    const int sub = c / TOK;
+    const float* const xrow = (const float*)a.x + (int64_t)min(t_base + c % TOK, a.batch - 1) * a.cols +
+                              (P == 1 ? 0 : wk<QT>(sub & 1, h)) + 32 * (sub >> 1);
+    WSrc ws[RT];
+#pragma unroll
+    for (int j = 0; j < RT; ++j) ws[j].row = a.w + (int64_t)min(r_base + 32 * j + c, a.rows - 1) * a.row_bytes;
+    using WQ = WGrp<QT>;
+    constexpr int G = WQ::G, RING = G == 1 ? 4 : 1;
+    WQ cur[RT], nxt[RING][RT];
+    constexpr int UX = 2;  // activation loads ahead
+    f32x4 xr[UX][XS][2];
+    auto load_x = [&](int kb, f32x4 (&r)[XS][2]) {
+        const float* const p = xrow + 32 * min(kb, lastb + 1 - XB);
+#pragma unroll
+        for (int s = 0; s < XS; ++s) {
+            r[s][0] = ldf4(p + (P == 1 ? wk<QT>(s, h) : 0));
+            r[s][1] = ldf4(p + (P == 1 ? wk<QT>(s, h) : 0) + 4);
+        }
+    };
+    f32x16 acc[RT];
+#pragma unroll
+    for (int j = 0; j < RT; ++j) acc[j] = f32x16{};
+    bf16x8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
+
+    if (g0 < g1) {
+#pragma unroll
+        for (int j = 0; j < RT; ++j)
+#pragma unroll
+            for (int b = 0; b < RING; ++b) nxt[b][j].load(ws[j], min(4 * g0 + b, lastb), h);
+#pragma unroll
+        for (int b = 0; b < UX; ++b) load_x(4 * g0 + XB * b, xr[b]);
+    }
+    for (int g = g0; g < g1; ++g) {
+        bf16x8 xa[XS][3];
+        f32x16 sx;  // (MIN) each row's sum over its columns
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int kb = 4 * g + u;
+            bf16x8 wb[RT][2][1];
+            float dv[RT][2], mn[RT];
+#pragma unroll
+            for (int j = 0; j < RT; ++j) {
+                if (G == 1 || u == 0) {
+                    cur[j] = nxt[G == 1 ? u : 0][j];
+                    cur[j].open();
+                    nxt[G == 1 ? u : 0][j].load(ws[j], G == 1 ? min(kb + 4, lastb) : min(4 * g + 4, 4 * g1 - 4), h);
+                }
+                const int un = G == 1 ? 0 : u;
+                cur[j].scale(un, kb, dv[j], mn[j]);
+                cur[j].template ops<0>(un, wb[j][0]);
+                cur[j].template ops<1>(un, wb[j][1]);
+            }
+            if (u % XB == 0) {
+                f32x4(&xv)[XS][2] = xr[u / XB % UX];
+#pragma unroll
+                for (int s = 0; s < XS; ++s) {
+                    uint32_t v[4][3];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) split3(xv[s][i / 2][2 * (i & 1)], xv[s][i / 2][2 * (i & 1) + 1], v[i]);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) xa[s][q] = __builtin_bit_cast(bf16x8, u32x4{v[0][q], v[1][q], v[2][q], v[3][q]});
+                }
+                load_x(kb + UX * XB, xv);
+                if constexpr (MIN) {
+#pragma unroll
+                    for (int s = 0; s < XS; ++s)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q)
+                            sx = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[s][q], ones, s + q ? sx : f32x16{}, 0, 0, 0);
+                }
+            }
+            // Chains of MFMAs: both of the block's (P = 1 with one scale), or one each, of which
+            // the registers [v0, v0 + VR) are its own
+#pragma unroll
+            for (int j = 0; j < RT; ++j) {
+                f32x16 part;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const bool start = s == 0 || HALVES || P > 1;
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[s % XS][q], wb[j][s][0],
+                                                                       q == 0 && start ? f32x16{} : part, 0, 0, 0);
+                    if (HALVES || P > 1 || s == 1) {
+                        const int v0 = P == 1 ? 0 : VR * (P == 4 ? 2 * (u & 1) + s : s);
+#pragma unroll
+                        for (int r = v0; r < v0 + VR; ++r) {
+                            if constexpr (MIN) acc[j][r] = fmaf(-mn[j], sx[r], acc[j][r]);
+                            acc[j][r] = SCALED ? fmaf(dv[j][HALVES ? s : 0], part[r], acc[j][r]) : acc[j][r] + part[r];
+                        }
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // (else the loads sink to their uses)
+        }
+    }
+    // the row groups' sums
+#pragma unroll
+    for (int j = 0; j < RT; ++j)
+#pragma unroll
+        for (int r = 0; r < VR; ++r)
+#pragma unroll
+            for (int i = 1; i < P; ++i) acc[j][r] += acc[j][i * VR + r];
+
+    // The waves' sums: the upper half's through the LDS into the lower half's, then those in wave
+    // order.
+    const int half = (ks + 1) / 2;
+    if (wave >= half) {
+#pragma unroll
+        for (int j = 0; j < RT; ++j)
+#pragma unroll
+            for (int r = 0; r < VR; ++r) s_red[(wave - half) * RT + j][r * kWave + lane] = acc[j][r];
+    }
+    __syncthreads();
+    if (wave < half) {
+#pragma unroll
+        for (int j = 0; j < RT; ++j)
+#pragma unroll
+            for (int r = 0; r < VR; ++r) {
+                float* const p = &s_red[wave * RT + j][r * kWave + lane];
+                *p = wave + half < ks ? acc[j][r] + *p : acc[j][r];
+            }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < RT * VR * kWave; i += (int)blockDim.x) {
+        const int tile = i / (VR * kWave), r = i / kWave % VR, l = i % kWave;
+        float v = s_red[tile][i % (VR * kWave)];
+        for (int w = 1; w < half; ++w) v += s_red[w * RT + tile][i % (VR * kWave)];
+        // register r of lane l: token 8 (r / 4) + 4 (l / 32) + r % 4, row l % 32
+        const int tok = t_base + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
+        const int row = r_base + 32 * tile + (l & 31);
+        if (tok >= a.batch || row >= a.rows) continue;
+        float* const y = (float*)a.y + (int64_t)tok * a.rows + row;
+        if (gridDim.z > 1) unsafeAtomicAdd(y, v);  // two halves into zeroed y: 0 + a + b in either order
+        else *y = v;
+    }
+}
+
+// Row tiles per wave, waves and K halves. n1, n2: workgroups at one and two row tiles. Measured, us
+// (Q4_0 unless said): 10240 x 2560, 8 tokens: one tile and 4 / 8 waves 12.0 / 13.8, two tiles
+// 13.0; 16 tokens 16.1 / 17.9, 15.2; 32 tokens 25.5 / 28.1, 20.1 (two tiles share a split of x,
+// worth it once that is large). 2560 x 10240, two halves added into zeroed y: 8 tokens 15.0, one
+// tile and no halves 20.3; 48 tokens 45.7, two tiles 35.5; at 128 tokens two tiles fill the chip
+// without halves, 57.3 against 66.6. 2048 x 2560, 16 tokens: 4 / 8 waves 8.7 / 9.6, halves 8.9;
+// 48 tokens 15.0, halves 12.3.
+template <int QT>
+static void launch_skinny_t(const GemmArgs& a, hipStream_t s) {
+    const int ng = a.cols / (4 * kKB);
+    const int p = a.batch > 16 ? 1 : a.batch > 8 ? 2 : 4;
+    const int64_t ttiles = cdiv(a.batch, 32 / p), n1 = cdiv(a.rows, 32) * ttiles, n2 = cdiv(a.rows, 64) * ttiles;
+    const bool deep = a.cols >= kSplitMinCols;
+    const int rt = deep ? (n1 >= 160 ? 2 : 1) : (p < 4 && n2 >= 160 ? 2 : 1);
+    const unsigned kz = (deep ? (rt == 2 ? n2 : n1) : p == 1 ? n1 : 1024) < 160 ? 2 : 1;
+    const int most = rt == 1 && kz == 1 ? 4 : 8;
+    const int half = (int)cdiv(ng, (int)kz), share = (int)cdiv(half, most);  // groups of a half, of a wave
+    const int ks = (int)cdiv(half, share);
+    if (kz > 1) launch_zero_f32((float*)a.y, (int64_t)a.batch * a.rows, s);
+    const dim3 grid((unsigned)cdiv(a.rows, 32 * rt), (unsigned)ttiles, kz);
+    auto go = [&](auto p_c) {
+        constexpr int PC = decltype(p_c)::value;
+        if (rt == 1) k_gemm_skinny<QT, PC, 1><<<grid, ks * kWave, 0, s>>>(a);
+        else k_gemm_skinny<QT, PC, 2><<<grid, ks * kWave, 0, s>>>(a);
+    };
+    if (p == 1) go(std::integral_constant<int, 1>{});
+    else if (p == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 4>{});
+}
+
+// Where k_gemm_skinny is the fastest path for f32 x and y: below it the vector kernels and
+// k_gemv_mb, above it k_gemm_mfma, which takes over early where the rows alone fill the chip
+// (gemm_mfma_min_batch). us, this kernel / the best other, at n rows x columns:
+//   Q4_0, Q4_K, Q6_K: at least 8192 rows to 32 tokens (10240 x 2560: Q4_0 2 tokens 11.7 / 18.3, 24
+//     19.4 / 23.5, 40 32.4 / 25.7; Q6_K 2 tokens 16.1 / 13.1, 4 16.3 / 21.4; 262144 x 2560 Q6_K 4
+//     tokens 247 / 471); at least 5120 to 64 tokens (6144 x 1536 Q4_K 64: 16.4 / 21.0, 128 30.5 /
+//     24.5); deep ones from 5 to 128 tokens (2560 x 10240 Q4_0 4 tokens 13.6 / 12.4, 8 15.0 / 21.1,
+//     96 36.2 / 78.9, 128 57.3 / 78.4); the rest from 9 tokens on 1536 rows (2048 x 2560: 2 tokens
+//     7.2 / 7.3, 16 8.7 / 10.0, 80 15.6 / 20.9; 256 x 1536 10 / 6);
+//   Q8_0 and BF16, whose 32-column blocks take a load each: deep products of 9 (17) to 128 tokens
+//     (2560 x 10240: Q8_0 4 tokens 25 / 16, 20 37.6 / 58.5, 80 61 / 93; BF16 16 tokens 26.0 / 23.4, 24
+//     32.8 / 37.3, 48 48.0 / 42.1, 80 48.3 / 70.4, so not between 33 and 63).
+static bool skinny_range(int qtype, int rows, int cols, int batch) {
+    const bool groups = qtype == HIP_BRIDGE_Q4_0 || qtype == HIP_BRIDGE_Q4_K || qtype == HIP_BRIDGE_Q6_K;
+    const bool deep = cols >= kSplitMinCols && rows < kWideRows;
+    if (qtype == HIP_BRIDGE_Q8_0) return deep && batch >= 9 && batch <= 128;
+    if (qtype == HIP_BRIDGE_BF16) return deep && ((batch >= 17 && batch <= 32) || (batch >= 64 && batch <= 128));
+    if (!groups) return false;
+    if (deep) return batch >= 5 && batch <= 128;
+    if (rows >= kMidRows) return batch >= (qtype == HIP_BRIDGE_Q6_K ? 3 : 2) && batch <= (rows >= kWideRows ? 32 : 64);
+    return rows >= 1536 && batch >= 9 && batch <= 127;
+}
+
+// Small-batch product, f32 x and y; false: not a shape, type or batch of this kernel (nothing
+// launched).
+bool launch_gemm_skinny(int qtype, const void* w, int64_t row_bytes, const float* x, float* y, int rows, int cols,
+                        int batch, hipStream_t s) {
+    const bool kq = qtype == HIP_BRIDGE_Q4_K || qtype == HIP_BRIDGE_Q6_K;
+    const uintptr_t wa = reinterpret_cast<uintptr_t>(w);
+    if (!skinny_range(qtype, rows, cols, batch) || !w || !x || !y) return false;
+    if (!aligned16(x) || cols % (kq ? 256 : 4 * kKB) != 0 || wa % (qtype == HIP_BRIDGE_BF16 ? 16 : 2) != 0) return false;
+    const GemmArgs a{(const unsigned char*)w, nullptr, x, y, row_bytes, rows, cols, batch, 0};
+    switch (qtype) {
+        case HIP_BRIDGE_Q4_0: launch_skinny_t<HIP_BRIDGE_Q4_0>(a, s); break;
+        case HIP_BRIDGE_Q8_0: launch_skinny_t<HIP_BRIDGE_Q8_0>(a, s); break;
+        case HIP_BRIDGE_BF16: launch_skinny_t<HIP_BRIDGE_BF16>(a, s); break;
+        case HIP_BRIDGE_Q4_K: launch_skinny_t<HIP_BRIDGE_Q4_K>(a, s); break;
+        default: launch_skinny_t<HIP_BRIDGE_Q6_K>(a, s); break;
+    }
+    check_launch();
+    return true;
+}
+
 // 0 = launched; otherwise why not (the caller decides between a fallback and an error).
 int launch_gemm_mfma_ex(int qtype, const void* w, const void* wu, int64_t row_bytes, int x_dtype, const void* x,
                         int y_dtype, void* y, int rows, int cols, int batch, hipStream_t s) {

@@ -2206,6 +2206,10 @@ extern "C" {
 void hip_gemm(int qtype, const void* weights, const float* x, float* y, int batch_size, int rows,
               int cols, HipStream_t stream) {
     if (batch_size <= 0 || rows <= 0 || cols <= 0) return;
+    if (batch_size > 1) {
+        const int64_t rb = gemv_row_bytes(qtype, cols);
+        if (rb > 0 && launch_gemm_skinny(qtype, weights, rb, x, y, rows, cols, batch_size, stream_of(stream))) return;
+    }
     if (batch_size >= gemm_mfma_min_batch(qtype, rows, cols) && weights && x) {
         const int64_t rb = gemv_row_bytes(qtype, cols);
         if (rb > 0 && launch_gemm_mfma(qtype, weights, rb, x, y, rows, cols, batch_size, stream_of(stream))) return;

@@ -49,31 +49,31 @@ inline int device_cus() {
 // path).
 // Products at least this deep count as deep for the split of K in two halves (gemm.hip).
 constexpr int kSplitMinCols = 4096;
-// The matrix-core kernel's smallest workgroup tile is 64 tokens x 64 rows, so below a few
-// hundred tiles it leaves most of the chip idle (2560 x 10240 at up to 128 tokens: 40-80
-// workgroups; split in two K halves ~130 us for Q4_0 whatever the batch), while the vector
-// kernels' time grows with the batch. The batch from which it wins, measured per type on
-// 10240 x 2560 (160 row tiles: "wide") and 2560 x 10240 (40, deep enough to split) products:
-// Q4_0 / Q8_0 96 / 64, Q4_K 128 / 96 (against the small-batch kernel: 44 / 86 us at 64 tokens,
-// the matrix cores 73 / 136), Q6_K 64 / 96 (small-batch kernel at 48 tokens 73 / 80 us, matrix
-// cores 86 / 173); narrow products too shallow to split keep the unsplit crossovers (128, 96,
-// 96).
+// Rows from which 32-row tiles alone fill the chip's CUs, and most of them.
+constexpr int kWideRows = 8192, kMidRows = 5120;
 // y[0, n) = 0 (a kernel, not hipMemsetAsync, so that graph captures of the products that
 // add into y replay correctly)
 void launch_zero_f32(float* y, int64_t n, hipStream_t s);
-#ifndef ZL_GEMM_MIN_BATCH
-#define ZL_GEMM_MIN_BATCH 0
-#endif
+// The batch from which the matrix-core GEMM (k_gemm_mfma; F16, F32: k_gemm_dense) is faster than
+// the kernels for smaller ones, where k_gemm_skinny does not take the call. Wide products (us,
+// 10240 x 2560, GEMM / k_gemm_skinny / k_gemv_mb): Q4_0 24 tokens 23.5 / 19.4 / 39.3, 40 tokens
+// 25.7 / 32.4 / 40.4; Q4_K 40 31.7 / 39.0 / 32.9; Q6_K 40 34.2 / 43.8 / 72.0; Q8_0 24 24.5 / 26.0 /
+// 39.8; BF16 24 22.0 / 26.3 / 29.3. 6144 x 1536 Q4_K: 45 tokens 18.1 / 15.5 / 21.0, 128 24.5 / 30.5.
+// Narrower ones keep the crossovers of the GEMM against k_gemv_mb and the vector kernels: from 64
+// tokens where deep enough to run in two K halves, else 128 (K-quants 96).
 inline int gemm_mfma_min_batch(int qtype, int rows, int cols) {
-    if (ZL_GEMM_MIN_BATCH) return ZL_GEMM_MIN_BATCH;
-    const bool wide = rows >= 128 * 64;  // enough row tiles to fill half the chip's workgroup slots
     const bool deep = cols >= kSplitMinCols;
-    if (qtype == HIP_BRIDGE_Q4_K) return wide ? 128 : 96;
-    if (qtype == HIP_BRIDGE_Q6_K) return wide ? 64 : 96;
-    return wide ? 96 : deep ? 64 : 128;
+    const bool kq = qtype == HIP_BRIDGE_Q4_K || qtype == HIP_BRIDGE_Q6_K;
+    if (qtype == HIP_BRIDGE_F16 || qtype == HIP_BRIDGE_F32) return rows >= kWideRows ? 96 : deep ? 64 : 128;
+    const bool single = qtype == HIP_BRIDGE_Q8_0 || qtype == HIP_BRIDGE_BF16;
+    if (rows >= kWideRows) return single ? 17 : 33;
+    if (rows >= kMidRows && !deep) return single ? 33 : 65;
+    return kq ? 96 : deep ? 64 : 128;
 }
 bool launch_gemm_mfma(int qtype, const void* w, int64_t row_bytes, const float* x, float* y, int rows, int cols,
                       int batch, hipStream_t s);
+bool launch_gemm_skinny(int qtype, const void* w, int64_t row_bytes, const float* x, float* y, int rows, int cols,
+                        int batch, hipStream_t s);
 // The same for any batch with f32 or bf16 activations and output and an optional up matrix
 // (y = gelu(W x) * (U x)); returns 0 when launched, else a HIP_BRIDGE_* code (nothing launched).
 int launch_gemm_mfma_ex(int qtype, const void* w, const void* wu, int64_t row_bytes, int x_dtype, const void* x,
