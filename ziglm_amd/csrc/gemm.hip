@@ -33,23 +33,24 @@
 // 2^-24 of a product, so a dot product lies within the f32 rounding of the sum, like the
 // decode GEMV's.
 //
-// Tiling. A workgroup of 4 waves owns 32 WT tokens x 128 WR rows; wave w computes all of the
-// tokens for its own 32 WR rows, as WT x WR tiles of v_mfma_f32_32x32x16_bf16 (tokens on the A
-// side, so a lane's accumulators are one weight row: the block scale is one value per lane and
-// tile, and stores of 32 lanes are 128 contiguous bytes of a token's output row). No two waves
-// share a weight row, so a lane loads the codes of its row straight into registers in the
+// Tiling (k_gemm_mfma). A workgroup of 4 waves owns 32 WT tokens x 128 RT rows; a wave computes
+// all of the tokens for its own 32 RT rows, as WT x RT tiles of v_mfma_f32_32x32x16_bf16 (tokens
+// on the A side, so a lane's accumulators are one weight row: the block scale is one value per
+// lane and tile, and stores of 32 lanes are 128 contiguous bytes of a token's output row). No two
+// waves share a weight row, so a lane loads the codes of its row straight into registers in the
 // B-operand layout and converts them there, once per workgroup, and only the activations go
 // through the LDS: a step's LDS reads are the activation terms alone (staged through the LDS
 // the weights were half of them, and their loop ran at 2-3 times the LDS traffic of this one).
-// With GE the wave's first tile column is 32 gate rows and its second the same 32 up rows, so
-// gelu(gate) * up needs no exchange.
+// With GE a tile's 32 columns are 16 gate rows and the same 16 up rows, so gelu(gate) * up takes
+// one lane shuffle.
 // The K loop takes one 32-column block per step. The LDS holds block k as bf16 terms (rows
-// padded to 80 bytes against bank conflicts) in one of two buffers while the registers hold the
-// raw bytes of the next blocks (UX activation and UW weight blocks ahead, more for the smaller
-// tiles, whose steps are shorter than a memory round trip); block k + 1 is converted into the
-// other buffer during block k's MFMAs, so a step takes one barrier. Activations load through a
-// range-checked resource (tokens past the batch read zeros); weight rows past the end are the
-// last row again, and nothing of them is stored.
+// permuted against bank conflicts, lds_chunk) in one of two buffers while the registers hold the
+// raw bytes of the next blocks (more activation blocks ahead for the smaller tiles, whose steps
+// are shorter than a memory round trip); block k + 1 is converted into the other buffer during
+// block k's MFMAs, so a step takes one barrier. Activations load through a range-checked resource
+// (tokens past the batch read zeros); weight rows past the end are the last row again, and nothing
+// of them is stored. F16 and F32 weights are staged through the LDS instead (k_gemm_dense), and a
+// few tokens take k_gemm_skinny.
 #include "zl_common.h"
 #include "zl_host.h"
 
@@ -1117,7 +1118,9 @@ static void launch_q(const GemmArgs& a, int xk, bool ge, hipStream_t s) {
 // columns: P = 2 (16 tokens) the block's second MFMA's, P = 4 (8 tokens) the next block's too. An
 // MFMA then gives its own sums in 32 / P of its rows (the rest is dropped), and a lane splits
 // and loads 1 / P of the activations: their split, 5.5 vector instructions a value, is what
-// bounds the kernel beside the weights' conversion.
+// bounds the kernel beside the weights' conversion, not the loads' latency: two groups of weights or
+// four activation loads ahead are slower nearly everywhere (10240 x 2560 Q4_0, weights not in cache, 8 tokens
+// 13.5 -> 14.3 / 15.1 us; 2560 x 10240 Q6_K, 45 tokens 45 -> 53 / 46).
 template <int QT, int P, int RT>
 __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
     constexpr bool SCALED = w_scaled<QT>(), HALVES = QT == HIP_BRIDGE_Q6_K, MIN = QT == HIP_BRIDGE_Q4_K;
