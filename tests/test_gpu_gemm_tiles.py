@@ -65,3 +65,20 @@ def test_large_tiles(dev):
     y = dev.alloc(batch * rows * 4)
     dev.gemmEx(B.Q4_0, dev.from_numpy(raw), None, B.F32, dev.from_numpy(x), B.F32, y, batch, rows, cols)
     np.testing.assert_array_equal(y.to_numpy((batch, rows), np.float32), exact.astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype", [B.Q4_0, B.Q8_0, B.BF16, B.Q4_K, B.Q6_K])
+@pytest.mark.parametrize("cols", [992, 1024, 1056, 1248, 1280, 2816])
+def test_k_shares(dev, qtype, cols):
+    """K in two shares per workgroup, and from 32 blocks in four (two of them added into zeroed y):
+    31 blocks (16 + 15), 32, 33, 39 (16 + 8 + 8 + 7), 40 and 88, on few and on more tiles."""
+    if qtype in (B.Q4_K, B.Q6_K) and cols % 256:
+        pytest.skip("K-quant rows are whole super-blocks")
+    for rows, batch in ((33, 129), (1025, 700)):
+        raw, x, exact = operands(qtype, rows, cols, batch, rows + cols)
+        assert np.all(np.abs(exact) < 2 ** 24)
+        w, xd, y = dev.from_numpy(raw), dev.from_numpy(x), dev.alloc(batch * rows * 4)
+        for _ in range(2):
+            y.fill(0xAB)
+            dev.gemmEx(qtype, w, None, B.F32, xd, B.F32, y, batch, rows, cols)
+            np.testing.assert_array_equal(y.to_numpy((batch, rows), np.float32), exact.astype(np.float32))

@@ -395,9 +395,11 @@ constexpr int x_ahead() {
     return WT >= 4 ? 1 : WT >= 2 ? 2 : 4;
 }
 
-template <int QT, int XK, int WT, int RT, int WAVES, bool GE>
-__global__ __launch_bounds__(64 * WAVES, 2) void k_gemm_mfma(GemmArgs a) {
-    constexpr int NT = 64 * WAVES;             // threads
+// TEAMS = 2: a second set of WAVES waves takes the other half of the workgroup's K steps, with LDS
+// buffers of its own, and its sums join the first's through the LDS at the end.
+template <int QT, int XK, int WT, int RT, int WAVES, bool GE, int TEAMS>
+__global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a) {
+    constexpr int NT = 64 * WAVES;             // threads of a team
     constexpr int XT = XK == X_BF16 ? 1 : 3;  // activation terms
     constexpr int NW = w_terms<QT>();
     constexpr bool SCALED = w_scaled<QT>();
@@ -410,20 +412,23 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm_mfma(GemmArgs a) {
     // planes: one per plane, added in plane order), four steps' worth.
     constexpr bool MIN = QT == HIP_BRIDGE_Q4_K;
     constexpr int XSP = XK == X_TERMS ? 3 : 1;  // sum planes
-    __shared__ __attribute__((aligned(16))) uint16_t s_x[2 * XT * XPLANE];
-    __shared__ __attribute__((aligned(16))) float s_xs[MIN ? 4 : 1][MIN ? XSP * BT : 1];
+    __shared__ __attribute__((aligned(16))) uint16_t s_x_all[TEAMS * 2 * XT * XPLANE];
+    __shared__ __attribute__((aligned(16))) float s_xs_all[TEAMS][MIN ? 4 : 1][MIN ? XSP * BT : 1];
 
-    const int tid = threadIdx.x;
+    const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+    const int tid = (int)threadIdx.x - team * NT;
+    uint16_t* const s_x = s_x_all + team * (2 * XT * XPLANE);
+    auto& s_xs = s_xs_all[team];
     const int lane = tid & 63, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int gx = (a.rows + OR - 1) / OR;
     const int r_base = ((int)blockIdx.x % gx) * OR, b_base = ((int)blockIdx.x / gx) * BT;
-    // K steps [kbb, kbe): all of them, or with a split launch (gridDim.y = 2, f32 output,
-    // added into zeroed y) one half per workgroup row, cut between super-blocks
-    const int nkb_all = a.cols / kKB;
-    const int mid = gridDim.y > 1 ? (nkb_all / 2 + 7) & ~7 : nkb_all;
-    const int kbb = blockIdx.y ? mid : 0;
-    const int kbe = blockIdx.y ? nkb_all : mid;
+    // K steps [kbb, kbe): the share of this team and (gridDim.y = 2, f32 output, added into zeroed y)
+    // workgroup row, cut between super-blocks; `steps`, of the team that has the most.
+    const int nkb_all = a.cols / kKB, parts = (int)gridDim.y * TEAMS, p0 = (int)blockIdx.y * TEAMS;
+    auto cut = [&](int p) { return p == parts ? nkb_all : (int)((int64_t)nkb_all * p / parts + 7) & ~7; };
+    const int kbb = cut(p0 + team), kbe = cut(p0 + team + 1);
+    const int steps = TEAMS == 1 ? kbe - kbb : max(cut(p0 + 1) - cut(p0), cut(p0 + TEAMS) - cut(p0 + TEAMS - 1));
 
     // X staging. f32 x: chunk c = tid + NT i is token c / 8, columns 4 (c % 8) .. (four
     // floats); bf16 x: token c / 4, columns 8 (c % 4) .. (eight bf16); term planes: the same
@@ -656,14 +661,28 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm_mfma(GemmArgs a) {
     __syncthreads();
     // A branch per step keeps each in a basic block of its own: unrolled into one, instruction
     // selection moves the scale products of several steps together, and their partial sums spill.
-    for (int k0 = kbb; k0 < kbe; k0 += U) {
+    for (int k0 = kbb; k0 < kbb + steps; k0 += U) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
             if (k0 + u < kbe) step(u, k0 + u);  // uniform
+            else if (TEAMS > 1 && k0 + u < kbb + steps) __syncthreads();  // the other team's step
+        }
     }
     if constexpr (SCALED) {  // the last unit's scale products
         if ((kbe - kbb) & 1) scale_unit(UNITS - 1, part[(UNITS - 1) & 1], 0, kbe - 1, 0, 16);
         else scale_unit(UNITS - 1, part[(UNITS - 1) & 1], 1, kbe - 1, 0, 16);
+    }
+
+    if constexpr (TEAMS > 1) {
+        static_assert(TEAMS == 2 && sizeof(s_x_all) >= sizeof(acc) * NT);
+        float* const sums = reinterpret_cast<float*>(s_x_all) + tid;  // (every step's barrier is behind)
+#pragma unroll
+        for (int q = 0; q < WT * RT * 16; ++q)
+            if (team) sums[q * NT] = acc[q / 16 / RT][q / 16 % RT][q % 16];
+        __syncthreads();
+        if (team) return;
+#pragma unroll
+        for (int q = 0; q < WT * RT * 16; ++q) acc[q / 16 / RT][q / 16 % RT][q % 16] += sums[q * NT];
     }
 
     // Epilogue: lane (l, r) of tile (i, j) holds token 8 (r / 4) + 4 (l / 32) + r % 4 and row
@@ -708,11 +727,11 @@ static unsigned split_k(const GemmArgs& a, bool ge, bool want, hipStream_t s) {
     return 2;
 }
 
-template <int QT, int XK, bool GE, int WT, int RT>
+template <int QT, int XK, bool GE, int WT, int RT, int TEAMS = 1>
 static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
     constexpr int W = 4;
     const dim3 grid((unsigned)(cdiv(a.rows, (GE ? 16 : 32) * W * RT) * cdiv(a.batch, 32 * WT)), ky);
-    k_gemm_mfma<QT, XK, WT, RT, W, GE><<<grid, 64 * W, 0, s>>>(a);
+    k_gemm_mfma<QT, XK, WT, RT, W, GE, TEAMS><<<grid, 64 * W * TEAMS, 0, s>>>(a);
 }
 // Workgroup tile (tokens x rows; GE: half the output rows), for 256 CUs that hold two workgroups
 // each. Large tiles convert an operand for more MFMAs, small ones fill the chip:
@@ -726,6 +745,13 @@ static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
 // x 2560 39 -> 32 us, 1024 rows 38 -> 26), or four times for deep products (2560 x 10240 x 2048:
 // 365 -> 341 us; at 333 tokens Q6_K 168 -> 117); at 333 tokens of 10240 x 2560 (480 tiles) the
 // halves cost more than they fill (87 -> 97 us).
+// Up to 128 tiles two halves leave each CU one workgroup or none, one wave per SIMD and a step's
+// latency bare: each half then runs as two teams. us, without / with: 2560 x 10240 at 150 tokens Q4_0
+// 85 / 63, Q4_K 101 / 78, Q8_0 98 / 82, Q6_K 98 / 86; 1024 x 2560 at 512 tokens Q4_0 25.5 / 22.7, Q4_K
+// 29.0 / 26.2, Q8_0 25.2 / 23.3; 2048 x 2560 at 200 tokens Q4_0 24.1 / 21.2, Q6_K 27.7 / 28.3 (so deep
+// ones only), BF16 25.5 / 28.2 (none); from 140 tiles on they lose (2048 x 2560 at 333 tokens 26.9 /
+// 28.5; Q4_K 2560 x 10240 119 / 146). Pre-split planes take the same shares, so that they give the same
+// sums (2560 x 10240 at 150 tokens Q4_0 73 / 62, Q4_K 123 / 95; 1024 x 2560 at 512 Q4_0 24.5 / 25.1).
 template <int QT, int XK, bool GE>
 static void launch_qt(const GemmArgs& a, hipStream_t s) {
     constexpr bool BIG = XK != X_BF16 && !GE && (QT == HIP_BRIDGE_Q4_0 || QT == HIP_BRIDGE_BF16);
@@ -733,6 +759,14 @@ static void launch_qt(const GemmArgs& a, hipStream_t s) {
     const bool big = BIG && wgs(2, 2) >= 768;
     const int wt = XK == X_BF16 && wgs(4, 1) >= 384 ? 4 : big || wgs(2, 1) >= 384 ? 2 : 1;
     const int64_t n = wgs(wt, big ? 2 : 1);
+    constexpr bool SHARES = XK != X_BF16 && !GE && QT != HIP_BRIDGE_BF16 && QT != kQ4_0Odd;
+    if constexpr (SHARES) {
+        const bool pays = QT != HIP_BRIDGE_Q6_K || a.cols >= kSplitMinCols;
+        if (wt == 1 && n <= 128 && pays && !a.y_bf16 && a.cols >= 32 * kKB) {
+            launch_tile<QT, XK, GE, 1, 1, 2>(a, split_k(a, GE, true, s), s);
+            return;
+        }
+    }
     const unsigned ky = split_k(a, GE, n < 384 || (n < 1024 && a.cols >= kSplitMinCols), s);
     if constexpr (BIG) {
         if (big) {
