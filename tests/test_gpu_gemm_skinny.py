@@ -68,3 +68,34 @@ def test_infinite_activation_stays_in_its_token(dev):
         keep = np.arange(batch) != 3
         np.testing.assert_array_equal(got[keep], exact[keep])
         assert not np.any(np.isfinite(got[3]) & (got[3] == exact[3]))
+
+
+# columns past 5120 (10240) and tokens below: products that the vector kernels can also take
+@pytest.mark.parametrize("qtype,rows,cols,batch", [(B.Q6_K, 8192, 256, 3), (B.Q6_K, 8192, 256, 7), (B.Q6_K, 40, 4352, 6),
+                                                   (B.Q8_0, 40, 5376, 9), (B.BF16, 40, 10752, 17), (B.Q4_0, 40, 4352, 5),
+                                                   (B.Q4_K, 40, 4352, 20), (B.Q6_K, 40, 4352, 33)])
+def test_infinite_activations_give_what_f32_gives(dev, qtype, rows, cols, batch):
+    """An infinite activation times a weight is an infinity of the product's sign (NaN for a zero
+    weight, or where infinities of both signs meet), as in f32 arithmetic on the values; a value past
+    bf16's largest is finite; the other tokens keep their exact sums."""
+    some = min(rows, 64)  # different rows, repeated
+    raw, wd = int_matrix(qtype, some, cols, seed=rows + cols, scale_pow=-1)
+    raw, wd = np.tile(raw, (rows // some, 1)), np.tile(wd, (rows // some, 1))
+    x = np.random.default_rng(batch).integers(-2, 3, (batch, cols)).astype(np.float32)
+    keep = np.arange(3, batch)
+    exact = x.astype(np.float64) @ wd.T
+    x[0, cols - 7] = np.inf
+    x[1, 5] = -np.inf
+    x[1, cols // 2] = np.inf
+    x[2] = 0
+    x[2, 77] = np.float32(3.4e38)  # (bf16 rounds it to infinity); with f32 sums: w * x
+    with np.errstate(invalid="ignore"):
+        want = np.stack([np.inf * wd[:, cols - 7], -np.inf * wd[:, 5] + np.inf * wd[:, cols // 2]]).astype(np.float32)
+    with np.errstate(over="ignore"):
+        big = (wd[:, 77] * np.float64(x[2, 77])).astype(np.float32)
+    y = dev.alloc(batch * rows * 4)
+    dev.gemm(qtype, dev.from_numpy(raw), dev.from_numpy(x), y, batch, rows, cols)
+    got = y.to_numpy((batch, rows), np.float32)
+    np.testing.assert_array_equal(got[:2], want)
+    np.testing.assert_array_equal(got[2], big)
+    np.testing.assert_array_equal(got[keep], exact[keep].astype(np.float32))

@@ -357,6 +357,43 @@ struct WGrp<HIP_BRIDGE_BF16> {
     }
     __device__ __forceinline__ void scale(int, int, float (&)[2], float&) const {}
 };
+// sum of w[c] * x[c] over columns [c0, c1) of a weight row, one column at a time: for sums that are
+// not finite. An infinite x (or one that bf16 rounds to infinity) has the terms inf, inf - inf,
+// inf - inf, so every product of its token is NaN on the matrix cores, and a block's sum of unscaled
+// codes can overflow where the scaled products do not; this gives what f32 arithmetic on the values
+// gives. Serial, some ms a call: the price of a result that has to be looked at, not of a usual one.
+template <int QT>
+__device__ float dot_columns(const unsigned char* row, const float* x, int c0, int c1) {
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int c = c0; c < c1; ++c) {
+        float w;
+        if constexpr (QT == HIP_BRIDGE_BF16) {
+            w = bf16_lo(*(const uint16_t*)(row + 2 * (int64_t)c));
+        } else if constexpr (QT == HIP_BRIDGE_Q8_0) {
+            const unsigned char* b = row + (int64_t)(c / 32) * 34;
+            w = (float)(int8_t)b[2 + c % 32] * f16_bits_to_f32(*(const uint16_t*)b);
+        } else if constexpr (QT == HIP_BRIDGE_Q4_K) {  // (layouts: WGrp)
+            const unsigned char* b = row + (int64_t)(c / 256) * 144;
+            const int j = c / 32 % 8, s0 = b[4 + j % 4], s1 = b[8 + j % 4], s2 = b[12 + j % 4];
+            const int sc = j < 4 ? s0 & 63 : (s2 & 15) | (s0 >> 6) << 4, m = j < 4 ? s1 & 63 : s2 >> 4 | (s1 >> 6) << 4;
+            const int q = b[16 + 32 * (j / 2) + c % 32] >> (4 * (j & 1)) & 15;
+            w = f16_bits_to_f32(*(const uint16_t*)b) * (float)sc * (float)q - f16_bits_to_f32(*(const uint16_t*)(b + 2)) * (float)m;
+        } else if constexpr (QT == HIP_BRIDGE_Q6_K) {
+            const unsigned char* b = row + (int64_t)(c / 256) * 210;
+            const int n = c / 128 % 2, t = c / 32 % 4, l = c % 32;
+            const int u = (b[64 * n + 32 * (t & 1) + l] >> (t < 2 ? 0 : 4) & 15) | (b[128 + 32 * n + l] >> (2 * t) & 3) << 4;
+            w = f16_bits_to_f32(*(const uint16_t*)(b + 208)) * (float)(int8_t)b[192 + 8 * n + l / 16 + 2 * t] * (float)(u - 32);
+        } else {
+            const unsigned char* b = row + (int64_t)(c / 32) * 18;
+            const int j = c % 32, q = b[2 + j % 16] >> (j < 16 ? 0 : 4) & 15;
+            w = (float)(q - 8) * f16_bits_to_f32(*(const uint16_t*)b);
+        }
+        sum = fmaf(w, x[c], sum);
+    }
+    return sum;
+}
+
 // The (x term, w term) products accumulated, largest first: down to relative size 2^-16
 // (x in XT terms: 3 for f32 activations, 1 for bf16 ones, which are exact).
 template <int XT, int NW>
@@ -1307,6 +1344,9 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
         const int tok = t_base + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
         const int row = r_base + 32 * tile + (l & 31);
         if (tok >= a.batch || row >= a.rows) continue;
+        if (!(fabsf(v) < INFINITY))
+            v = dot_columns<QT>(a.w + (int64_t)row * a.row_bytes, (const float*)a.x + (int64_t)tok * a.cols, 4 * kKB * z0,
+                                4 * kKB * z1);
         float* const y = (float*)a.y + (int64_t)tok * a.rows + row;
         if (gridDim.z > 1) unsafeAtomicAdd(y, v);  // two halves into zeroed y: 0 + a + b in either order
         else *y = v;
