@@ -99,3 +99,25 @@ def test_infinite_activations_give_what_f32_gives(dev, qtype, rows, cols, batch)
     np.testing.assert_array_equal(got[:2], want)
     np.testing.assert_array_equal(got[2], big)
     np.testing.assert_array_equal(got[keep], exact[keep].astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype,rows,cols,batches",
+                         [(q, 40, 4352, (5, 9, 20, 64, 96, 128)) for q in GROUPED] + [(q, 5121, 512, (5, 16, 40)) for q in GROUPED] +
+                         [(B.Q8_0, 40, 4352, (9, 20, 64, 96, 128)), (B.BF16, 40, 4352, (64, 96, 128))] +
+                         [(q, 2561, 4096, (65, 128)) for q in (*GROUPED, B.Q8_0, B.BF16)])
+def test_split_activations_give_the_same_bits(dev, qtype, rows, cols, batches):
+    """Activations split beforehand (F32_TERMS): hip_gemm's bits on the f32 activations wherever that
+    runs this kernel."""
+    raw, _ = int_matrix(qtype, rows, cols, seed=rows + cols, scale_pow=-1)
+    w = dev.from_numpy(raw)
+    for batch in batches:
+        x = np.random.default_rng(batch).standard_normal((batch, cols)).astype(np.float32)
+        xd, planes = dev.from_numpy(x), dev.alloc(3 * batch * cols * 2)
+        dev.splitTerms(xd, planes, batch * cols)
+        got = []
+        for x_dtype, xs in ((B.F32, xd), (B.F32_TERMS, planes)):
+            y = dev.alloc(batch * rows * 4)
+            y.fill(0xAB)
+            dev.gemmEx(qtype, w, None, x_dtype, xs, B.F32, y, batch, rows, cols)
+            got.append(y.to_numpy((batch, rows), np.uint32))
+        np.testing.assert_array_equal(got[0], got[1], err_msg=f"batch {batch}")

@@ -1192,7 +1192,8 @@ static void launch_q(const GemmArgs& a, int xk, bool ge, hipStream_t s) {
 // bounds the kernel beside the weights' conversion, not the loads' latency: two groups of weights or
 // four activation loads ahead are slower nearly everywhere (10240 x 2560 Q4_0, weights not in cache, 8 tokens
 // 13.5 -> 14.3 / 15.1 us; 2560 x 10240 Q6_K, 45 tokens 45 -> 53 / 46).
-template <int QT, int P, int RT>
+// XK: f32 activations, or the same split beforehand (X_TERMS), which gives the same bits.
+template <int QT, int XK, int P, int RT>
 __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
     constexpr bool SCALED = w_scaled<QT>(), HALVES = QT == HIP_BRIDGE_Q6_K, MIN = QT == HIP_BRIDGE_Q4_K;
     constexpr int TOK = 32 / P, VR = 16 / P;  // tokens; accumulator registers of an MFMA's own rows
@@ -1211,8 +1212,10 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
     // (P = 1) or the only two, the MFMA (and block) given by the lane's row group c / TOK
     constexpr int XS = P == 1 ? 2 : 1, XB = P == 4 ? 2 : 1;  // MFMAs held apart; blocks per load
     const int sub = c / TOK;
-    const float* const xrow = (const float*)a.x + (int64_t)min(t_base + c % TOK, a.batch - 1) * a.cols +
-                              (P == 1 ? 0 : wk<QT>(sub & 1, h)) + 32 * (sub >> 1);
+    const int64_t xat = (int64_t)min(t_base + c % TOK, a.batch - 1) * a.cols + (P == 1 ? 0 : wk<QT>(sub & 1, h)) + 32 * (sub >> 1);
+    constexpr int XL = XK == X_TERMS ? 3 : 2;  // 128-bit loads of an MFMA's columns: planes, or halves
+    const unsigned char* const xrow = (const unsigned char*)a.x + xat * (XK == X_TERMS ? 2 : 4);
+    const int64_t plane_bytes = (int64_t)a.batch * a.cols * 2;
     WSrc ws[RT];
 #pragma unroll
     for (int j = 0; j < RT; ++j) ws[j].row = a.w + (int64_t)min(r_base + 32 * j + c, a.rows - 1) * a.row_bytes;
@@ -1220,13 +1223,15 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
     constexpr int G = WQ::G, RING = G == 1 ? 4 : 1;
     WQ cur[RT], nxt[RING][RT];
     constexpr int UX = 2;  // activation loads ahead
-    f32x4 xr[UX][XS][2];
-    auto load_x = [&](int kb, f32x4 (&r)[XS][2]) {
-        const float* const p = xrow + 32 * min(kb, lastb + 1 - XB);
+    u32x4 xr[UX][XS][XL];
+    auto load_x = [&](int kb, u32x4 (&r)[XS][XL]) {
+        const int at = 32 * min(kb, lastb + 1 - XB);
 #pragma unroll
         for (int s = 0; s < XS; ++s) {
-            r[s][0] = ldf4(p + (P == 1 ? wk<QT>(s, h) : 0));
-            r[s][1] = ldf4(p + (P == 1 ? wk<QT>(s, h) : 0) + 4);
+            const int col = at + (P == 1 ? wk<QT>(s, h) : 0);
+#pragma unroll
+            for (int q = 0; q < XL; ++q)
+                r[s][q] = XK == X_TERMS ? ld16(xrow + 2 * (int64_t)col + q * plane_bytes) : ld16(xrow + 4 * (int64_t)col + 16 * q);
         }
     };
     f32x16 acc[RT];
@@ -1265,14 +1270,18 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
                 cur[j].template ops<1>(un, wb[j][1]);
             }
             if (u % XB == 0) {
-                f32x4(&xv)[XS][2] = xr[u / XB % UX];
+                u32x4(&xv)[XS][XL] = xr[u / XB % UX];
 #pragma unroll
                 for (int s = 0; s < XS; ++s) {
                     uint32_t v[4][3];
+                    if constexpr (XK == X_F32) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) split3(xv[s][i / 2][2 * (i & 1)], xv[s][i / 2][2 * (i & 1) + 1], v[i]);
+                        for (int i = 0; i < 4; ++i)
+                            split3(__uint_as_float(xv[s][i / 2][2 * (i & 1)]), __uint_as_float(xv[s][i / 2][2 * (i & 1) + 1]), v[i]);
+                    }
 #pragma unroll
-                    for (int q = 0; q < 3; ++q) xa[s][q] = __builtin_bit_cast(bf16x8, u32x4{v[0][q], v[1][q], v[2][q], v[3][q]});
+                    for (int q = 0; q < 3; ++q)
+                        xa[s][q] = __builtin_bit_cast(bf16x8, XK == X_F32 ? u32x4{v[0][q], v[1][q], v[2][q], v[3][q]} : xv[s][q % XL]);
                 }
                 load_x(kb + UX * XB, xv);
                 if constexpr (MIN) {
@@ -1344,7 +1353,7 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
         const int tok = t_base + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
         const int row = r_base + 32 * tile + (l & 31);
         if (tok >= a.batch || row >= a.rows) continue;
-        if (!(fabsf(v) < INFINITY))
+        if (XK == X_F32 && !(fabsf(v) < INFINITY))
             v = dot_columns<QT>(a.w + (int64_t)row * a.row_bytes, (const float*)a.x + (int64_t)tok * a.cols, 4 * kKB * z0,
                                 4 * kKB * z1);
         float* const y = (float*)a.y + (int64_t)tok * a.rows + row;
@@ -1360,7 +1369,7 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
 // tile and no halves 20.3; 48 tokens 45.7, two tiles 35.5; at 128 tokens two tiles fill the chip
 // without halves, 57.3 against 66.6. 2048 x 2560, 16 tokens: 4 / 8 waves 8.7 / 9.6, halves 8.9;
 // 48 tokens 15.0, halves 12.3.
-template <int QT>
+template <int QT, int XK>
 static void launch_skinny_t(const GemmArgs& a, hipStream_t s) {
     const int ng = a.cols / (4 * kKB);
     const int p = a.batch > 16 ? 1 : a.batch > 8 ? 2 : 4;
@@ -1375,8 +1384,8 @@ static void launch_skinny_t(const GemmArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)cdiv(a.rows, 32 * rt), (unsigned)ttiles, kz);
     auto go = [&](auto p_c) {
         constexpr int PC = decltype(p_c)::value;
-        if (rt == 1) k_gemm_skinny<QT, PC, 1><<<grid, ks * kWave, 0, s>>>(a);
-        else k_gemm_skinny<QT, PC, 2><<<grid, ks * kWave, 0, s>>>(a);
+        if (rt == 1) k_gemm_skinny<QT, XK, PC, 1><<<grid, ks * kWave, 0, s>>>(a);
+        else k_gemm_skinny<QT, XK, PC, 2><<<grid, ks * kWave, 0, s>>>(a);
     };
     if (p == 1) go(std::integral_constant<int, 1>{});
     else if (p == 2) go(std::integral_constant<int, 2>{});
@@ -1406,21 +1415,26 @@ static bool skinny_range(int qtype, int rows, int cols, int batch) {
     return rows >= 1536 && batch >= 9 && batch <= 127;
 }
 
-// Small-batch product, f32 x and y; false: not a shape, type or batch of this kernel (nothing
-// launched).
-bool launch_gemm_skinny(int qtype, const void* w, int64_t row_bytes, const float* x, float* y, int rows, int cols,
-                        int batch, hipStream_t s) {
+// Small-batch product, f32 x (or its F32_TERMS planes) and f32 y; false: not a shape, type or batch
+// of this kernel (nothing launched).
+bool launch_gemm_skinny(int qtype, const void* w, int64_t row_bytes, int x_dtype, const void* x, float* y, int rows,
+                        int cols, int batch, hipStream_t s) {
     const bool kq = qtype == HIP_BRIDGE_Q4_K || qtype == HIP_BRIDGE_Q6_K;
     const uintptr_t wa = reinterpret_cast<uintptr_t>(w);
     if (!skinny_range(qtype, rows, cols, batch) || !w || !x || !y) return false;
     if (!aligned16(x) || cols % (kq ? 256 : 4 * kKB) != 0 || wa % (qtype == HIP_BRIDGE_BF16 ? 16 : 2) != 0) return false;
     const GemmArgs a{(const unsigned char*)w, nullptr, x, y, row_bytes, rows, cols, batch, 0};
+    const bool terms = x_dtype == HIP_BRIDGE_F32_TERMS;
+    auto go = [&](auto q_c) {
+        constexpr int QT = decltype(q_c)::value;
+        terms ? launch_skinny_t<QT, X_TERMS>(a, s) : launch_skinny_t<QT, X_F32>(a, s);
+    };
     switch (qtype) {
-        case HIP_BRIDGE_Q4_0: launch_skinny_t<HIP_BRIDGE_Q4_0>(a, s); break;
-        case HIP_BRIDGE_Q8_0: launch_skinny_t<HIP_BRIDGE_Q8_0>(a, s); break;
-        case HIP_BRIDGE_BF16: launch_skinny_t<HIP_BRIDGE_BF16>(a, s); break;
-        case HIP_BRIDGE_Q4_K: launch_skinny_t<HIP_BRIDGE_Q4_K>(a, s); break;
-        default: launch_skinny_t<HIP_BRIDGE_Q6_K>(a, s); break;
+        case HIP_BRIDGE_Q4_0: go(std::integral_constant<int, HIP_BRIDGE_Q4_0>{}); break;
+        case HIP_BRIDGE_Q8_0: go(std::integral_constant<int, HIP_BRIDGE_Q8_0>{}); break;
+        case HIP_BRIDGE_BF16: go(std::integral_constant<int, HIP_BRIDGE_BF16>{}); break;
+        case HIP_BRIDGE_Q4_K: go(std::integral_constant<int, HIP_BRIDGE_Q4_K>{}); break;
+        default: go(std::integral_constant<int, HIP_BRIDGE_Q6_K>{}); break;
     }
     check_launch();
     return true;

@@ -2208,7 +2208,8 @@ void hip_gemm(int qtype, const void* weights, const float* x, float* y, int batc
     if (batch_size <= 0 || rows <= 0 || cols <= 0) return;
     if (batch_size > 1) {
         const int64_t rb = gemv_row_bytes(qtype, cols);
-        if (rb > 0 && launch_gemm_skinny(qtype, weights, rb, x, y, rows, cols, batch_size, stream_of(stream))) return;
+        if (rb > 0 && launch_gemm_skinny(qtype, weights, rb, HIP_BRIDGE_F32, x, y, rows, cols, batch_size, stream_of(stream)))
+            return;
     }
     if (batch_size >= gemm_mfma_min_batch(qtype, rows, cols) && weights && x) {
         const int64_t rb = gemv_row_bytes(qtype, cols);
@@ -2239,6 +2240,10 @@ void hip_gemm_ex(int qtype, const void* weights, const void* up_weights, int x_d
         return;
     }
     const int64_t rb = gemv_row_bytes(qtype, cols);
+    // pre-split f32: the kernel that hip_gemm takes for these sizes, so that the products are the same
+    if (rb > 0 && !up_weights && x_dtype == HIP_BRIDGE_F32_TERMS && y_dtype == HIP_BRIDGE_F32 &&
+        launch_gemm_skinny(qtype, weights, rb, x_dtype, x, (float*)y, rows, cols, batch_size, stream_of(stream)))
+        return;
     const int rc = rb > 0 ? launch_gemm_mfma_ex(qtype, weights, up_weights, rb, x_dtype, x, y_dtype, y, rows, cols,
                                                 batch_size, stream_of(stream))
                           : HIP_BRIDGE_EUNSUPPORTED;
