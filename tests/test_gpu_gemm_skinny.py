@@ -6,7 +6,7 @@ second call gives the same bits (the halves are two addends)."""
 import numpy as np
 import pytest
 
-from test_oracle_gemv_cpu import int_matrix
+from test_oracle_gemv_cpu import int_matrix, random_matrix
 from ziglm_amd import bridge as B
 
 pytestmark = pytest.mark.gpu
@@ -121,3 +121,27 @@ def test_split_activations_give_the_same_bits(dev, qtype, rows, cols, batches):
             dev.gemmEx(qtype, w, None, x_dtype, xs, B.F32, y, batch, rows, cols)
             got.append(y.to_numpy((batch, rows), np.uint32))
         np.testing.assert_array_equal(got[0], got[1], err_msg=f"batch {batch}")
+
+
+# the routes of few tokens with the longest sums: wide products on the GEMM (FINE tiles, in one and in two
+# teams), deep ones on k_gemm_skinny
+@pytest.mark.parametrize("qtype,rows,cols,batch", [
+    (B.BF16, 8192, 2560, 33), (B.BF16, 8192, 10496, 17), (B.Q6_K, 8192, 2560, 33), (B.Q4_K, 8192, 10496, 48),
+    (B.Q4_0, 8192, 10496, 80), (B.Q8_0, 8192, 10496, 80), (B.BF16, 192, 21504, 17), (B.Q4_K, 192, 21504, 17),
+    (B.Q4_K, 192, 21504, 64), (B.Q6_K, 192, 21504, 33), (B.Q4_0, 192, 21504, 48)])
+def test_error_does_not_grow_with_depth(dev, qtype, rows, cols, batch):
+    """A result is a total of short sums: its error (2-norms over all results) is that of a few f32
+    roundings (2^-24, of which a random one costs 0.58 of the size rounded) at the result's size,
+    whatever the depth: those of a block's products, about 1, of a chain of 8 or 16 block sums, about
+    1.3, and of the result; 2.5 in all. One chain over 10496 columns is 3 (block sums) to 14 (single
+    products, BF16) of them off."""
+    some = 64  # different rows, repeated
+    raw, wd = random_matrix(qtype, some, cols, seed=cols + batch)
+    w = dev.from_numpy(np.tile(np.ascontiguousarray(raw).reshape(some, -1), (rows // some, 1)))
+    x = np.random.default_rng(batch).standard_normal((batch, cols)).astype(np.float32)
+    exact = x.astype(np.float64) @ wd.T
+    y = dev.alloc(batch * rows * 4)
+    dev.gemm(qtype, w, dev.from_numpy(x), y, batch, rows, cols)
+    got = y.to_numpy((batch, rows // some, some), np.float32).astype(np.float64)
+    err = np.linalg.norm(got - exact[:, None]) / (np.linalg.norm(exact) * (rows // some) ** 0.5)
+    assert err <= 2.5 * 2.0 ** -24, err * 2 ** 24

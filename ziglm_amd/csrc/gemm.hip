@@ -131,18 +131,12 @@ __device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
 __device__ __forceinline__ uint32_t pack_exact(float a, float b) {
     return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
-// The signed (unsigned) bytes of two words as 8 bf16 values, exact.
+// The signed bytes of two words as 8 bf16 values, exact.
 __device__ __forceinline__ bf16x8 bytes_s(uint32_t v, uint32_t w) {
     return __builtin_bit_cast(bf16x8, u32x4{pack_exact((float)(int8_t)v, (float)(int8_t)(v >> 8)),
                                             pack_exact((float)(int8_t)(v >> 16), (float)(int8_t)(v >> 24)),
                                             pack_exact((float)(int8_t)w, (float)(int8_t)(w >> 8)),
                                             pack_exact((float)(int8_t)(w >> 16), (float)(int8_t)(w >> 24))});
-}
-__device__ __forceinline__ bf16x8 bytes_u(uint32_t v, uint32_t w) {
-    return __builtin_bit_cast(bf16x8, u32x4{pack_exact((float)(v & 0xffu), (float)((v >> 8) & 0xffu)),
-                                            pack_exact((float)((v >> 16) & 0xffu), (float)(v >> 24)),
-                                            pack_exact((float)(w & 0xffu), (float)((w >> 8) & 0xffu)),
-                                            pack_exact((float)((w >> 16) & 0xffu), (float)(w >> 24))});
 }
 // a = {a of lanes 0-31, b of lanes 0-31}, b = {a of lanes 32-63, b of lanes 32-63}
 __device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
@@ -282,8 +276,9 @@ struct WGrp<HIP_BRIDGE_Q4_K> {
     __device__ __forceinline__ void open() {}
     template <int S>
     __device__ __forceinline__ void ops(int u, bf16x8 (&o)[1]) const {
-        const int sh = (u & 1) * 4;
-        o[0] = bytes_u((q[u >> 1][2 * S] >> sh) & 0x0f0f0f0fu, (q[u >> 1][2 * S + 1] >> sh) & 0x0f0f0f0fu);
+        const int sh = u & 1 ? 0 : 4;
+        const uint32_t x = (q[u >> 1][2 * S] << sh) & 0xf0f0f0f0u, y = (q[u >> 1][2 * S + 1] << sh) & 0xf0f0f0f0u;
+        o[0] = bytes_s(x ^ 0x80808080u, y ^ 0x80808080u);
     }
     __device__ __forceinline__ void scale(int u, int kb, float (&dv)[2], float& mn) const {
         // 6-bit scale and min of sub-block j (quant.zig:285-290): j < 4: scales[j] & 63 and
@@ -294,8 +289,9 @@ struct WGrp<HIP_BRIDGE_Q4_K> {
         const uint32_t hi = 0u - (((uint32_t)kb >> 2) & 1u);  // j >= 4: all ones (masks: no branch)
         const uint32_t sc = (s0 & 63u & ~hi) | (((s2 & 15u) | ((s0 >> 6) << 4)) & hi);
         const uint32_t m = (s1 & 63u & ~hi) | (((s2 >> 4) | ((s1 >> 6) << 4)) & hi);
-        dv[0] = f16_bits_to_f32(hd.x & 0xffffu) * (float)sc;
-        mn = f16_bits_to_f32(hd.x >> 16) * (float)m;
+        const float A = f16_bits_to_f32(hd.x & 0xffffu) * (float)sc;
+        dv[0] = A * 0.0625f;
+        mn = fmaf(-8.0f, A, f16_bits_to_f32(hd.x >> 16) * (float)m);
     }
 };
 template <>
@@ -395,7 +391,9 @@ __device__ float dot_columns(const unsigned char* row, const float* x, int c0, i
 }
 
 // The (x term, w term) products accumulated, largest first: down to relative size 2^-16
-// (x in XT terms: 3 for f32 activations, 1 for bf16 ones, which are exact).
+// (x in XT terms: 3 for f32 activations, 1 for bf16 ones, which are exact). Smallest first, the
+// large products lose low bits of the small sum they are added to, always in one direction, so
+// that the error grows with the depth: 2560 x 10240 Q4_0, 8 tokens, 1.0e-7 -> 2.3e-7 off.
 template <int XT, int NW>
 struct TermPairs;
 template <>
@@ -426,21 +424,32 @@ struct TermPairs<1, NW> {
 // pairs (out = gelu(g) * u).
 enum XKind { X_F32 = 0, X_BF16 = 1, X_TERMS = 2 };
 
+constexpr int kFine = 8;  // K steps between additions to a compensated total (a power of two of rounds)
 // Activation blocks a thread holds ahead: more for the smaller tiles, whose steps are shorter.
 template <int WT>
 constexpr int x_ahead() {
     return WT >= 4 ? 1 : WT >= 2 ? 2 : 4;
 }
 
+// total += part, with what the rounding lost carried on in `lost` (Kahan's sum)
+__device__ __forceinline__ void add_kahan(float& total, float& lost, float part) {
+    const float y = part - lost, t = total + y;
+    lost = (t - total) - y;
+    total = t;
+}
+
+// FINE (tiles of 32 tokens): the accumulators hold kFine steps and then join a compensated total, so
+// that a deep product's error does not grow with its depth.
 // TEAMS = 2: a second set of WAVES waves takes the other half of the workgroup's K steps, with LDS
 // buffers of its own, and its sums join the first's through the LDS at the end.
-template <int QT, int XK, int WT, int RT, int WAVES, bool GE, int TEAMS>
+template <int QT, int XK, int WT, int RT, int WAVES, bool GE, int TEAMS, bool FINE>
 __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a) {
     constexpr int NT = 64 * WAVES;             // threads of a team
     constexpr int XT = XK == X_BF16 ? 1 : 3;  // activation terms
     constexpr int NW = w_terms<QT>();
     constexpr bool SCALED = w_scaled<QT>();
     constexpr bool HALVES = QT == HIP_BRIDGE_Q6_K;  // a scale per MFMA rather than per block
+    constexpr bool SUMS = SCALED || FINE;           // a step's products form a sum of their own
     constexpr int BT = 32 * WT;                // tokens per workgroup
     constexpr int TR = GE ? 16 : 32;           // output rows per tile
     constexpr int OR = TR * WAVES * RT;        // and per workgroup
@@ -582,7 +591,17 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
         } else {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                if (r >= r0 && r < r1) acc[tile][j][r] = fmaf(d, pt[r], acc[tile][j][r]);
+                if (r >= r0 && r < r1) acc[tile][j][r] = SCALED ? fmaf(d, pt[r], acc[tile][j][r]) : acc[tile][j][r] + pt[r];
+        }
+    };
+
+    f32x16 total = f32x16{}, lost = f32x16{};
+    auto flush = [&]() {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float t = total[r], l = lost[r];
+            add_kahan(t, l, acc[0][0][r]);
+            total[r] = t, lost[r] = l, acc[0][0][r] = 0.0f;
         }
     };
 
@@ -624,7 +643,7 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
             }
         };
         read_tile(0);
-        if constexpr (SCALED) scale_unit(UNITS - 1, part[(UNITS - 1) & 1], pn, kb - 1, 0, 16);
+        if constexpr (SUMS) scale_unit(UNITS - 1, part[(UNITS - 1) & 1], pn, kb - 1, 0, 16);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < WT; ++i) {
@@ -639,12 +658,12 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
                         const int unit = (i * RT + j) * UPT + (HALVES ? s : 0);  // and its place in its unit
                         const int m = HALVES ? p : s * NP + p;
                         const bf16x8 A = xa[i & 1][s][TP::xt[p]], Bv = wb[pc][j][s][TP::wt[p]];
-                        if constexpr (SCALED)
+                        if constexpr (SUMS)
                             part[unit & 1] =
                                 __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, m == 0 ? f32x16{} : part[unit & 1], 0, 0, 0);
                         else
                             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A, Bv, acc[i][j], 0, 0, 0);
-                        if (SCALED && unit > 0) {
+                        if (SUMS && unit > 0) {
                             constexpr int M1 = NMU > 1 ? NMU - 1 : 1;
                             const int mm = NMU > 1 ? m - 1 : 0;
                             if (mm >= 0)
@@ -704,10 +723,15 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
             if (k0 + u < kbe) step(u, k0 + u);  // uniform
             else if (TEAMS > 1 && k0 + u < kbb + steps) __syncthreads();  // the other team's step
         }
+        if (FINE && ((k0 + U) & (kFine - 1)) == 0) flush();
     }
-    if constexpr (SCALED) {  // the last unit's scale products
+    if constexpr (SUMS) {  // the last unit's scale products
         if ((kbe - kbb) & 1) scale_unit(UNITS - 1, part[(UNITS - 1) & 1], 0, kbe - 1, 0, 16);
         else scale_unit(UNITS - 1, part[(UNITS - 1) & 1], 1, kbe - 1, 0, 16);
+    }
+    if constexpr (FINE) {
+        flush();
+        acc[0][0] = total;
     }
 
     if constexpr (TEAMS > 1) {
@@ -764,11 +788,11 @@ static unsigned split_k(const GemmArgs& a, bool ge, bool want, hipStream_t s) {
     return 2;
 }
 
-template <int QT, int XK, bool GE, int WT, int RT, int TEAMS = 1>
+template <int QT, int XK, bool GE, int WT, int RT, int TEAMS = 1, bool FINE = false>
 static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
     constexpr int W = 4;
     const dim3 grid((unsigned)(cdiv(a.rows, (GE ? 16 : 32) * W * RT) * cdiv(a.batch, 32 * WT)), ky);
-    k_gemm_mfma<QT, XK, WT, RT, W, GE, TEAMS><<<grid, 64 * W * TEAMS, 0, s>>>(a);
+    k_gemm_mfma<QT, XK, WT, RT, W, GE, TEAMS, FINE><<<grid, 64 * W * TEAMS, 0, s>>>(a);
 }
 // Workgroup tile (tokens x rows; GE: half the output rows), for 256 CUs that hold two workgroups
 // each. Large tiles convert an operand for more MFMAs, small ones fill the chip:
@@ -789,22 +813,40 @@ static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
 // ones only), BF16 25.5 / 28.2 (none); from 140 tiles on they lose (2048 x 2560 at 333 tokens 26.9 /
 // 28.5; Q4_K 2560 x 10240 119 / 146). Pre-split planes take the same shares, so that they give the same
 // sums (2560 x 10240 at 150 tokens Q4_0 73 / 62, Q4_K 123 / 95; 1024 x 2560 at 512 Q4_0 24.5 / 25.1).
+// f32 products of few tokens take the compensated totals (FINE) where the kernels for small batches,
+// whose sums are short chains, are closer to the exact product than the plain loop: below the batches
+// from which all of these shapes run it, BF16 and Q6_K always, the others from the depth where those
+// kernels change theirs.
+static bool fine_sums(int qtype, int rows, int cols, int batch) {
+    const bool wide = rows >= kWideRows, q6 = qtype == HIP_BRIDGE_Q6_K;
+    const int below = qtype == HIP_BRIDGE_Q4_K ? (wide ? 128 : 96) : q6 ? (wide ? 64 : 96) : wide ? 96 : 128;
+    return batch < below && (q6 || qtype == HIP_BRIDGE_BF16 || cols > (qtype == HIP_BRIDGE_Q4_K ? 5120 : 10240));
+}
 template <int QT, int XK, bool GE>
 static void launch_qt(const GemmArgs& a, hipStream_t s) {
     constexpr bool BIG = XK != X_BF16 && !GE && (QT == HIP_BRIDGE_Q4_0 || QT == HIP_BRIDGE_BF16);
     auto wgs = [&](int wt, int rt) { return cdiv(a.rows, 128 * rt / (GE ? 2 : 1)) * cdiv(a.batch, 32 * wt); };
-    const bool big = BIG && wgs(2, 2) >= 768;
-    const int wt = XK == X_BF16 && wgs(4, 1) >= 384 ? 4 : big || wgs(2, 1) >= 384 ? 2 : 1;
+    constexpr bool F32 = XK != X_BF16 && !GE;
+    const bool fine = F32 && !a.y_bf16 && fine_sums(QT & 0xff, a.rows, a.cols, a.batch);
+    const bool big = BIG && !fine && wgs(2, 2) >= 768;
+    const int wt = fine ? 1 : XK == X_BF16 && wgs(4, 1) >= 384 ? 4 : big || wgs(2, 1) >= 384 ? 2 : 1;
     const int64_t n = wgs(wt, big ? 2 : 1);
-    constexpr bool SHARES = XK != X_BF16 && !GE && QT != HIP_BRIDGE_BF16 && QT != kQ4_0Odd;
+    constexpr bool SHARES = F32 && QT != HIP_BRIDGE_BF16 && QT != kQ4_0Odd;
     if constexpr (SHARES) {
         const bool pays = QT != HIP_BRIDGE_Q6_K || a.cols >= kSplitMinCols;
         if (wt == 1 && n <= 128 && pays && !a.y_bf16 && a.cols >= 32 * kKB) {
-            launch_tile<QT, XK, GE, 1, 1, 2>(a, split_k(a, GE, true, s), s);
+            const unsigned ky = split_k(a, GE, true, s);
+            fine ? launch_tile<QT, XK, GE, 1, 1, 2, true>(a, ky, s) : launch_tile<QT, XK, GE, 1, 1, 2>(a, ky, s);
             return;
         }
     }
     const unsigned ky = split_k(a, GE, n < 384 || (n < 1024 && a.cols >= kSplitMinCols), s);
+    if constexpr (F32) {
+        if (fine) {
+            launch_tile<QT, XK, GE, 1, 1, 1, true>(a, ky, s);
+            return;
+        }
+    }
     if constexpr (BIG) {
         if (big) {
             launch_tile<QT, XK, GE, 2, 2>(a, ky, s);
@@ -1197,8 +1239,8 @@ template <int QT, int XK, int P, int RT>
 __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
     constexpr bool SCALED = w_scaled<QT>(), HALVES = QT == HIP_BRIDGE_Q6_K, MIN = QT == HIP_BRIDGE_Q4_K;
     constexpr int TOK = 32 / P, VR = 16 / P;  // tokens; accumulator registers of an MFMA's own rows
-    constexpr int MAXH = 4;                   // half of the most waves
-    __shared__ __attribute__((aligned(16))) float s_red[MAXH * RT][VR * kWave];
+    constexpr int MAXW = 8;                   // the most waves
+    __shared__ __attribute__((aligned(16))) float s_red[MAXW * RT * VR * kWave];
     const int lane = threadIdx.x & 63, h = lane >> 5, c = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), ks = (int)blockDim.x / kWave;
     const int r_base = (int)blockIdx.x * 32 * RT, t_base = (int)blockIdx.y * TOK;
@@ -1240,6 +1282,38 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
     bf16x8 ones;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
+    // The row groups' sums over FG groups of blocks join a total in the LDS, so that a deep product's
+    // error does not grow with the length of a wave's share (BF16: a compensated total, shorter sums;
+    // 5376 x 21504 at 24 tokens 1.27e-7 off without, the vector kernel 1.14e-7).
+    constexpr bool KAHAN = QT == HIP_BRIDGE_BF16;
+    constexpr int FG = KAHAN ? 1 : 4, OWN = RT * VR * kWave;
+    __shared__ float s_lost[KAHAN ? MAXW * OWN : 1];
+    float *const total = s_red + wave * OWN + lane, *const lost = s_lost + (KAHAN ? wave * OWN + lane : 0);
+    auto flush = [&](bool first) {
+#pragma unroll
+        for (int j = 0; j < RT; ++j) {
+#pragma unroll
+            for (int r = 0; r < VR; ++r) {
+                float v = acc[j][r];
+#pragma unroll
+                for (int i = 1; i < P; ++i) v += acc[j][i * VR + r];
+                const int at = (j * VR + r) * kWave;
+                float t = v, l = 0.0f;
+                if (!first) {
+                    t = total[at];
+                    if (KAHAN) {
+                        l = lost[at];
+                        add_kahan(t, l, v);
+                    } else {
+                        t += v;
+                    }
+                }
+                total[at] = t;
+                if (KAHAN) lost[at] = l;
+            }
+            acc[j] = f32x16{};
+        }
+    };
 
     if (g0 < g1) {
 #pragma unroll
@@ -1316,39 +1390,20 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
             }
             __builtin_amdgcn_sched_barrier(0);  // (else the loads sink to their uses)
         }
+        if ((g - g0) % FG == FG - 1 || g + 1 == g1) flush(g - g0 < FG);  // uniform
     }
-    // the row groups' sums
-#pragma unroll
-    for (int j = 0; j < RT; ++j)
-#pragma unroll
-        for (int r = 0; r < VR; ++r)
-#pragma unroll
-            for (int i = 1; i < P; ++i) acc[j][r] += acc[j][i * VR + r];
+    if (g0 >= g1) flush(true);
 
-    // The waves' sums: the upper half's through the LDS into the lower half's, then those in wave
-    // order.
+    // The waves' sums, in a tree of two halves: w and w + half, then those in order.
     const int half = (ks + 1) / 2;
-    if (wave >= half) {
-#pragma unroll
-        for (int j = 0; j < RT; ++j)
-#pragma unroll
-            for (int r = 0; r < VR; ++r) s_red[(wave - half) * RT + j][r * kWave + lane] = acc[j][r];
-    }
-    __syncthreads();
-    if (wave < half) {
-#pragma unroll
-        for (int j = 0; j < RT; ++j)
-#pragma unroll
-            for (int r = 0; r < VR; ++r) {
-                float* const p = &s_red[wave * RT + j][r * kWave + lane];
-                *p = wave + half < ks ? acc[j][r] + *p : acc[j][r];
-            }
-    }
     __syncthreads();
     for (int i = threadIdx.x; i < RT * VR * kWave; i += (int)blockDim.x) {
         const int tile = i / (VR * kWave), r = i / kWave % VR, l = i % kWave;
-        float v = s_red[tile][i % (VR * kWave)];
-        for (int w = 1; w < half; ++w) v += s_red[w * RT + tile][i % (VR * kWave)];
+        float v = 0.0f;
+        for (int w = 0; w < half; ++w) {
+            const float lo = s_red[w * (RT * VR * kWave) + i], hi = w + half < ks ? s_red[(w + half) * (RT * VR * kWave) + i] : 0.0f;
+            v = w ? v + (lo + hi) : lo + hi;
+        }
         // register r of lane l: token 8 (r / 4) + 4 (l / 32) + r % 4, row l % 32
         const int tok = t_base + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
         const int row = r_base + 32 * tile + (l & 31);
