@@ -73,7 +73,9 @@ def test_infinite_activation_stays_in_its_token(dev):
 # columns past 5120 (10240) and tokens below: products that the vector kernels can also take
 @pytest.mark.parametrize("qtype,rows,cols,batch", [(B.Q6_K, 8192, 256, 3), (B.Q6_K, 8192, 256, 7), (B.Q6_K, 40, 4352, 6),
                                                    (B.Q8_0, 40, 5376, 9), (B.BF16, 40, 10752, 17), (B.Q4_0, 40, 4352, 5),
-                                                   (B.Q4_K, 40, 4352, 20), (B.Q6_K, 40, 4352, 33)])
+                                                   (B.Q4_K, 40, 4352, 20), (B.Q6_K, 40, 4352, 33),
+                                                   (B.Q8_0, 8192, 10496, 17), (B.BF16, 8192, 10496, 24),
+                                                   (B.Q6_K, 8192, 10496, 33)])
 def test_infinite_activations_give_what_f32_gives(dev, qtype, rows, cols, batch):
     """An infinite activation times a weight is an infinity of the product's sign (NaN for a zero
     weight, or where infinities of both signs meet), as in f32 arithmetic on the values; a value past

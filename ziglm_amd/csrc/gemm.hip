@@ -748,6 +748,12 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
 
     // Epilogue: lane (l, r) of tile (i, j) holds token 8 (r / 4) + 4 (l / 32) + r % 4 and row
     // l % 32.
+    constexpr bool CHECK = FINE && XK == X_F32;  // sums that are not finite are formed again (dot_columns)
+    uint32_t again = 0;
+    if constexpr (CHECK) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) again |= !(fabsf(acc[0][0][r]) < INFINITY) ? 1u << r : 0u;
+    }
     auto out = [&](auto put) {
 #pragma unroll
         for (int j = 0; j < RT; ++j) {
@@ -759,8 +765,17 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
                     float v = acc[i][j][r];
                     if constexpr (GE) v = gelu_fast(v) * __shfl_xor(v, 16);
                     const int tok = b_base + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (tok < a.batch && row < a.rows && !(GE && (lane & 16))) put((int64_t)tok * a.rows + row, v);
+                    if (tok < a.batch && row < a.rows && !(GE && (lane & 16)) && !(CHECK && again >> r & 1))
+                        put((int64_t)tok * a.rows + row, v);
                 }
+        }
+        if constexpr (CHECK) {
+            for (; again; again &= again - 1) {
+                const int r = __builtin_ctz(again), tok = b_base + 8 * (r >> 2) + 4 * h + (r & 3), row = wrow + trow;
+                if (tok < a.batch && row < a.rows)
+                    put((int64_t)tok * a.rows + row,
+                        dot_columns<QT>(ws[0].row, (const float*)a.x + (int64_t)tok * a.cols, kKB * cut(p0), kKB * cut(p0 + TEAMS)));
+            }
         }
     };
     if (a.y_bf16)
