@@ -58,13 +58,61 @@ def test_bf16_and_pair_edges(dev, qtype, cols, rows, batch):
     np.testing.assert_allclose(pair, want, rtol=2.0 ** -8, atol=1e-30)
 
 
-def test_large_tiles(dev):
-    """The 64 x 256 tile (three workgroups per CU) with ragged last tiles in both dimensions."""
-    rows, cols, batch = 8200, 160, 1990
-    raw, x, exact = operands(B.Q4_0, rows, cols, batch, 5)
-    y = dev.alloc(batch * rows * 4)
-    dev.gemmEx(B.Q4_0, dev.from_numpy(raw), None, B.F32, dev.from_numpy(x), B.F32, y, batch, rows, cols)
-    np.testing.assert_array_equal(y.to_numpy((batch, rows), np.float32), exact.astype(np.float32))
+def rows_of(qtype, rows, cols, seed, some=61):
+    """A matrix of `some` different rows repeated, and which of them each row is."""
+    raw, wd = int_matrix(qtype, some, cols, seed=seed, scale_pow=-1)
+    pick = np.arange(rows) % some
+    return np.ascontiguousarray(raw).reshape(some, -1)[pick], wd, pick
+
+
+def product(dev, qtype, w, wu, x, x_dtype, batch, rows, cols):
+    """One hip_gemm_ex product of f32 activations, as they are or split beforehand."""
+    xd, y = dev.from_numpy(x), dev.alloc(batch * rows * 4)
+    y.fill(0xAB)
+    if x_dtype == B.F32_TERMS:
+        planes = dev.alloc(3 * batch * cols * 2)
+        dev.splitTerms(xd, planes, batch * cols)
+        xd = planes
+    dev.gemmEx(qtype, w, wu, x_dtype, xd, B.F32, y, batch, rows, cols)
+    return y.to_numpy((batch, rows), np.float32)
+
+
+# tokens x rows of a workgroup's tile (gemm.hip launch_qt), with ragged last tiles in both dimensions:
+LARGE = [(B.Q4_0, 160, 1990),                       # 64 x 128 (single blocks)
+         (B.Q4_0, 128, 1990), (B.Q4_0, 640, 1990),  # 64 x 256, a group of blocks and more than a round
+         (B.Q4_0, 4096, 1510),                      # 64 x 256 in two K halves (792 tiles)
+         (B.Q8_0, 128, 1990), (B.Q8_0, 640, 1990), (B.Q8_0, 160, 1990),  # 128 x 128, groups and single blocks
+         (B.Q8_0, 640, 300),                        # 64 x 128: single blocks (f32), groups (planes)
+         (B.BF16, 640, 1990), (B.BF16, 4096, 1510)]  # 64 x 256 (f32) and 128 x 128 (planes), 128 x 128
+
+
+@pytest.mark.parametrize("x_dtype", [B.F32, B.F32_TERMS])
+@pytest.mark.parametrize("qtype,cols,batch", LARGE)
+def test_large_tiles(dev, qtype, cols, batch, x_dtype):
+    rows = 8200
+    raw, wd, pick = rows_of(qtype, rows, cols, cols)
+    x = np.random.default_rng(cols).integers(-3, 4, (batch, cols)).astype(np.float32)
+    exact = x.astype(np.float64) @ wd.T
+    assert np.all(np.abs(exact) < 2 ** 24)
+    got = product(dev, qtype, dev.from_numpy(raw), None, x, x_dtype, batch, rows, cols)
+    np.testing.assert_array_equal(got, exact.astype(np.float32)[:, pick])
+
+
+@pytest.mark.parametrize("x_dtype", [B.F32, B.F32_TERMS])
+@pytest.mark.parametrize("qtype,cols", [(B.Q8_0, 640), (B.BF16, 640), (B.BF16, 4096)])
+def test_large_pair_tiles(dev, qtype, cols, x_dtype):
+    """The gate.up pair on the same large tiles against the two exact products' GeGLU."""
+    rows, batch = 4100, 1990
+    raw, wd, pick = rows_of(qtype, 2 * rows, cols, cols)
+    x = np.random.default_rng(cols).integers(-3, 4, (batch, cols)).astype(np.float32) / 64
+    exact = (x.astype(np.float64) @ wd.T).astype(np.float32)[:, pick]
+    w, wu = dev.from_numpy(np.ascontiguousarray(raw[:rows])), dev.from_numpy(np.ascontiguousarray(raw[rows:]))
+    got = product(dev, qtype, w, wu, x, x_dtype, batch, rows, cols)
+    want = dev.alloc(batch * rows * 4)
+    dev.geglu(dev.from_numpy(np.ascontiguousarray(exact[:, :rows])), dev.from_numpy(np.ascontiguousarray(exact[:, rows:])),
+              want, batch * rows)
+    # gelu and its product are the same f32 expression in both, up to a fused rounding (2^-23)
+    np.testing.assert_allclose(got, want.to_numpy((batch, rows), np.float32), rtol=2.0 ** -22, atol=1e-30)
 
 
 @pytest.mark.parametrize("qtype", [B.Q4_0, B.Q8_0, B.BF16, B.Q4_K, B.Q6_K])

@@ -75,8 +75,8 @@ __device__ __forceinline__ int lds_chunk(int row, int c) { return row * kLdsRow 
 // Q6_K: its scale per 16-column half multiplies each K = 16 MFMA half's partial sum, the
 // quants u - 32 one exact term. (sc * (u - 32) as two exact terms with one scale d per step
 // instead: 5 term products, 10240 x 2560 x 2048 with f32 activations 555 against 453 us.)
-// Q4_0 rows whose block count is no multiple of four (see WGrp).
-constexpr int kQ4_0Odd = 0x100 + HIP_BRIDGE_Q4_0;
+// Q4_0 and Q8_0 rows whose block count is no multiple of four (see WGrp).
+constexpr int kQ4_0Odd = 0x100 + HIP_BRIDGE_Q4_0, kQ8_0Odd = 0x100 + HIP_BRIDGE_Q8_0;
 template <int QT>
 constexpr bool is_q4_0() {
     return QT == HIP_BRIDGE_Q4_0 || QT == kQ4_0Odd;
@@ -87,7 +87,7 @@ constexpr int w_terms() {
 }
 template <int QT>
 constexpr bool w_scaled() {
-    return is_q4_0<QT>() || QT == HIP_BRIDGE_Q8_0 || QT == HIP_BRIDGE_Q4_K || QT == HIP_BRIDGE_Q6_K;
+    return is_q4_0<QT>() || QT == HIP_BRIDGE_Q8_0 || QT == kQ8_0Odd || QT == HIP_BRIDGE_Q4_K || QT == HIP_BRIDGE_Q6_K;
 }
 // bf16 (RNE) of two floats and the f32 values of the result.
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b, float& ra, float& rb) {
@@ -245,6 +245,44 @@ struct WGrp<kQ4_0Odd> {
 };
 template <>
 struct WGrp<HIP_BRIDGE_Q8_0> {
+    // Half h loads blocks 2 h and 2 h + 1 (68 bytes: f16 d, 32 codes, twice); open() swaps codes
+    // between the halves so that each has columns [16 h, + 16) of all four.
+    static constexpr int G = 4;
+    u32x4 a[4];
+    uint32_t e;
+    __device__ __forceinline__ void load(const WSrc& s, int kb, int h) {
+        const uint32_t o = 68u * h, so = 34u * (uint32_t)kb;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = s.b128(o + 16u * i, so);
+        e = s.b32(o + 64, so);
+    }
+    __device__ __forceinline__ void open() {
+        auto w = [&](int i) { return i < 16 ? a[i >> 2][i & 3] : e; };
+        // the first block's codes: the halfwords from byte 2 on; the second's start at byte 36
+        uint32_t d0 = __builtin_amdgcn_perm(w(8), w(0), 0x07060100u), d1 = d0;  // both blocks' d
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t x = __builtin_amdgcn_alignbit(w(i + 1), w(i), 16), y = __builtin_amdgcn_alignbit(w(i + 5), w(i + 4), 16);
+            swap_halves(x, y);
+            q[0][i] = x, q[2][i] = y;
+            x = w(9 + i), y = w(13 + i);
+            swap_halves(x, y);
+            q[1][i] = x, q[3][i] = y;
+        }
+        swap_halves(d0, d1);
+        d[0] = d0, d[1] = d1;
+    }
+    uint32_t q[4][4], d[2];
+    template <int S>
+    __device__ __forceinline__ void ops(int u, bf16x8 (&o)[1]) const {
+        o[0] = bytes_s(q[u][2 * S], q[u][2 * S + 1]);
+    }
+    __device__ __forceinline__ void scale(int u, int, float (&dv)[2], float&) const {
+        dv[0] = f16_bits_to_f32(u & 1 ? d[u >> 1] >> 16 : d[u >> 1] & 0xffffu);
+    }
+};
+template <>
+struct WGrp<kQ8_0Odd> {
     static constexpr int G = 1;
     u32x4 q;
     uint32_t d;
@@ -366,7 +404,7 @@ __device__ float dot_columns(const unsigned char* row, const float* x, int c0, i
         float w;
         if constexpr (QT == HIP_BRIDGE_BF16) {
             w = bf16_lo(*(const uint16_t*)(row + 2 * (int64_t)c));
-        } else if constexpr (QT == HIP_BRIDGE_Q8_0) {
+        } else if constexpr (QT == HIP_BRIDGE_Q8_0 || QT == kQ8_0Odd) {
             const unsigned char* b = row + (int64_t)(c / 32) * 34;
             w = (float)(int8_t)b[2 + c % 32] * f16_bits_to_f32(*(const uint16_t*)b);
         } else if constexpr (QT == HIP_BRIDGE_Q4_K) {  // (layouts: WGrp)
@@ -810,13 +848,25 @@ static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
     k_gemm_mfma<QT, XK, WT, RT, W, GE, TEAMS, FINE><<<grid, 64 * W * TEAMS, 0, s>>>(a);
 }
 // Workgroup tile (tokens x rows; GE: half the output rows), for 256 CUs that hold two workgroups
-// each. Large tiles convert an operand for more MFMAs, small ones fill the chip:
-//   bf16 activations: 128 x 128 from 1.5 workgroups per CU (10240 x 2560 x 2048 Q4_0: 140 us,
-//     64 x 128 151, 32 x 128 212), else 64 x 128 likewise, else 32 x 128.
-//   f32 (three-term) activations: 64 x 256 from three per CU for the types whose conversion
-//     leaves it registers (it reads the LDS half as often per MFMA; the same product: 284 us,
-//     128 x 128 336, 64 x 128 322), else 64 x 128 from 1.5 per CU, else 32 x 128 (512 tokens of
-//     2048 x 2560: 39 us, 64 x 128 49).
+// each. Large tiles convert an operand for more MFMAs, small ones fill the chip. us at 10240 x 2560
+// unless said:
+//   bf16 activations: 128 x 128 from 1.5 workgroups per CU (2048 tokens Q4_0: 140, 64 x 128 151,
+//     32 x 128 212), else 64 x 128 likewise, else 32 x 128.
+//   f32 (three-term) activations: 64 x 256 from three per CU for Q4_0 (it reads the LDS half as often
+//     per MFMA; 2048 tokens 284, 128 x 128 336, 64 x 128 322), from 400 tiles for BF16 rows that are
+//     not deep (700 tokens 123, 128 x 128 132, 64 x 128 147; gate.up 1024: 344, 361, 384; at 320 tiles, 512
+//     tokens, 111 against 102). 128 x 128 from 448 tiles for Q8_0 (2048 tokens 367, 64 x 128 400;
+//     21504 x 5376 gate.up 333: 590, 695; 320 tiles: 122, 116) and deep BF16 (21504 x 5376 at 333 tokens
+//     274, 64 x 256 283, 64 x 128 302), unless a quarter more of it is padding. The K-quants' conversion
+//     leaves no registers for either. Else 64 x 128 from 1.5 per CU, else 32 x 128 (512 tokens of 2048 x
+//     2560: 39 us, 64 x 128 49); deep BF16 rows 64 x 128 from 160 tiles (2560 x 10240 at 512 tokens 129, 32
+//     x 128 156; at 333, 120 tiles, 114 against 101).
+//   planes: nothing to convert, so large tiles pay earlier. 128 x 128 from 320 tiles for Q8_0 and BF16
+//     (512 tokens BF16 110, 64 x 128 122), 64 x 128 from 80 (BF16 at 200 tokens 63, 32 x 128 95; Q6_K 2560 x
+//     10240 at 333 111, 136), but for Q4_0, whose 32 x 128 tiles are as fast (150 tokens 42, 44).
+//   Q8_0 rows that are not deep take single blocks on 64 x 128 tiles of f32 activations: groups need
+//     more registers and a swap of halves (512 tokens 116 against 124); deep ones are bound by the
+//     loads (2560 x 10240 at 700 tokens 287 with single blocks, 166 with groups).
 // Two K halves per tile (f32 output) where the tiles do not fill the CUs twice (512 tokens of 2048
 // x 2560 39 -> 32 us, 1024 rows 38 -> 26), or four times for deep products (2560 x 10240 x 2048:
 // 365 -> 341 us; at 333 tokens Q6_K 168 -> 117); at 333 tokens of 10240 x 2560 (480 tiles) the
@@ -839,38 +889,54 @@ static bool fine_sums(int qtype, int rows, int cols, int batch) {
 }
 template <int QT, int XK, bool GE>
 static void launch_qt(const GemmArgs& a, hipStream_t s) {
-    constexpr bool BIG = XK != X_BF16 && !GE && (QT == HIP_BRIDGE_Q4_0 || QT == HIP_BRIDGE_BF16);
-    auto wgs = [&](int wt, int rt) { return cdiv(a.rows, 128 * rt / (GE ? 2 : 1)) * cdiv(a.batch, 32 * wt); };
+    constexpr bool Q8 = QT == HIP_BRIDGE_Q8_0 || QT == kQ8_0Odd, B16 = QT == HIP_BRIDGE_BF16, TERMS = XK == X_TERMS;
     constexpr bool F32 = XK != X_BF16 && !GE;
+    auto wgs = [&](int wt, int rt) { return cdiv(a.rows, 128 * rt / (GE ? 2 : 1)) * cdiv(a.batch, 32 * wt); };
+    const bool deep = a.cols >= kSplitMinCols;
     const bool fine = F32 && !a.y_bf16 && fine_sums(QT & 0xff, a.rows, a.cols, a.batch);
-    const bool big = BIG && !fine && wgs(2, 2) >= 768;
-    const int wt = fine ? 1 : XK == X_BF16 && wgs(4, 1) >= 384 ? 4 : big || wgs(2, 1) >= 384 ? 2 : 1;
+    const bool big = F32 && (QT == HIP_BRIDGE_Q4_0 || B16) && !fine && wgs(2, 2) >= 768;
+    // The shares of K, from the tiles that f32 activations had the shares measured on, so that planes
+    // and f32 activations give the same sums whichever tile they take
+    int wt = fine ? 1 : XK == X_BF16 && wgs(4, 1) >= 384 ? 4 : big || wgs(2, 1) >= 384 ? 2 : 1;
     const int64_t n = wgs(wt, big ? 2 : 1);
-    constexpr bool SHARES = F32 && QT != HIP_BRIDGE_BF16 && QT != kQ4_0Odd;
-    if constexpr (SHARES) {
-        const bool pays = QT != HIP_BRIDGE_Q6_K || a.cols >= kSplitMinCols;
+    if constexpr (F32 && !B16 && QT != kQ4_0Odd) {
+        const bool pays = QT != HIP_BRIDGE_Q6_K || deep;
         if (wt == 1 && n <= 128 && pays && !a.y_bf16 && a.cols >= 32 * kKB) {
             const unsigned ky = split_k(a, GE, true, s);
             fine ? launch_tile<QT, XK, GE, 1, 1, 2, true>(a, ky, s) : launch_tile<QT, XK, GE, 1, 1, 2>(a, ky, s);
             return;
         }
     }
-    const unsigned ky = split_k(a, GE, n < 384 || (n < 1024 && a.cols >= kSplitMinCols), s);
+    const unsigned ky = split_k(a, GE, n < 384 || (n < 1024 && deep), s);
     if constexpr (F32) {
         if (fine) {
             launch_tile<QT, XK, GE, 1, 1, 1, true>(a, ky, s);
             return;
         }
     }
-    if constexpr (BIG) {
-        if (big) {
+    int rt = big ? 2 : 1;
+    if constexpr (XK != X_BF16) {
+        if (wt == 1 && (TERMS ? QT != HIP_BRIDGE_Q4_0 && wgs(2, 1) >= 80 : B16 && deep && wgs(2, 1) >= 160)) wt = 2;
+        const bool whole = cdiv(a.batch, 128) * 8 <= cdiv(a.batch, 64) * 5;  // at most a quarter more padding
+        if ((Q8 || B16) && whole && wgs(4, 1) >= (TERMS ? 320 : 448) && (Q8 || TERMS || deep)) wt = 4, rt = 1;
+        else if (B16 && !TERMS && wgs(2, 2) >= 400 && !deep) wt = rt = 2;
+        else if (B16 && TERMS) rt = 1;
+    }
+    if constexpr ((QT == HIP_BRIDGE_Q4_0 && F32) || (B16 && XK == X_F32)) {
+        if (rt == 2) {
             launch_tile<QT, XK, GE, 2, 2>(a, ky, s);
             return;
         }
     }
-    if constexpr (XK == X_BF16) {
+    if constexpr (XK == X_BF16 || Q8 || B16) {
         if (wt == 4) {
             launch_tile<QT, XK, GE, 4, 1>(a, ky, s);
+            return;
+        }
+    }
+    if constexpr (Q8 && XK == X_F32) {
+        if (wt == 2 && !deep) {
+            launch_tile<kQ8_0Odd, XK, GE, 2, 1>(a, ky, s);
             return;
         }
     }
@@ -1537,7 +1603,10 @@ int launch_gemm_mfma_ex(int qtype, const void* w, const void* wu, int64_t row_by
             if (cols % (4 * kKB) == 0) launch_q<HIP_BRIDGE_Q4_0>(a, xk, ge, s);
             else launch_q<kQ4_0Odd>(a, xk, ge, s);
             break;
-        case HIP_BRIDGE_Q8_0: launch_q<HIP_BRIDGE_Q8_0>(a, xk, ge, s); break;
+        case HIP_BRIDGE_Q8_0:
+            if (cols % (4 * kKB) == 0) launch_q<HIP_BRIDGE_Q8_0>(a, xk, ge, s);
+            else launch_q<kQ8_0Odd>(a, xk, ge, s);
+            break;
         case HIP_BRIDGE_F16: launch_q<HIP_BRIDGE_F16>(a, xk, ge, s); break;
         case HIP_BRIDGE_BF16: launch_q<HIP_BRIDGE_BF16>(a, xk, ge, s); break;
         case HIP_BRIDGE_Q4_K: launch_q<HIP_BRIDGE_Q4_K>(a, xk, ge, s); break;
