@@ -83,7 +83,8 @@ LARGE = [(B.Q4_0, 160, 1990),                       # 64 x 128 (single blocks)
          (B.Q4_0, 4096, 1510),                      # 64 x 256 in two K halves (792 tiles)
          (B.Q8_0, 128, 1990), (B.Q8_0, 640, 1990), (B.Q8_0, 160, 1990),  # 128 x 128, groups and single blocks
          (B.Q8_0, 640, 300),                        # 64 x 128: single blocks (f32), groups (planes)
-         (B.BF16, 640, 1990), (B.BF16, 4096, 1510)]  # 64 x 256 (f32) and 128 x 128 (planes), 128 x 128
+         (B.BF16, 640, 1990), (B.BF16, 4096, 1510),  # 64 x 256 (f32) and 128 x 128 (planes), 128 x 128
+         (B.Q4_K, 256, 1990), (B.Q4_K, 768, 900)]   # 64 x 128: min terms on the matrix cores
 
 
 @pytest.mark.parametrize("x_dtype", [B.F32, B.F32_TERMS])
@@ -99,7 +100,7 @@ def test_large_tiles(dev, qtype, cols, batch, x_dtype):
 
 
 @pytest.mark.parametrize("x_dtype", [B.F32, B.F32_TERMS])
-@pytest.mark.parametrize("qtype,cols", [(B.Q8_0, 640), (B.BF16, 640), (B.BF16, 4096)])
+@pytest.mark.parametrize("qtype,cols", [(B.Q8_0, 640), (B.BF16, 640), (B.BF16, 4096), (B.Q4_K, 768)])
 def test_large_pair_tiles(dev, qtype, cols, x_dtype):
     """The gate.up pair on the same large tiles against the two exact products' GeGLU."""
     rows, batch = 4100, 1990

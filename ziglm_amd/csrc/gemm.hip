@@ -492,12 +492,13 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
     constexpr int TR = GE ? 16 : 32;           // output rows per tile
     constexpr int OR = TR * WAVES * RT;        // and per workgroup
     constexpr int XPLANE = BT * kLdsRow;
-    // Q4_K: per-token sums of each K step's activations (f32 or bf16 x: one sum; pre-split
-    // planes: one per plane, added in plane order), four steps' worth.
-    constexpr bool MIN = QT == HIP_BRIDGE_Q4_K;
-    constexpr int XSP = XK == X_TERMS ? 3 : 1;  // sum planes
+    // Q4_K: per-token sums of each K step's activations, four steps' worth.
+    // The min terms are an f32 MFMA per tile and two blocks where a wave has several tiles (as FMAs they
+    // are a fifth of the loop's vector instructions: 10240 x 2560 x 2048 f32 500 -> 463 us); for one tile the
+    // MFMA's latency shows (1024 x 2560 at 1024 tokens 40.6 -> 47.6), so FMAs there.
+    constexpr bool MIN = QT == HIP_BRIDGE_Q4_K, MIN_MFMA = MIN && WT * RT > 1;
     __shared__ __attribute__((aligned(16))) uint16_t s_x_all[TEAMS * 2 * XT * XPLANE];
-    __shared__ __attribute__((aligned(16))) float s_xs_all[TEAMS][MIN ? 4 : 1][MIN ? XSP * BT : 1];
+    __shared__ __attribute__((aligned(16))) float s_xs_all[TEAMS][MIN ? 4 : 1][MIN ? BT : 1];
 
     const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
     const int tid = (int)threadIdx.x - team * NT;
@@ -548,14 +549,24 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
         r[q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
                                              rsx[q / XPP], xoff[q % XPP], (uint32_t)(min(kb, last) * kKB * xes), 0));
     };
+    float csum[XPP];
     auto store_x = [&](int kb, int buf, int q, const u32x4& v) {
         uint16_t* const sx = s_x + buf * (XT * XPLANE) + (q / XPP) * XPLANE;
         const int cc = (tid + NT * (q % XPP)) % XCC, tok = cc / XCPT, k = XE * (cc % XCPT);
         uint16_t* const dst = sx + lds_chunk(tok, k / 8) + k % 8;
         // (MIN) the token's sum over the step's 32 columns of one term: pairs, then the
         // XCPT consecutive lanes holding its chunks (8 of 4 f32 or 4 of 8 bf16: the same
-        // tree over the 32 values); each of them writes it (a branch would cut the step in two)
-        auto put_sum = [&](float cs) { s_xs[MIN ? kb & 3 : 0][(q / XPP) * BT + tok] = group_sum<XCPT>(cs); };
+        // tree over the 32 values); each of them writes it (a branch would cut the step in two).
+        // Planes: a thread holds the same chunk of all three, whose sums it adds first.
+        auto put_sum = [&](float cs) {
+            if constexpr (XK == X_TERMS) {
+                float& c = csum[q % XPP];
+                c = q < XPP ? cs : c + cs;
+                if (q >= 2 * XPP) s_xs[MIN ? kb & 3 : 0][tok] = group_sum<XCPT>(c);
+            } else {
+                s_xs[MIN ? kb & 3 : 0][tok] = group_sum<XCPT>(cs);
+            }
+        };
         if constexpr (XK == X_F32) {
             uint32_t t0[3], t1[3];
             split3(__uint_as_float(v.x), __uint_as_float(v.y), t0);
@@ -604,32 +615,32 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
     // accumulators: a block of one tile, or with HALVES each of its MFMAs.
     constexpr int UPT = HALVES ? 2 : 1, UNITS = WT * RT * UPT, NMU = 2 * NP / UPT;
     f32x16 part[2] = {f32x16{}, f32x16{}};
-    f32x4 xsv[MIN ? 4 : 1];  // the unit's per-token sums (Q4_K)
+    f32x4 xsv[MIN ? 4 : 1];  // (min in FMAs) the unit's per-token sums
     // FMAs [r0, r1) of a finished unit: acc += d * part [- mn * (token sums)]
     auto scale_unit = [&](int unit, const f32x16& pt, int par, int kb, int r0, int r1) {
         const int tile = unit / UPT / RT, j = unit / UPT % RT;
-        const float d = dv[par][j][HALVES ? unit & 1 : 0], m = mn[par][j];
-        if constexpr (MIN) {
+        const float d = dv[par][j][HALVES ? unit & 1 : 0];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                if (r < r0 || r >= r1) continue;
-                if (r % 4 == 0) {
-                    // lane (l, r) of a tile holds token 8 (r / 4) + 4 (l / 32) + r % 4
-                    const int t0 = 32 * tile + 8 * (r >> 2) + 4 * h;
-                    f32x4 v = *reinterpret_cast<const f32x4*>(&s_xs[kb & 3][t0]);
-#pragma unroll
-                    for (int u = 1; u < XSP; ++u) {
-                        const f32x4 w = *reinterpret_cast<const f32x4*>(&s_xs[kb & 3][u * BT + t0]);
-                        v.x += w.x, v.y += w.y, v.z += w.z, v.w += w.w;
-                    }
-                    xsv[r >> 2] = v;
-                }
-                acc[tile][j][r] = fmaf(d, pt[r], fmaf(-m, xsv[r >> 2][r & 3], acc[tile][j][r]));
+        for (int r = 0; r < 16; ++r) {
+            if (r < r0 || r >= r1) continue;
+            float v = acc[tile][j][r];
+            if constexpr (MIN && !MIN_MFMA) {
+                // lane (l, r) of a tile holds token 8 (r / 4) + 4 (l / 32) + r % 4
+                if (r % 4 == 0) xsv[r >> 2] = *reinterpret_cast<const f32x4*>(&s_xs[kb & 3][32 * tile + 8 * (r >> 2) + 4 * h]);
+                v = fmaf(-mn[par][j], xsv[r >> 2][r & 3], v);
             }
-        } else {
+            acc[tile][j][r] = SCALED ? fmaf(d, pt[r], v) : v + pt[r];
+        }
+    };
+    // Q4_K: acc -= (token sums) x (min factors) of blocks kb - 1 and kb, an f32 MFMA over the two (half
+    // h's operands are block kb - 1 + h's; mn[par] is block kb's).
+    auto min_pair = [&](int kb, int par) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                if (r >= r0 && r < r1) acc[tile][j][r] = SCALED ? fmaf(d, pt[r], acc[tile][j][r]) : acc[tile][j][r] + pt[r];
+        for (int i = 0; i < WT; ++i) {
+            const float xs = s_xs[(kb - 1 + h) & 3][32 * i + (lane & 31)];
+#pragma unroll
+            for (int j = 0; j < RT; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xs, h ? -mn[par][j] : -mn[par ^ 1][j], acc[i][j], 0, 0, 0);
         }
     };
 
@@ -682,6 +693,9 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
         };
         read_tile(0);
         if constexpr (SUMS) scale_unit(UNITS - 1, part[(UNITS - 1) & 1], pn, kb - 1, 0, 16);
+        if constexpr (MIN_MFMA) {
+            if (u & 1) min_pair(kb, pc);  // (shares of K-quants are whole super-blocks)
+        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < WT; ++i) {
@@ -747,10 +761,8 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
         cur[j].template ops<0>(0, wb[0][j][0]);
         cur[j].template ops<1>(0, wb[0][j][1]);
     }
-    if constexpr (MIN) {  // the first step's scaling of "the unit before" adds 0 * 0
-        if (tid < BT)
-#pragma unroll
-            for (int u = 0; u < XSP; ++u) s_xs[3][u * BT + tid] = 0.0f;
+    if constexpr (MIN && !MIN_MFMA) {  // the first step's scaling of "the unit before" adds 0 * 0
+        if (tid < BT) s_xs[3][tid] = 0.0f;
     }
     __syncthreads();
     // A branch per step keeps each in a basic block of its own: unrolled into one, instruction
