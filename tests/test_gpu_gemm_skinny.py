@@ -31,19 +31,34 @@ def check(dev, qtype, rows, cols, batch):
 
 
 # two K halves: 4096 columns (32 groups of four blocks), 4352 (34: 17 a half, uneven over the waves)
-@pytest.mark.parametrize("qtype,batches", [(q, (5, 8, 9, 16, 17, 31, 33, 128)) for q in GROUPED] +
-                         [(B.Q8_0, (9, 16, 17, 33, 128)), (B.BF16, (17, 32, 64, 128))])
+@pytest.mark.parametrize("qtype,batches", [(B.Q4_0, (9, 16, 17, 24, 33, 128)), (B.Q4_K, (5, 8, 9, 16, 17, 24, 33, 128)),
+                                           (B.Q6_K, (5, 8, 9, 16, 17, 31, 33, 128)), (B.Q8_0, (9, 16, 17, 33, 128)),
+                                           (B.BF16, (64, 96, 128))])
 @pytest.mark.parametrize("rows,cols", [(1, 4096), (33, 4352), (95, 4096)])
 def test_deep(dev, qtype, batches, rows, cols):
     for batch in batches:
         check(dev, qtype, rows, cols, batch)
 
 
-# many rows: one and two row tiles per wave, a single group of blocks (128 columns; K-quants two)
+# many rows, a group of blocks or two of a wave's share
 @pytest.mark.parametrize("qtype", GROUPED)
 @pytest.mark.parametrize("rows,cols,batches", [(8193, 256, (3, 7, 8, 9, 15, 17, 32)), (5121, 768, (3, 16, 33, 63)),
-                                               (1537, 256, (9, 17, 65, 127))])
+                                               (2561, 256, (10, 17, 65, 127))])
 def test_wide(dev, qtype, rows, cols, batches):
+    for batch in batches:
+        check(dev, qtype, rows, cols, batch)
+
+
+# Two row tiles per wave (RT = 2), by operand packing (P = 4, 2, 1 for up to 8, 16, 32 tokens) and K halves;
+# the launch rule gives: shallow rows RT = 2 where 64-row tiles x token tiles reach 160 and P < 4; deep ones
+# where 32-row tiles x token tiles reach 160, in two halves where 64-row ones do not.
+@pytest.mark.parametrize("qtype,rows,cols,batches",
+                         [(q, 10241, 256, (9, 16, 17, 32)) for q in GROUPED] +            # P = 2, 1, no halves
+                         [(q, 5153, 4096, (5, 8, 9, 16)) for q in GROUPED] +              # P = 4, 2, no halves
+                         [(B.Q8_0, 5153, 4096, (9, 16, 17))] +                            # P = 2, 1, no halves
+                         [(q, 2561, 4096, (33, 64)) for q in (*GROUPED, B.Q8_0)] +        # P = 1, two halves
+                         [(B.BF16, 2561, 4096, (65, 96)), (B.BF16, 5153, 4352, (17, 32))])  # P = 1, halves and not
+def test_two_row_tiles(dev, qtype, rows, cols, batches):
     for batch in batches:
         check(dev, qtype, rows, cols, batch)
 
@@ -56,7 +71,7 @@ def test_single_groups(dev, cols):
 
 def test_infinite_activation_stays_in_its_token(dev):
     """Packed tokens share an operand's rows with their own other columns only."""
-    rows, cols = 40, 4096
+    rows, cols = 2048, 4096
     raw, wd = int_matrix(B.Q4_0, rows, cols, seed=1, scale_pow=-1)
     for batch in (6, 12, 20):
         x = np.random.default_rng(batch).integers(-2, 3, (batch, cols)).astype(np.float32)
@@ -72,7 +87,7 @@ def test_infinite_activation_stays_in_its_token(dev):
 
 # columns past 5120 (10240) and tokens below: products that the vector kernels can also take
 @pytest.mark.parametrize("qtype,rows,cols,batch", [(B.Q6_K, 8192, 256, 3), (B.Q6_K, 8192, 256, 7), (B.Q6_K, 40, 4352, 6),
-                                                   (B.Q8_0, 40, 5376, 9), (B.BF16, 40, 10752, 17), (B.Q4_0, 40, 4352, 5),
+                                                   (B.Q8_0, 40, 5376, 9), (B.BF16, 2560, 10752, 17), (B.Q4_0, 40, 4352, 9),
                                                    (B.Q4_K, 40, 4352, 20), (B.Q6_K, 40, 4352, 33),
                                                    (B.Q8_0, 8192, 10496, 17), (B.BF16, 8192, 10496, 24),
                                                    (B.Q6_K, 8192, 10496, 33)])
@@ -104,7 +119,7 @@ def test_infinite_activations_give_what_f32_gives(dev, qtype, rows, cols, batch)
 
 
 @pytest.mark.parametrize("qtype,rows,cols,batches",
-                         [(q, 40, 4352, (5, 9, 20, 64, 96, 128)) for q in GROUPED] + [(q, 5121, 512, (5, 16, 40)) for q in GROUPED] +
+                         [(q, 40, 4352, (9, 20, 64, 96, 128)) for q in GROUPED] + [(q, 5121, 512, (5, 16, 40)) for q in GROUPED] +
                          [(B.Q8_0, 40, 4352, (9, 20, 64, 96, 128)), (B.BF16, 40, 4352, (64, 96, 128))] +
                          [(q, 2561, 4096, (65, 128)) for q in (*GROUPED, B.Q8_0, B.BF16)])
 def test_split_activations_give_the_same_bits(dev, qtype, rows, cols, batches):
@@ -129,7 +144,7 @@ def test_split_activations_give_the_same_bits(dev, qtype, rows, cols, batches):
 # teams), deep ones on k_gemm_skinny
 @pytest.mark.parametrize("qtype,rows,cols,batch", [
     (B.BF16, 8192, 2560, 33), (B.BF16, 8192, 10496, 17), (B.Q6_K, 8192, 2560, 33), (B.Q4_K, 8192, 10496, 48),
-    (B.Q4_0, 8192, 10496, 80), (B.Q8_0, 8192, 10496, 80), (B.BF16, 192, 21504, 17), (B.Q4_K, 192, 21504, 17),
+    (B.Q4_0, 8192, 10496, 80), (B.Q8_0, 8192, 10496, 80), (B.BF16, 2560, 21504, 17), (B.Q4_K, 192, 21504, 17),
     (B.Q4_K, 192, 21504, 64), (B.Q6_K, 192, 21504, 33), (B.Q4_0, 192, 21504, 48)])
 def test_error_does_not_grow_with_depth(dev, qtype, rows, cols, batch):
     """A result is a total of short sums: its error (2-norms over all results) is that of a few f32

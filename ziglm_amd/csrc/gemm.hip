@@ -1545,22 +1545,38 @@ static void launch_skinny_t(const GemmArgs& a, hipStream_t s) {
 // (gemm_mfma_min_batch). us, this kernel / the best other, at n rows x columns:
 //   Q4_0, Q4_K, Q6_K: at least 8192 rows to 32 tokens (10240 x 2560: Q4_0 2 tokens 11.7 / 18.3, 24
 //     19.4 / 23.5, 40 32.4 / 25.7; Q6_K 2 tokens 16.1 / 13.1, 4 16.3 / 21.4; 262144 x 2560 Q6_K 4
-//     tokens 247 / 471); at least 5120 to 64 tokens (6144 x 1536 Q4_K 64: 16.4 / 21.0, 128 30.5 /
-//     24.5); deep ones from 5 to 128 tokens (2560 x 10240 Q4_0 4 tokens 13.6 / 12.4, 8 15.0 / 21.1,
-//     96 36.2 / 78.9, 128 57.3 / 78.4); the rest from 9 tokens on 1536 rows (2048 x 2560: 2 tokens
-//     7.2 / 7.3, 16 8.7 / 10.0, 80 15.6 / 20.9; 256 x 1536 10 / 6);
-//   Q8_0 and BF16, whose 32-column blocks take a load each: deep products of 9 (17) to 128 tokens
-//     (2560 x 10240: Q8_0 4 tokens 25 / 16, 20 37.6 / 58.5, 80 61 / 93; BF16 16 tokens 26.0 / 23.4, 24
-//     32.8 / 37.3, 48 48.0 / 42.1, 80 48.3 / 70.4, so not between 33 and 63).
+//     tokens 247 / 471; 21504 x 5376 Q4_0 2 tokens 40 / 23, 3 40 / 41); at least 5120 to 64 tokens (6144 x
+//     1536 Q4_K 64: 16.4 / 21.0, 128 30.5 / 24.5); deep ones from 5 to 128 tokens (2560 x 10240 Q4_0 4
+//     tokens 13.6 / 12.4, 8 15.0 / 21.1, 96 36.2 / 78.9; 1536 x 6144 Q4_0 8 tokens 11.2 / 10.3, 9 11.6 /
+//     13.6); the rest from 9 tokens on 1536 rows (2048 x 2560: 2 tokens 7.2 / 7.3, 16 8.7 / 10.0, 80 15.6 /
+//     20.9; 256 x 1536 10 / 6), but
+//       Q4_K of up to 2047 rows 33 to 64 and from 96 (1536 x 2048: 32 11.4 / 9.6, 45 11.5 / 13.5, 80 15.5 /
+//       13.5), to 2559 from 49 (2048 x 2560: 9 11.2 / 8.5, 45 13.0 / 11.5, 63 13.1 / 17.7), above from 10;
+//       Q6_K of up to 2047 rows 9 to 16 and as Q4_K (1536 x 2048: 32 12.0 / 10.4, 45 12.2 / 16.8);
+//       Q4_0 of up to 2048 short rows not where k_gemv_mb's second (third) 16-token tile fills up (1536 x
+//       2048: 24 10.3 / 10.4, 32 11.2 / 10.5, 33 11.3 / 15.4; 2048 x 1536: 45 9.9 / 9.4, 63 9.9 / 14.0);
+//   Q8_0 and BF16: deep products of 9 to 128 tokens (2560 x 10240 Q8_0 9 30 / 43); BF16, whose blocks
+//     take a load each, of 17 to 32 from 2560 rows (1536 x 6144, 24 22.6 / 16.0; 2560 x 10240 32.8 / 37.3; 48
+//     tokens 48.0 / 42.1) and of 64 to 128, to 96 from 5120 rows (5376 x 4096: 96 42 / 53, 128 78 / 43).
+//   All but BF16 leave 25 to 32 tokens of at most 2048 rows of up to 176 blocks to k_gemv_mb, whose two
+//     halves are shortest there (2048 x 5376 at 32 tokens: Q4_0 17.6 / 16.6, Q8_0 18.4 / 16.8, Q4_K 18.0 /
+//     15.5; 24 15.5 / 16.9, 16.3 / 18.3, 16.2 / 15.5).
 static bool skinny_range(int qtype, int rows, int cols, int batch) {
-    const bool groups = qtype == HIP_BRIDGE_Q4_0 || qtype == HIP_BRIDGE_Q4_K || qtype == HIP_BRIDGE_Q6_K;
-    const bool deep = cols >= kSplitMinCols && rows < kWideRows;
-    if (qtype == HIP_BRIDGE_Q8_0) return deep && batch >= 9 && batch <= 128;
-    if (qtype == HIP_BRIDGE_BF16) return deep && ((batch >= 17 && batch <= 32) || (batch >= 64 && batch <= 128));
-    if (!groups) return false;
-    if (deep) return batch >= 5 && batch <= 128;
-    if (rows >= kMidRows) return batch >= (qtype == HIP_BRIDGE_Q6_K ? 3 : 2) && batch <= (rows >= kWideRows ? 32 : 64);
-    return rows >= 1536 && batch >= 9 && batch <= 127;
+    const bool q4 = qtype == HIP_BRIDGE_Q4_0, q4k = qtype == HIP_BRIDGE_Q4_K, q6 = qtype == HIP_BRIDGE_Q6_K;
+    if (rows < kWideRows && cols >= kSplitMinCols) {  // deep
+        if (batch > 128) return false;
+        if (qtype == HIP_BRIDGE_BF16)
+            return (batch >= 17 && batch <= 32 && rows >= 2560) || (batch >= 64 && batch <= (rows >= kMidRows ? 96 : 128));
+        if (rows <= 2048 && cols <= 176 * kKB && batch >= 25 && batch <= 32 && !q6) return false;
+        if (qtype == HIP_BRIDGE_Q8_0) return batch >= 9;
+        return (q4 || q4k || q6) && batch >= (q4 && rows < 2048 ? 9 : 5);
+    }
+    if (!(q4 || q4k || q6)) return false;
+    if (rows >= kMidRows) return batch >= (q6 || (q4 && cols > 5120) ? 3 : 2) && batch <= (rows >= kWideRows ? 32 : 64);
+    if (rows < 1536 || batch < 9 || batch > 127) return false;
+    if (q4) return !(rows <= 2048 && cols <= 2048 && batch >= 25 && batch <= (cols <= 1536 ? 48 : 32));
+    if (rows < 2048) return (q6 && batch <= 16) || (batch >= 33 && batch <= 64) || batch >= 96;
+    return q6 || batch >= (rows < 2560 ? 49 : 10);
 }
 
 // Small-batch product, f32 x (or its F32_TERMS planes) and f32 y; false: not a shape, type or batch

@@ -57,18 +57,17 @@ void launch_zero_f32(float* y, int64_t n, hipStream_t s);
 // The batch from which the matrix-core GEMM (k_gemm_mfma; F16, F32: k_gemm_dense) is faster than
 // the kernels for smaller ones, where k_gemm_skinny does not take the call. Wide products (us,
 // 10240 x 2560, GEMM / k_gemm_skinny / k_gemv_mb): Q4_0 24 tokens 23.5 / 19.4 / 39.3, 40 tokens
-// 25.7 / 32.4 / 40.4; Q4_K 40 31.7 / 39.0 / 32.9; Q6_K 40 34.2 / 43.8 / 72.0; Q8_0 24 24.5 / 26.0 /
-// 39.8; BF16 24 22.0 / 26.3 / 29.3. 6144 x 1536 Q4_K: 45 tokens 18.1 / 15.5 / 21.0, 128 24.5 / 30.5.
-// Narrower ones keep the crossovers of the GEMM against k_gemv_mb and the vector kernels: from 64
-// tokens where deep enough to run in two K halves, else 128 (K-quants 96).
+// 25.7 / 32.4 / 40.4; Q4_K 45 33.0 / 38.7 / 30.9, 63 34.8 / 40.4 / 43.4; Q6_K 40 34.2 / 43.8 / 72.0; Q8_0
+// 24 24.5 / 26.0 / 39.8; BF16 24 22.0 / 26.3 / 29.3. 6144 x 1536 Q4_K: 45 tokens 16.9 / 16.3 / 20.7, 80
+// 23.3 / 29.1 / 21.3, 96 24.5 / 30.1 / 40.8. Narrower ones keep the crossovers of the GEMM against
+// k_gemv_mb and the vector kernels: from 64 tokens where deep, else 128 (K-quants 96).
 inline int gemm_mfma_min_batch(int qtype, int rows, int cols) {
-    const bool deep = cols >= kSplitMinCols;
-    const bool kq = qtype == HIP_BRIDGE_Q4_K || qtype == HIP_BRIDGE_Q6_K;
+    const bool deep = cols >= kSplitMinCols, q4k = qtype == HIP_BRIDGE_Q4_K;
     if (qtype == HIP_BRIDGE_F16 || qtype == HIP_BRIDGE_F32) return rows >= kWideRows ? 96 : deep ? 64 : 128;
     const bool single = qtype == HIP_BRIDGE_Q8_0 || qtype == HIP_BRIDGE_BF16;
-    if (rows >= kWideRows) return single ? 17 : 33;
-    if (rows >= kMidRows && !deep) return single ? 33 : 65;
-    return kq ? 96 : deep ? 64 : 128;
+    if (rows >= kWideRows) return single ? 17 : q4k && cols <= 5120 ? 49 : 33;  // (k_gemv_mb's longest rows)
+    if (rows >= kMidRows && !deep) return single ? 33 : q4k ? 96 : 65;
+    return q4k || qtype == HIP_BRIDGE_Q6_K ? 96 : deep ? 64 : 128;
 }
 bool launch_gemm_mfma(int qtype, const void* w, int64_t row_bytes, const float* x, float* y, int rows, int cols,
                       int batch, hipStream_t s);
