@@ -25,10 +25,10 @@ def data(seed, T, nh, nkv, d, rows):
             synth.normal_f32(seed, "v", (rows, nkv * d), 0, 1))
 
 
-# every shape launches the chunk kernel: 96 workgroups, or 8 heads per kv head from 8 tokens
-@pytest.mark.parametrize("nh,nkv,d,T,pos", [(16, 16, 64, 97, 0), (8, 4, 256, 193, 0), (8, 4, 256, 200, 37),
-                                            (8, 2, 128, 195, 64), (8, 1, 256, 9, 0), (8, 1, 256, 8, 250),
-                                            (8, 1, 64, 31, 15), (32, 16, 128, 65, 100)])
+# every shape launches the chunk kernel: 128 workgroups, or 8 heads per kv head and 16 rows of kv heads
+@pytest.mark.parametrize("nh,nkv,d,T,pos", [(16, 16, 64, 129, 0), (8, 4, 256, 257, 0), (8, 4, 256, 260, 37),
+                                            (8, 2, 128, 257, 30), (8, 1, 256, 17, 0), (8, 1, 256, 16, 250),
+                                            (8, 1, 64, 31, 15), (16, 2, 256, 9, 100), (32, 16, 128, 65, 100)])
 @pytest.mark.parametrize("cap,window", [(0.0, 0), (20.0, 0), (0.0, 33), (0.0, 16)])
 def test_against_f64(dev, nh, nkv, d, T, pos, cap, window):
     max_seq, layer, scale = 320, 1, d ** -0.5

@@ -538,13 +538,15 @@ static void launch_g(const AttnArgs& a, bool qk, hipStream_t s) {
 // with all heads, 70.4 us with one head per workgroup, before the per-sequence split).
 constexpr int64_t kFewGroups = 16;
 constexpr double kKvResidentBytes = 32.0 * (1 << 20);
+static bool few_groups(const AttnArgs& a, int es) {
+    const int len = a.window > 0 ? std::min(a.window, a.max_len) : a.max_len;
+    return (int64_t)a.batch * a.nkv < kFewGroups && (double)a.batch * len * a.nkv * a.D * 2.0 * es <= kKvResidentBytes;
+}
 static void choose_heads(AttnArgs& a, int es) {
     a.gq = a.nh / a.nkv;
-    const int len = a.window > 0 ? std::min(a.window, a.max_len) : a.max_len;
-    const double kv = (double)a.batch * len * a.nkv * a.D * 2.0 * es;
     int gw = a.gq;
     if (ZL_ATTN_GW > 0) gw = std::min(a.gq, ZL_ATTN_GW);
-    else if ((int64_t)a.batch * a.nkv < kFewGroups && kv <= kKvResidentBytes) gw = 1;
+    else if (few_groups(a, es)) gw = 1;
     a.hg = a.gq / gw;
 }
 
@@ -634,7 +636,7 @@ static void launch_attn(int kv_dtype, AttnArgs& a, size_t ws_bytes, hipStream_t 
 // token's rows for itself, 512 tokens over 512-1024 positions of 8 / 4 heads x 256 read 2 GB
 // through the L2 and took 218 us. Here a workgroup takes 16 query rows of one kv head (16 / gq
 // tokens x gq heads), its 8 waves the 16-key blocks of the rows' range in turn, with the f32 MFMA
-// 16x16x4 (exact f32 products and f32 sums, a quarter of the vector units' instruction count per
+// 16x16x4 (exact f32 products and f32 sums, a sixteenth of the vector units' instruction count per
 // product; splitting K and V into bf16 terms instead would cost more vector work per workgroup
 // than the faster MFMA saves, at 16 rows per conversion).
 // Scores are formed transposed, S^T = K Q^T, so that lane (n = lane % 16, g = lane / 16) holds query
@@ -643,7 +645,6 @@ static void launch_attn(int kv_dtype, AttnArgs& a, size_t ws_bytes, hipStream_t 
 // registers by 128-bit loads, four MFMAs to a load (the order of the contraction and of the output
 // columns follows the loads); each quarter of a block's rows is requested one quarter (a
 // thousand cycles at head size 256) ahead. The waves' online softmax states merge through LDS.
-// Limited by the f32 matrix rate (64 multiply-adds per cycle and CU).
 typedef float acc4 __attribute__((ext_vector_type(4)));
 constexpr int kChunkWaves = 8;
 template <int D>
@@ -879,11 +880,13 @@ __global__ __launch_bounds__(kChunkWaves * kWave, 2) void k_attn_chunk(AttnArgs 
 // call (which also reports bad arguments). The decode kernel runs a workgroup per token and kv
 // head, so it loses with the tokens that share their rows, this one while its workgroups leave
 // most CUs idle. Measured (us, decode kernel / this; span: keys seen by the last token): 8 / 4
-// heads x 256: 128 tokens over 128 keys 13.3 / 14.3, 256 over 256 31.6 / 20.4, 100 over 200
-// 18.4 / 18.0, 64 over 364 22.6 / 24.2, 48 over 2548 129 / 112, 512 over 1024 216 / 56; 32 / 16
-// heads x 128: 16 tokens over 116 7.2 / 8.4, 24 over 1024 37 / 27, 64 over 64 11.0 / 7.2, 512
-// over 1024 360 / 84. With 8 heads per kv head two tokens fill the rows: 8 tokens over 108 keys
-// 23 / 13, over 3008 427 / 129 (fewer tokens: 4 over 3004 88 / 129).
+// heads x 256: 128 tokens over 128 keys 12.0 / 14.5, 100 over 200 17.3 / 19.0, 128 over 428 31.4 /
+// 27.0, 48 over 3048 154 / 139, 512 over 1024 216 / 56; 32 / 16 heads x 128: 16 tokens over 116
+// 7.2 / 8.8, 24 over 624 29 / 24, 12 over 3012 69 / 74, 48 within a window of 128 (nine blocks of keys
+// for eight waves) 9.5 / 10.2, 64 over 64 11.0 / 7.2, 512 over 1024 360 / 84; 8 / 8 heads x 64: 64 over
+// 3064 33 / 45, 128 over 728 22 / 18. With 8 heads per kv head two tokens fill the rows: 8 tokens over
+// 108 keys 23 / 13, over 3008 427 / 129 (fewer tokens: 4 over 3004 88 / 129), but not where the
+// decode kernel takes a workgroup per head (8 within a window of 128 7.0 / 16.3, of 512 17.9 / 31.1).
 static bool launch_chunk(AttnArgs& a, hipStream_t s) {
     if (!a.q || !a.kc || !a.vc || !a.out || a.nkv <= 0 || a.nh <= 0 || a.nh % a.nkv != 0 || a.max_len <= 0) return false;
     a.gq = a.nh / a.nkv;
@@ -893,7 +896,9 @@ static bool launch_chunk(AttnArgs& a, hipStream_t s) {
     if (!shapes || !aligned) return false;
     const int64_t wgs = cdiv(a.batch, 16 / a.gq) * a.nkv, end = (int64_t)a.pos_base + a.batch;
     const int64_t span = a.window > 0 ? std::min<int64_t>(a.window, end) : end;
-    const bool faster = a.gq == 8 ? a.batch >= 8 : wgs >= 96 || (wgs >= 48 && span >= 200) || (wgs >= 24 && span >= 2048);
+    const bool faster = a.gq == 8 ? a.batch >= 8 && span >= 16 && !few_groups(a, 4)
+                                  : wgs >= 128 || (wgs >= 96 && (a.window == 0 || span >= 160)) || (wgs >= 48 && span >= 240) ||
+                                        (wgs >= 24 && span >= 2048 && a.D == 256);
     if (!faster || wgs > INT32_MAX || end > INT32_MAX) return false;
     a.inv_cap = a.softcap > 0.0f ? 1.0f / a.softcap : 0.0f;
     const dim3 grid((unsigned)wgs), threads(kChunkWaves * kWave);
