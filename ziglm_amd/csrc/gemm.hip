@@ -891,13 +891,13 @@ static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
 // 28.5; Q4_K 2560 x 10240 119 / 146). Pre-split planes take the same shares, so that they give the same
 // sums (2560 x 10240 at 150 tokens Q4_0 73 / 62, Q4_K 123 / 95; 1024 x 2560 at 512 Q4_0 24.5 / 25.1).
 // f32 products of few tokens take the compensated totals (FINE) where the kernels for small batches,
-// whose sums are short chains, are closer to the exact product than the plain loop: below the batches
-// from which all of these shapes run it, BF16 and Q6_K always, the others from the depth where those
-// kernels change theirs.
+// whose sums are short chains, are closer to the exact product than the plain loop: from the batch at
+// which hip_gemm takes this kernel to that where all of these shapes do, BF16 and Q6_K always, the
+// others from the depth where those kernels change theirs.
 static bool fine_sums(int qtype, int rows, int cols, int batch) {
     const bool wide = rows >= kWideRows, q6 = qtype == HIP_BRIDGE_Q6_K;
     const int below = qtype == HIP_BRIDGE_Q4_K ? (wide ? 128 : 96) : q6 ? (wide ? 64 : 96) : wide ? 96 : 128;
-    return batch < below && (q6 || qtype == HIP_BRIDGE_BF16 || cols > (qtype == HIP_BRIDGE_Q4_K ? 5120 : 10240));
+    return batch < below && batch >= gemm_mfma_min_batch(qtype, rows, cols) && (q6 || qtype == HIP_BRIDGE_BF16 || cols > (qtype == HIP_BRIDGE_Q4_K ? 5120 : 10240));
 }
 template <int QT, int XK, bool GE>
 static void launch_qt(const GemmArgs& a, hipStream_t s) {
@@ -928,7 +928,7 @@ static void launch_qt(const GemmArgs& a, hipStream_t s) {
     }
     int rt = big ? 2 : 1;
     if constexpr (XK != X_BF16) {
-        if (wt == 1 && (TERMS ? QT != HIP_BRIDGE_Q4_0 && wgs(2, 1) >= 80 : B16 && deep && wgs(2, 1) >= 160)) wt = 2;
+        if (wt == 1 && !fine && (TERMS ? QT != HIP_BRIDGE_Q4_0 && a.batch > 32 && wgs(2, 1) >= 80 : B16 && deep && wgs(2, 1) >= 160)) wt = 2;
         const bool whole = cdiv(a.batch, 128) * 8 <= cdiv(a.batch, 64) * 5;  // at most a quarter more padding
         if ((Q8 || B16) && whole && wgs(4, 1) >= (TERMS ? 320 : 448) && (Q8 || TERMS || deep)) wt = 4, rt = 1;
         else if (B16 && !TERMS && wgs(2, 2) >= 400 && !deep) wt = rt = 2;
@@ -1557,16 +1557,18 @@ static void launch_skinny_t(const GemmArgs& a, hipStream_t s) {
 //       2048: 24 10.3 / 10.4, 32 11.2 / 10.5, 33 11.3 / 15.4; 2048 x 1536: 45 9.9 / 9.4, 63 9.9 / 14.0);
 //   Q8_0 and BF16: deep products of 9 to 128 tokens (2560 x 10240 Q8_0 9 30 / 43); BF16, whose blocks
 //     take a load each, of 17 to 32 from 2560 rows (1536 x 6144, 24 22.6 / 16.0; 2560 x 10240 32.8 / 37.3; 48
-//     tokens 48.0 / 42.1) and of 64 to 128, to 96 from 5120 rows (5376 x 4096: 96 42 / 53, 128 78 / 43).
+//     tokens 48.0 / 42.1) and of 64 to 128.
+//   From 2560 rows all but the K-quants to 96 tokens (2560 x 10240 at 112: Q4_0 58 / 59, Q8_0 68 / 69, BF16
+//     85 / 94, Q4_K 61 / 73, Q6_K 74 / 85, and from planes, six loads a block where f32 takes four, Q4_0 82 /
+//     62, BF16 128 / 88; 5376 x 4096 at 128: Q4_0 53 / 42, BF16 78 / 43).
 //   All but BF16 leave 25 to 32 tokens of at most 2048 rows of up to 176 blocks to k_gemv_mb, whose two
 //     halves are shortest there (2048 x 5376 at 32 tokens: Q4_0 17.6 / 16.6, Q8_0 18.4 / 16.8, Q4_K 18.0 /
 //     15.5; 24 15.5 / 16.9, 16.3 / 18.3, 16.2 / 15.5).
 static bool skinny_range(int qtype, int rows, int cols, int batch) {
     const bool q4 = qtype == HIP_BRIDGE_Q4_0, q4k = qtype == HIP_BRIDGE_Q4_K, q6 = qtype == HIP_BRIDGE_Q6_K;
     if (rows < kWideRows && cols >= kSplitMinCols) {  // deep
-        if (batch > 128) return false;
-        if (qtype == HIP_BRIDGE_BF16)
-            return (batch >= 17 && batch <= 32 && rows >= 2560) || (batch >= 64 && batch <= (rows >= kMidRows ? 96 : 128));
+        if (batch > (rows >= 2560 && !q4k && !q6 ? 96 : 128)) return false;
+        if (qtype == HIP_BRIDGE_BF16) return (batch >= 17 && batch <= 32 && rows >= 2560) || batch >= 64;
         if (rows <= 2048 && cols <= 176 * kKB && batch >= 25 && batch <= 32 && !q6) return false;
         if (qtype == HIP_BRIDGE_Q8_0) return batch >= 9;
         return (q4 || q4k || q6) && batch >= (q4 && rows < 2048 ? 9 : 5);
