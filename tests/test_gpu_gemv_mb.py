@@ -1,11 +1,12 @@
 """Small-batch products on the matrix cores (gemv.hip k_gemv_mb: from 2 tokens up to the
-prefill GEMM's threshold, 96 tokens for 8192 rows or more, 64 for narrower products at
-least 4096 deep, else 128; Q4_0 / Q8_0 / BF16 weights) through the C-ABI, over its
+prefill GEMM's, where k_gemm_skinny does not take the call) through the C-ABI, over its
 launch choices: 1, 2 or 4 sixteen-row tiles per wave and 4, 8 or 16 waves splitting the
-blocks of a row, rows too long for that in two halves added into zeroed y (so row counts that leave tiles and tile groups partly empty, block counts
-that the waves split unevenly, one or two 16-token tiles, tokens that leave a tile partly
-empty), and the shapes it leaves to the vector kernels (x not 16-byte aligned, other types,
-a column count that is not a whole number of blocks).
+blocks of a row, rows too long for that in two halves added into zeroed y (so row counts that
+leave tiles and tile groups partly empty, block counts that the waves split unevenly, one or two
+16-token tiles, tokens that leave a tile partly empty), and the shapes it leaves to the vector
+kernels (x not 16-byte aligned, other types, a column count that is not a whole number of
+blocks). Products of 2560, 6144 and 10240 columns are k_gemm_skinny's for some types and batches;
+the columns of 2592, 6176 and 10208 (odd block counts, no groups of four) are k_gemv_mb's for all.
 
 Integer-valued weights and activations make every partial sum exact in f32 (the three bf16
 terms of an integer x are x, 0, 0), so each product must equal the exact (float64) one bit
@@ -41,9 +42,10 @@ def gemm(dev, qtype, raw, X, rows, cols, batch, x_offset=0):
 
 @pytest.mark.parametrize("qtype", MB_TYPES)
 @pytest.mark.parametrize("rows,cols,batch", [
-    (10240, 2560, 8),   # 4 tiles per wave, 8 waves per workgroup
+    (10240, 2592, 8), (10240, 2560, 8),  # 4 tiles per wave, 16 (8) waves per workgroup
     (2560, 10240, 8),   # rows too long for 16 waves of 10 blocks: the vector kernels below 12 tokens,
-    (2500, 10240, 40), (130, 6144, 20), (2560, 10240, 12),  # two halves added into y from 12
+    (2500, 10208, 40), (130, 6176, 20), (2560, 10208, 12),  # two halves added into y from 12
+    (2500, 10240, 40), (130, 6144, 20), (2560, 10240, 12),
     (4096, 2560, 2), (1000, 2560, 16), (37, 2560, 17), (300, 1536, 31), (19, 96, 3),
     (5, 32, 2), (64, 160, 9), (777, 4096, 24), (100, 64, 5)])
 def test_mb_integer_bitexact(dev, qtype, rows, cols, batch):
@@ -95,10 +97,8 @@ def test_mb_leaves_other_cases_to_the_vector_kernels(dev, qtype):
     (B.Q4_K, 2560, 2560, 63), (B.Q6_K, 10240, 2560, 12), (B.Q6_K, 2048, 1024, 95), (B.F16, 1024, 512, 100),
     (B.F32, 512, 512, 77), (B.Q4_K, 8192, 512, 7), (B.Q4_K, 2560, 4096, 31), (B.Q6_K, 1024, 8192, 47)])
 def test_below_matrix_core_threshold_vs_f64(dev, qtype, rows, cols, batch):
-    """Batches below the prefill GEMM's threshold for their type and shape (8192 rows or more
-    / narrower but at least 4096 deep / the rest: Q4_0 and the dense types 96 / 64 / 128, Q4_K
-    128 / 96 / 96, Q6_K 64 / 96 / 96 tokens) take the small-batch or the vector kernels: within
-    2^-20 * sum |w_i x_i| of float64."""
+    """Batches around the crossovers of the small-batch kernels, the vector kernels and the GEMM for
+    their type and shape: within 2^-20 * sum |w_i x_i| of float64."""
     raw, wd = random_matrix(qtype, rows, cols, seed=rows + 5 * batch)
     X = synth.normal_f32(rows + batch + 1, "Xt", (batch, cols), 0, 2)
     exact = X.astype(np.float64) @ wd.T
@@ -109,9 +109,11 @@ def test_below_matrix_core_threshold_vs_f64(dev, qtype, rows, cols, batch):
 
 @pytest.mark.parametrize("qtype", [B.Q4_K, B.Q6_K])
 @pytest.mark.parametrize("rows,cols,batch", [(10240, 2560, 8), (2560, 10240, 16), (1000, 2560, 3), (37, 2048, 31),
-                                             (300, 1536, 17), (2500, 10240, 40), (64, 256, 2)])
+                                             (300, 1536, 17), (2500, 10240, 40), (64, 256, 2), (2048, 2560, 33),
+                                             (1600, 1536, 24), (2048, 5376, 30)])
 def test_mb_kquant_integer_bitexact_and_random(dev, qtype, rows, cols, batch):
-    """K-quants on the small-batch kernel. Q4_K: each 32-column block is one sub-block of a
+    """K-quants on the small-batch kernels (Q4_K rows of 2560 and 5376 columns, the latter in two halves, on
+    k_gemv_mb). Q4_K: each 32-column block is one sub-block of a
     256-column super-block, scaled by d * sc_j with dmin * m_j * sum x subtracted (scale and min
     decoded from the 12 packed bytes); Q6_K: sc * (u - 32) per 16 columns as two exact bf16
     terms, d per super-block. Integer operands exact, random ones within the bound."""

@@ -1877,7 +1877,7 @@ static void launch_gemv(int qtype, GemvArgs& a, hipStream_t s) {
 
 // ---- small batches on the matrix cores ------------------------------------------------------
 // Products of 2 to gemm_mfma_min_batch - 1 tokens (hip_gemm below the prefill GEMM) with Q4_0,
-// Q8_0, Q4_K, Q6_K or BF16 weights: v_mfma_f32_16x16x32_bf16 over tiles of 16 tokens x 16 rows x one
+// Q8_0, Q4_K, Q6_K or BF16 weights that k_gemm_skinny does not take (gemm.hip skinny_range): v_mfma_f32_16x16x32_bf16 over tiles of 16 tokens x 16 rows x one
 // 32-column block, tokens on the A side (each x as three bf16 terms h + m + l, as the prefill
 // GEMM: exact to the f32 value's 24 bits), rows on the B side. Block quants enter as their
 // unsigned codes u (Q4_0 nibbles 0..15, Q8_0 q ^ 0x80: exact in bf16) and a block's sum is
@@ -2136,13 +2136,13 @@ static bool launch_mb_t(const GemvArgs& a, hipStream_t s) {
     int ks = 0;
     for (int k : {4, 8, 16})
         if (!ks && cdiv(nblk, k) <= 10) ks = k;
-    // Rows too long for 16 waves of 10 blocks: from 12 tokens (Q4_K 8), two halves of the blocks
-    // per row tile added into zeroed y, at most 2 row tiles per wave (Q4_0 2560 x 10240 at 16 /
-    // 32 / 48 / 63 tokens: 36 / 67 / 68 / 99 us against the vector kernel's 39 / 73 / 105 / ~137;
-    // at 8 tokens 33 against 23, so fewer tokens keep the vector kernel; Q4_K's is slower: 46
-    // us at 8 tokens).
+    // Rows too long for 16 waves of 10 blocks: from 12 tokens, two halves of the blocks per row tile
+    // added into zeroed y, at most 2 row tiles per wave (Q4_0 2560 x 10240 at 16 / 32 / 48 / 63
+    // tokens: 36 / 67 / 68 / 99 us against the vector kernel's 39 / 73 / 105 / ~137; at 8 tokens 33
+    // against 23, so fewer tokens keep the vector kernel). Not Q6_K, whose long rows are
+    // k_gemm_skinny's or the GEMM's.
     unsigned kz = 1;
-    if (!ks && ZL_GEMV_MB_SPLIT && a.batch >= (QT == HIP_BRIDGE_Q4_K ? 8 : 12) && cdiv(nblk, 2 * 16) <= 10) {
+    if (!ks && ZL_GEMV_MB_SPLIT && QT != HIP_BRIDGE_Q6_K && a.batch >= 12 && cdiv(nblk, 2 * 16) <= 10) {
         ks = 16;
         kz = 2;
     }
