@@ -32,9 +32,10 @@ def run(dev, qtype, raw, X, rows, cols):
     return d_y.to_numpy((batch, rows), np.float32)
 
 
-# Workgroup tiles (tokens x rows) by launch size: 128 x 128 from 512 such tiles (e.g. 4096 rows
-# x 2048 tokens), else 64 x 128 from 512 (4096 x 1024; 2560 x 2048, 2500 x 1900 with a ragged
-# last tile), else 64 x 64.
+# Workgroup tiles (tokens x rows) by launch size: F16 and F32 weights 128 x 128 from 512 such tiles
+# (e.g. 4096 rows x 2048 tokens), else 64 x 128 from 512 (4096 x 1024; 2560 x 2048, 2500 x 1900 with a
+# ragged last tile), else 64 x 64; the other types 32 to 128 x 128 or 64 x 256 (gemm.hip launch_qt,
+# test_gpu_gemm_tiles.py).
 @pytest.mark.parametrize("qtype", TYPES)
 @pytest.mark.parametrize("rows,cols,batch", [(128, 64, 32), (200, 96, 37), (129, 2560, 128), (77, 160, 300),
                                              (256, 512, 64), (4096, 96, 2048), (4100, 64, 2050),

@@ -116,13 +116,14 @@ def test_large_pair_tiles(dev, qtype, cols, x_dtype):
     np.testing.assert_allclose(got, want.to_numpy((batch, rows), np.float32), rtol=2.0 ** -22, atol=1e-30)
 
 
-@pytest.mark.parametrize("qtype", [B.Q4_0, B.Q8_0, B.BF16, B.Q4_K, B.Q6_K])
-@pytest.mark.parametrize("cols", [992, 1024, 1056, 1248, 1280, 2816])
+SHARES = [(q, c) for q in (B.Q4_0, B.Q8_0, B.BF16) for c in (992, 1024, 1056, 1248, 1280, 2816)]
+SHARES += [(q, c) for q in (B.Q4_K, B.Q6_K) for c in (1024, 1280, 2816)]
+
+
+@pytest.mark.parametrize("qtype,cols", SHARES)
 def test_k_shares(dev, qtype, cols):
     """K in two shares per workgroup, and from 32 blocks in four (two of them added into zeroed y):
     31 blocks (16 + 15), 32, 33, 39 (16 + 8 + 8 + 7), 40 and 88, on few and on more tiles."""
-    if qtype in (B.Q4_K, B.Q6_K) and cols % 256:
-        pytest.skip("K-quant rows are whole super-blocks")
     for rows, batch in ((33, 129), (1025, 700)):
         raw, x, exact = operands(qtype, rows, cols, batch, rows + cols)
         assert np.all(np.abs(exact) < 2 ** 24)
@@ -131,3 +132,12 @@ def test_k_shares(dev, qtype, cols):
             y.fill(0xAB)
             dev.gemmEx(qtype, w, None, B.F32, xd, B.F32, y, batch, rows, cols)
             np.testing.assert_array_equal(y.to_numpy((batch, rows), np.float32), exact.astype(np.float32))
+
+
+@pytest.mark.parametrize("qtype,cols", [(B.Q6_K, 4352), (B.Q4_K, 1280), (B.Q8_0, 1056), (B.Q4_0, 4224)])
+def test_teams_of_planes(dev, qtype, cols):
+    """The two-team kernel on pre-split activations (Q6_K from 4096 columns)."""
+    rows, batch = 100, 150
+    raw, x, exact = operands(qtype, rows, cols, batch, cols)
+    got = product(dev, qtype, dev.from_numpy(raw), None, x, B.F32_TERMS, batch, rows, cols)
+    np.testing.assert_array_equal(got, exact.astype(np.float32))
