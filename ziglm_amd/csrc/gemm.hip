@@ -1375,11 +1375,12 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
     bf16x8 ones;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.0f;
-    // The row groups' sums over FG groups of blocks join a total in the LDS, so that a deep product's
-    // error does not grow with the length of a wave's share (BF16: a compensated total, shorter sums;
+    // The row groups' sums over FG groups of blocks (a share of up to WHOLE at once: 10240 x 2560 Q4_0, 8 tokens,
+    // 12.4 us in two sums, 11.9 in one) join a total in the LDS, so that a deep product's error does not
+    // grow with the length of a wave's share (BF16: a compensated total, shorter sums;
     // 5376 x 21504 at 24 tokens 1.27e-7 off without, the vector kernel 1.14e-7).
     constexpr bool KAHAN = QT == HIP_BRIDGE_BF16;
-    constexpr int FG = KAHAN ? 1 : 4, OWN = RT * VR * kWave;
+    constexpr int FG = KAHAN ? 1 : 4, WHOLE = HALVES && P == 1 ? 3 : 6, OWN = RT * VR * kWave;
     __shared__ float s_lost[KAHAN ? MAXW * OWN : 1];
     float *const total = s_red + wave * OWN + lane, *const lost = s_lost + (KAHAN ? wave * OWN + lane : 0);
     auto flush = [&](bool first) {
@@ -1422,6 +1423,8 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int kb = 4 * g + u;
+    bool first = true;
+    int stop = !KAHAN && g1 - g0 <= WHOLE ? g1 : min(g0 + FG, g1);
             bf16x8 wb[RT][2][1];
             float dv[RT][2], mn[RT];
 #pragma unroll
@@ -1483,9 +1486,13 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
             }
             __builtin_amdgcn_sched_barrier(0);  // (else the loads sink to their uses)
         }
-        if ((g - g0) % FG == FG - 1 || g + 1 == g1) flush(g - g0 < FG);  // uniform
+        if (g + 1 == stop) {  // uniform
+            flush(first);
+            first = false;
+            stop = min(stop + FG, g1);
+        }
     }
-    if (g0 >= g1) flush(true);
+    if (first) flush(true);  // (no groups)
 
     // The waves' sums, in a tree of two halves: w and w + half, then those in order.
     const int half = (ks + 1) / 2;
