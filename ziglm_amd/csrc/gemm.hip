@@ -863,7 +863,8 @@ static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
 // each. Large tiles convert an operand for more MFMAs, small ones fill the chip. us at 10240 x 2560
 // unless said:
 //   bf16 activations: 128 x 128 from 1.5 workgroups per CU (2048 tokens Q4_0: 140, 64 x 128 151,
-//     32 x 128 212), else 64 x 128 likewise, else 32 x 128.
+//     32 x 128 212), else 64 x 128 likewise, else 32 x 128; single blocks, two loads a step whatever the
+//     tile, 128 x 128 from 80 tiles and 64 x 128 from 64 (10240 x 2592 at 200 tokens Q8_0 101 -> 51, Q4_0 60 -> 46; Q4_0 128 x 128 as other rows).
 //   f32 (three-term) activations: 64 x 256 from three per CU for Q4_0 (it reads the LDS half as often
 //     per MFMA; 2048 tokens 284, 128 x 128 336, 64 x 128 322), from 400 tiles for BF16 rows that are
 //     not deep (700 tokens 123, 128 x 128 132, 64 x 128 147; gate.up 1024: 344, 361, 384; at 320 tiles, 512
@@ -909,7 +910,13 @@ static void launch_qt(const GemmArgs& a, hipStream_t s) {
     const bool big = F32 && (QT == HIP_BRIDGE_Q4_0 || B16) && !fine && wgs(2, 2) >= 768;
     // The shares of K, from the tiles that f32 activations had the shares measured on, so that planes
     // and f32 activations give the same sums whichever tile they take
-    int wt = fine ? 1 : XK == X_BF16 && wgs(4, 1) >= 384 ? 4 : big || wgs(2, 1) >= 384 ? 2 : 1;
+    constexpr bool ODD = QT == kQ4_0Odd || QT == kQ8_0Odd;
+    const bool whole = cdiv(a.batch, 128) * 8 <= cdiv(a.batch, 64) * 5;  // 128 tokens: at most a quarter more padding
+    int wt = fine ? 1 : big || wgs(2, 1) >= 384 ? 2 : 1;
+    if (XK == X_BF16) {
+        if (ODD) wt = whole && wgs(4, 1) >= (Q8 ? 80 : 384) ? 4 : a.batch > 32 && wgs(2, 1) >= 64 ? 2 : 1;
+        else if (wgs(4, 1) >= 384) wt = 4;
+    }
     const int64_t n = wgs(wt, big ? 2 : 1);
     if constexpr (F32 && !B16 && QT != kQ4_0Odd) {
         const bool pays = QT != HIP_BRIDGE_Q6_K || deep;
@@ -928,8 +935,7 @@ static void launch_qt(const GemmArgs& a, hipStream_t s) {
     }
     int rt = big ? 2 : 1;
     if constexpr (XK != X_BF16) {
-        if (wt == 1 && !fine && (TERMS ? QT != HIP_BRIDGE_Q4_0 && a.batch > 32 && wgs(2, 1) >= 80 : B16 && deep && wgs(2, 1) >= 160)) wt = 2;
-        const bool whole = cdiv(a.batch, 128) * 8 <= cdiv(a.batch, 64) * 5;  // at most a quarter more padding
+        if (wt == 1 && !fine && (TERMS || QT == kQ8_0Odd ? QT != HIP_BRIDGE_Q4_0 && a.batch > 32 && wgs(2, 1) >= 80 : B16 && deep && wgs(2, 1) >= 160)) wt = 2;
         if ((Q8 || B16) && whole && wgs(4, 1) >= (TERMS ? 320 : 448) && (Q8 || TERMS || deep)) wt = 4, rt = 1;
         else if (B16 && !TERMS && wgs(2, 2) >= 400 && !deep) wt = rt = 2;
         else if (B16 && TERMS) rt = 1;
@@ -1417,14 +1423,14 @@ __global__ __launch_bounds__(512, 2) void k_gemm_skinny(GemmArgs a) {
 #pragma unroll
         for (int b = 0; b < UX; ++b) load_x(4 * g0 + XB * b, xr[b]);
     }
+    bool first = true;
+    int stop = !KAHAN && g1 - g0 <= WHOLE ? g1 : min(g0 + FG, g1);
     for (int g = g0; g < g1; ++g) {
         bf16x8 xa[XS][3];
         f32x16 sx;  // (MIN) each row's sum over its columns
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int kb = 4 * g + u;
-    bool first = true;
-    int stop = !KAHAN && g1 - g0 <= WHOLE ? g1 : min(g0 + FG, g1);
             bf16x8 wb[RT][2][1];
             float dv[RT][2], mn[RT];
 #pragma unroll
