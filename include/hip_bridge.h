@@ -277,9 +277,9 @@ void hip_gemv_qkv_pro(int qtype, const void* q_w, const void* k_w, const void* v
                       float* q_out, float* k_out, float* v_out, int q_rows, int k_rows, int v_rows,
                       int cols, const HipGemvPrologue* pro, HipStream_t stream);
 /* Y[b*rows + r] = W[r] . X[b*cols ...], b < batch_size (batch 1 is the GEMV). y must not
- * overlap x or the weights: deep products and small batches of long rows clear y and add two
- * halves of each dot product into it (0 + a + b, the same bits in either order) while other
- * workgroups still read x; y in device memory (float atomics). */
+ * overlap x or the weights: where a product's tiles are few, f32 products of more than one token
+ * clear y and add two halves of each dot product into it (0 + a + b, the same bits in either order)
+ * while other workgroups still read x; y in device memory (float atomics). */
 void hip_gemm_q4_0(const void* weights, const float* x, float* y, int batch_size, int rows,
                    int cols, HipStream_t stream);                           /* cuda_bridge.h:47 */
 void hip_gemm_q8_0(const void* weights, const float* x, float* y, int batch_size, int rows,
@@ -296,9 +296,9 @@ void hip_gemm(int qtype, const void* weights, const float* x, float* y, int batc
  * (one term), so a bf16 norm output feeds the product directly. Q4_0, Q8_0, F16, BF16, F32
  * weights with cols % 32 == 0, Q4_K and Q6_K with cols % 256 == 0; x 16-byte aligned;
  * 128 * cols * sizeof(x element) < 4 GiB; else EUNSUPPORTED. f32 x and y without
- * up_weights is hip_gemm, which chooses by type, shape and batch between the matrix-core GEMM
- * (quantised and BF16 weights of 8192 rows or more from 17-33 tokens, narrower ones from 64-129),
- * the small-batch or vector kernels below. */
+ * up_weights is hip_gemm, which chooses by type, shape and batch between the matrix-core GEMM, the
+ * small-batch and the vector kernels. On the matrix cores f32 activations are three bf16 terms, so
+ * an infinite one can make its token's outputs NaN where f32 arithmetic gives infinities. */
 void hip_gemm_ex(int qtype, const void* weights, const void* up_weights /*NULL*/, int x_dtype,
                  const void* x, int y_dtype, void* y, int batch_size, int rows, int cols,
                  HipStream_t stream);
@@ -306,9 +306,10 @@ void hip_gemm_ex(int qtype, const void* weights, const void* up_weights /*NULL*/
  * m = bf16(x - h), l = bf16(x - h - m); h + m + l carries x's 24 significant bits), the
  * HIP_BRIDGE_F32_TERMS input of hip_gemm_ex: split once and shared by every product of the
  * same activations (QKV, gate and up), the K loop then converts weights only. The products
- * equal hip_gemm's on the f32 activations bit for bit where hip_gemm runs on the matrix cores
- * (Q4_K: within f32 rounding, its min term summing the planes rather than x). n % 4 == 0, x
- * 16-byte and planes 8-byte aligned; else EUNSUPPORTED. */
+ * of finite activations equal hip_gemm's on the f32 ones bit for bit where hip_gemm runs the GEMM
+ * (gemm.hip; Q4_K: within f32 rounding, its min term summing the planes rather than x) or
+ * k_gemm_skinny, its first choice for small batches. n % 4 == 0, x 16-byte and planes 8-byte
+ * aligned; else EUNSUPPORTED. */
 void hip_split_terms(const float* x, void* planes, int64_t n, HipStream_t stream);
 
 /* ---------------------------------------------------------------------------------- */

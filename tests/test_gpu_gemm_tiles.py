@@ -66,8 +66,8 @@ def rows_of(qtype, rows, cols, seed, some=61):
 
 
 def product(dev, qtype, w, wu, x, x_dtype, batch, rows, cols):
-    """One hip_gemm_ex product of f32 activations, as they are or split beforehand."""
-    xd, y = dev.from_numpy(x), dev.alloc(batch * rows * 4)
+    """One hip_gemm_ex product of f32 activations, as they are, split beforehand or rounded to bf16."""
+    xd, y = dev.from_numpy(synth.f32_to_bf16(x) if x_dtype == B.BF16 else x), dev.alloc(batch * rows * 4)
     y.fill(0xAB)
     if x_dtype == B.F32_TERMS:
         planes = dev.alloc(3 * batch * cols * 2)
@@ -87,7 +87,7 @@ LARGE = [(B.Q4_0, 160, 1990),                       # 64 x 128 (single blocks)
          (B.Q4_K, 256, 1990), (B.Q4_K, 768, 900)]   # 64 x 128: min terms on the matrix cores
 
 
-@pytest.mark.parametrize("x_dtype", [B.F32, B.F32_TERMS])
+@pytest.mark.parametrize("x_dtype", [B.F32, B.F32_TERMS, B.BF16])
 @pytest.mark.parametrize("qtype,cols,batch", LARGE)
 def test_large_tiles(dev, qtype, cols, batch, x_dtype):
     rows = 8200

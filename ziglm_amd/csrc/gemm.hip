@@ -4,9 +4,9 @@
 // prefill at cuda_model.zig:1264-1383), with ziglm's CPU arithmetic (math.zig:440-616): weights
 // dequantised exactly, activations kept in full, f32 sums. Outputs are f32 or bf16, and the
 // gate.up pair of a GeGLU FFN runs as one launch that writes gelu(gate) * up (the reference's
-// two prefill GEMMs and k_geglu, cuda_model.zig:1372-1387, cuda_bridge.cu:2247-2269): the
-// workgroup's W tile holds its output rows of both matrices, the up half's accumulators pass
-// to the gate half's waves through LDS, and the gate and up outputs never reach HBM.
+// two prefill GEMMs and k_geglu, cuda_model.zig:1372-1387, cuda_bridge.cu:2247-2269): a tile holds
+// its output rows of both matrices, an output's two sums meet by a lane shuffle (in k_gemm_dense
+// through the LDS), and the gate and up outputs never reach HBM.
 //
 // Exact operands on a bf16 matrix core. The MFMA multiplies bf16 operands exactly into f32
 // accumulators, so every operand is written as a short sum of bf16 terms that is exact or
@@ -21,10 +21,11 @@
 //   BF16 weights are exact; F16 weights (11 significant bits) are hi + lo, both exact in bf16;
 //   F32 weights are split like x;
 //   Q4_K (math.zig:440-496): a 32-column block is one sub-block j of a 256-column
-//     super-block, value q * (d * sc_j) - dmin * m_j with q in 0..15 (exact in bf16): the
-//     block's partial sum_k q_k x_k is scaled by A_j = d * sc_j and the min term
-//     B_j * sum_k x_k subtracted, with the per-token sums of x formed while staging x (the
-//     decode GEMV's decomposition);
+//     super-block, value q * (d * sc_j) - dmin * m_j with q in 0..15. The codes enter as q - 8 (exact
+//     in bf16): the block's partial sum_k (q_k - 8) x_k is scaled by A_j = d * sc_j and the min term
+//     (dmin * m_j - 8 A_j) * sum_k x_k subtracted, with the per-token sums of x formed while staging x.
+//     (With q itself the two parts of a value near the middle of the codes cancel and leave their
+//     rounding: 10240 x 2560, 33 tokens, 2.4e-7 off against 1.7e-7.)
 //   Q6_K (math.zig:556-616): value d * sc * (u - 32) with an int8 scale per 16 columns;
 //     u - 32 is exact in bf16 and d * sc (exact in f32) scales each K = 16 half's partial
 //     sum.
@@ -33,7 +34,7 @@
 // 2^-24 of a product, so a dot product lies within the f32 rounding of the sum, like the
 // decode GEMV's.
 //
-// Tiling (k_gemm_mfma). A workgroup of 4 waves owns 32 WT tokens x 128 RT rows; a wave computes
+// Tiling (k_gemm_mfma: quantised and BF16 weights). A workgroup of 4 waves owns 32 WT tokens x 128 RT rows; a wave computes
 // all of the tokens for its own 32 RT rows, as WT x RT tiles of v_mfma_f32_32x32x16_bf16 (tokens
 // on the A side, so a lane's accumulators are one weight row: the block scale is one value per
 // lane and tile, and stores of 32 lanes are 128 contiguous bytes of a token's output row). No two
@@ -112,7 +113,6 @@ __device__ __forceinline__ void split2(float x0, float x1, uint32_t* t) {
     t[0] = bf16_pair(x0, x1, a, b);
     t[1] = pack_bf16x2(x0 - a, x1 - b);
 }
-
 
 struct GemmArgs {
     const unsigned char* w;
@@ -455,8 +455,6 @@ struct TermPairs<1, NW> {
     static constexpr int xt[3] = {0, 0, 0}, wt[3] = {0, 1, 2};
 };
 
-
-
 // XK: activation form (X_F32: f32, split into three terms while staging; X_BF16: bf16, one
 // term; X_TERMS: three bf16 planes split beforehand, staged as they are). GE: gate.up GeGLU
 // pairs (out = gelu(g) * u).
@@ -478,11 +476,11 @@ __device__ __forceinline__ void add_kahan(float& total, float& lost, float part)
 
 // FINE (tiles of 32 tokens): the accumulators hold kFine steps and then join a compensated total, so
 // that a deep product's error does not grow with its depth.
-// TEAMS = 2: a second set of WAVES waves takes the other half of the workgroup's K steps, with LDS
+// TEAMS = 2: a second set of four waves takes the other half of the workgroup's K steps, with LDS
 // buffers of its own, and its sums join the first's through the LDS at the end.
-template <int QT, int XK, int WT, int RT, int WAVES, bool GE, int TEAMS, bool FINE>
-__global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a) {
-    constexpr int NT = 64 * WAVES;             // threads of a team
+template <int QT, int XK, int WT, int RT, bool GE, int TEAMS, bool FINE>
+__global__ __launch_bounds__(256 * TEAMS, 2) void k_gemm_mfma(GemmArgs a) {
+    constexpr int NT = 256;                    // threads of a team: four waves
     constexpr int XT = XK == X_BF16 ? 1 : 3;  // activation terms
     constexpr int NW = w_terms<QT>();
     constexpr bool SCALED = w_scaled<QT>();
@@ -490,7 +488,7 @@ __global__ __launch_bounds__(64 * WAVES * TEAMS, 2) void k_gemm_mfma(GemmArgs a)
     constexpr bool SUMS = SCALED || FINE;           // a step's products form a sum of their own
     constexpr int BT = 32 * WT;                // tokens per workgroup
     constexpr int TR = GE ? 16 : 32;           // output rows per tile
-    constexpr int OR = TR * WAVES * RT;        // and per workgroup
+    constexpr int OR = TR * 4 * RT;            // and per workgroup
     constexpr int XPLANE = BT * kLdsRow;
     // Q4_K: per-token sums of each K step's activations, four steps' worth.
     // The min terms are an f32 MFMA per tile and two blocks where a wave has several tiles (as FMAs they
@@ -855,9 +853,8 @@ static unsigned split_k(const GemmArgs& a, bool ge, bool want, hipStream_t s) {
 
 template <int QT, int XK, bool GE, int WT, int RT, int TEAMS = 1, bool FINE = false>
 static void launch_tile(const GemmArgs& a, unsigned ky, hipStream_t s) {
-    constexpr int W = 4;
-    const dim3 grid((unsigned)(cdiv(a.rows, (GE ? 16 : 32) * W * RT) * cdiv(a.batch, 32 * WT)), ky);
-    k_gemm_mfma<QT, XK, WT, RT, W, GE, TEAMS, FINE><<<grid, 64 * W * TEAMS, 0, s>>>(a);
+    const dim3 grid((unsigned)(cdiv(a.rows, (GE ? 64 : 128) * RT) * cdiv(a.batch, 32 * WT)), ky);
+    k_gemm_mfma<QT, XK, WT, RT, GE, TEAMS, FINE><<<grid, 256 * TEAMS, 0, s>>>(a);
 }
 // Workgroup tile (tokens x rows; GE: half the output rows), for 256 CUs that hold two workgroups
 // each. Large tiles convert an operand for more MFMAs, small ones fill the chip. us at 10240 x 2560
@@ -1032,7 +1029,6 @@ __device__ __forceinline__ void store_d(const DRaw<QT>& r, int h, uint16_t* sw, 
         }
     }
 }
-
 
 // Workgroups per CU the launch asks registers for: three (170 VGPRs a lane) for bf16
 // activations when the LDS holds three, so a third wave per SIMD has MFMAs ready while the
@@ -1278,7 +1274,6 @@ __global__ __launch_bounds__(kDenseThreads, (dense_wgs_per_cu<QT, XK, WT, WR>())
             }
         }
 }
-
 
 // Workgroup tile: the largest of 128 x 128, 64 x 128 and 64 x 64 (tokens x W rows) that still
 // gives at least two workgroups per CU (bigger tiles convert each operand for more MFMAs;

@@ -47,7 +47,8 @@ inline int device_cus() {
 // launches and returns true when the type, shape (cols % 32 == 0, K-quants % 256) and
 // alignment suit it, else launches nothing and returns false (the caller takes the vector
 // path).
-// Products at least this deep count as deep for the split of K in two halves (gemm.hip).
+// Products at least this deep count as deep: K in two halves at more tiles, and their own crossovers
+// (gemm.hip).
 constexpr int kSplitMinCols = 4096;
 // Rows from which 32-row tiles alone fill the chip's CUs, and most of them.
 constexpr int kWideRows = 8192, kMidRows = 5120;
