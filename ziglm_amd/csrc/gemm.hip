@@ -63,8 +63,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kKB = 32;       // columns per K step (one Q4_0 / Q8_0 block)
 // A token's LDS row is the block's 32 columns of one term: 64 bytes, its four 16-byte chunks
 // permuted by the row so that neither the reads (8 rows' same chunk a cycle) nor the writes (two
-// whole rows a cycle) meet on a bank. (Rows padded to 80 bytes: the writes' conflicts were 12% of
-// the kernel's cycles.)
+// whole rows a cycle) meet on a bank (counters: no conflict cycles; rows padded to 80 bytes had 32
+// million in a 10240 x 2560 x 2048 product).
 constexpr int kLdsRow = 32;
 __device__ __forceinline__ int lds_chunk(int row, int c) { return row * kLdsRow + ((c ^ (row >> 2)) & 3) * 8; }
 
@@ -173,8 +173,8 @@ struct WSrc {  // the lane's weight row; offsets: the lane's, and a wave-uniform
 // ops<S>(u) gives the B operands of block kb + u's MFMA S, and scale() the block's scale(s)
 // (one per MFMA for Q6_K) and min factor (Q4_K). A lane's loads are few and wide: its row lies
 // alone in its cache line, so an instruction costs as many cache accesses as it has rows
-// whatever its width, and with two narrow loads per block these were the kernel's next limit
-// (the texture path busy for half of the time).
+// whatever its width (Q8_0 with two loads per block: 2560 x 10240 at 700 tokens, bf16 activations,
+// 285 us, in groups 159).
 // Signed 4- and 6-bit codes are taken as 16 (u - 8) and 4 (u - 32), the signed bytes that a
 // shift and a sign flip leave, so each costs one conversion; the power of two goes into the
 // scale.
