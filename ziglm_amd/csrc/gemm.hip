@@ -395,7 +395,8 @@ struct WGrp<HIP_BRIDGE_BF16> {
 // not finite. An infinite x (or one that bf16 rounds to infinity) has the terms inf, inf - inf,
 // inf - inf, so every product of its token is NaN on the matrix cores, and a block's sum of unscaled
 // codes can overflow where the scaled products do not; this gives what f32 arithmetic on the values
-// gives. Serial, some ms a call: the price of a result that has to be looked at, not of a usual one.
+// gives. Serial, some ms a call: the price of a result that has to be looked at, not of a usual one. A
+// NaN ends it (a token of NaN, say a slot that holds none, costs next to nothing).
 template <int QT>
 __device__ float dot_columns(const unsigned char* row, const float* x, int c0, int c1) {
     float sum = 0.0f;
@@ -424,6 +425,7 @@ __device__ float dot_columns(const unsigned char* row, const float* x, int c0, i
             w = (float)(q - 8) * f16_bits_to_f32(*(const uint16_t*)b);
         }
         sum = fmaf(w, x[c], sum);
+        if (!(sum == sum)) break;
     }
     return sum;
 }
